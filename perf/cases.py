@@ -2,11 +2,13 @@
 
 Reads are drawn on the GPU from a seeded genome (GC content, interspersed and tandem repeats,
 substitution errors, both strands), as the benchmark's read sets are, and handed over as the host
-CSR arrays that every entry point takes. Five kinds of work, over read sets of a loader batch to
+CSR arrays that every entry point takes. Six kinds of work, over read sets of a loader batch to
 tens of millions of reads:
 
   resident  a batch already uploaded goes through phase 1 and the count and the table stays in
-        HBM, as in a benchmark step: all counters of both calls come back;
+            HBM, as in a benchmark step: what both calls return comes back, every partition's
+            bytes, superkmers, k-mers and rows and the distinct total (a copy of the whole table
+            to the host would take many times the pass);
   table     the whole call of a program that wants its table: host reads in, the rows of every
             partition in ascending key order out;
   store     the counting call of the drop-in: reference-format partitions from the host, the
