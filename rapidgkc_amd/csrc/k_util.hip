@@ -2,6 +2,8 @@
 #include "rgkc_device.h"
 #include "rgkc_internal.h"
 
+#include <algorithm>
+
 namespace rgkc {
 namespace {
 
@@ -74,7 +76,39 @@ __global__ void k_add(const uint64_t* a, const uint64_t* b, uint64_t* o, size_t 
     if (i < n) o[i] = a[i] + b[i];
 }
 
+// Rows [r0, r1) of the dense table (the partitions' rows back to back) into a host buffer. Partition i
+// owns dense rows [first[i], first[i + 1]), found by a binary search over the prefix staged in LDS;
+// its rows start at row src[i] of the main table, or of the second one where the top bit is set.
+// Bound by the PCIe writes into the pinned buffer (coalesced: consecutive lanes write consecutive rows).
+template <typename K>
+__global__ __launch_bounds__(256) void k_gather_rows(GatherArgs a) {
+    __shared__ uint64_t first[kGatherParts + 1];
+    for (int i = threadIdx.x; i <= a.n_parts; i += 256) first[i] = a.first[i];
+    __syncthreads();
+    for (uint64_t r = a.r0 + (uint64_t)blockIdx.x * 256 + threadIdx.x; r < a.r1; r += (uint64_t)gridDim.x * 256) {
+        int lo = 0, hi = a.n_parts;  // first[lo] <= r < first[hi]
+        while (hi - lo > 1) {
+            const int m = (lo + hi) >> 1;
+            if (first[m] <= r) lo = m;
+            else hi = m;
+        }
+        const uint64_t s = a.src[lo];
+        const bool two = (s >> 63) != 0;
+        const uint64_t row = (s & ~(1ull << 63)) + (r - first[lo]);
+        if (a.dst_keys) ((K*)a.dst_keys)[r - a.r0] = ((const K*)(two ? a.keys2 : a.keys))[row];
+        if (a.dst_counts) a.dst_counts[r - a.r0] = (two ? a.counts2 : a.counts)[row];
+    }
+}
+
 }  // namespace
+
+hipError_t launch_gather_rows(const GatherArgs& a, int key_bytes, hipStream_t s) {
+    if (a.r1 <= a.r0) return hipSuccess;
+    const unsigned grid = (unsigned)std::min<uint64_t>((a.r1 - a.r0 + 255) / 256, 512);
+    if (key_bytes == 8) hipLaunchKernelGGL(k_gather_rows<uint64_t>, dim3(grid), dim3(256), 0, s, a);
+    else hipLaunchKernelGGL(k_gather_rows<ulonglong2>, dim3(grid), dim3(256), 0, s, a);
+    return hipGetLastError();
+}
 
 size_t scan_tmp_words(size_t n) {
     size_t w = 0;

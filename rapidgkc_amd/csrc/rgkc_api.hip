@@ -49,6 +49,11 @@ constexpr size_t kNoAllocBytes = kNoAllocRowBytes + kNoAllocSegBytes + kNoAllocC
 static_assert(kNoAllocBytes == RGKC_NOALLOC_SCRATCH_BYTES, "header and library agree on the area");
 static __device__ __align__(256) uint8_t scratch[kNoAllocBytes];
 
+// Bytes of each of the two pinned buffers a table is copied out through. A buffer costs its
+// allocation on a context's first copy (a 4 MiB pair made a first k=55 table of 20 MB slower than
+// 128 separate copies); 1 MiB keeps the copy at the host's copying rate.
+constexpr size_t kTableChunk = 1u << 20;
+
 constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
 uint8_t* g_scratch_ptr[kMaxDevices] = {};
@@ -116,6 +121,11 @@ struct rgkc_ctx {
     std::vector<uint8_t> h_row_buf;
     std::vector<uint64_t> h_row_start;
     DevBuf keys2, counts2, part_distinct;
+    // copying the table out: its partitions' places, and two pinned buffers filled by turns
+    DevBuf gather_plan;
+    uint8_t* table_pin[2] = {nullptr, nullptr};
+    uint64_t table_pin_cap = 0;
+    hipEvent_t table_ev[2] = {nullptr, nullptr};
     bool table_ok = false;
     uint32_t inst_cap = 0;
     uint32_t count_wg_per_cu = 0;  // count kernel: resident workgroups per CU (0: four)
@@ -1061,6 +1071,10 @@ int rgkc_destroy(rgkc_ctx* c) {
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     stream_free(c);
     for (int i = 0; i < EV_N; i++) if (c->ev[i]) (void)hipEventDestroy(c->ev[i]);
+    for (int i = 0; i < 2; i++) {
+        if (c->table_ev[i]) (void)hipEventDestroy(c->table_ev[i]);
+        if (c->table_pin[i]) (void)hipHostFree(c->table_pin[i]);
+    }
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
     return 0;
@@ -1286,23 +1300,75 @@ int rgkc_count_host_store(rgkc_ctx* c, const uint8_t* store, const uint64_t* par
     return 0;
 }
 
+// The partitions' rows leave the device as one dense table: chunks of it are gathered straight into
+// two pinned buffers by turns, and the host copies one chunk to the caller while the device fills the
+// other. A copy per partition and array (1024 of them for 512 partitions) cost 11-12 us each.
 int rgkc_copy_table(rgkc_ctx* c, void* keys, uint32_t* counts) {
     if (!c) return RGKC_E_ARG;
     if (!c->table_ok) return fail(c, RGKC_E_STATE, "no table");
+    (void)hipGetLastError();
+    HIPC(c, hipSetDevice(c->device));
+    if (!keys && !counts) return 0;
     const size_t W = c->k <= 32 ? 8 : 16;
-    uint64_t o = 0;
-    for (int i = 0; i < c->parts; i++) {
-        const uint64_t n = c->h_rows[i], b = c->h_row_start[i];
-        const bool two = c->h_row_buf[i] != 0;
-        if (n) {
-            if (keys) HIPC(c, hipMemcpyAsync((uint8_t*)keys + o * W, (uint8_t*)(two ? c->keys2.p : c->keys.p) + b * W, n * W,
-                                             hipMemcpyDeviceToHost, c->stream));
-            if (counts) HIPC(c, hipMemcpyAsync(counts + o, (two ? c->counts2 : c->counts).as<uint32_t>() + b, n * 4,
-                                               hipMemcpyDeviceToHost, c->stream));
-        }
-        o += n;
+    const int n = c->parts;
+    hipStream_t s = c->stream;
+    std::vector<uint64_t> plan(2 * (size_t)n + 1);  // first dense row of each partition, then its place
+    uint64_t* const first = plan.data();
+    for (int i = 0; i < n; i++) {
+        first[i + 1] = first[i] + c->h_rows[i];
+        plan[(size_t)n + 1 + i] = c->h_row_start[i] | (c->h_row_buf[i] ? 1ull << 63 : 0);
     }
-    HIPC(c, hipStreamSynchronize(c->stream));
+    const uint64_t total = first[n];
+    if (!total) return 0;
+    const uint64_t chunk = std::min<uint64_t>(total, kTableChunk / (W + 4));
+    if (c->table_pin_cap < chunk * (W + 4)) {
+        for (int i = 0; i < 2; i++) {
+            if (c->table_pin[i]) (void)hipHostFree(c->table_pin[i]);
+            c->table_pin[i] = nullptr;
+        }
+        c->table_pin_cap = 0;
+        for (int i = 0; i < 2; i++)
+            if (hipHostMalloc((void**)&c->table_pin[i], chunk * (W + 4), hipHostMallocDefault) != hipSuccess) {
+                (void)hipGetLastError();
+                return fail(c, RGKC_E_NOMEM, "pinned allocation of %zu bytes failed", (size_t)(chunk * (W + 4)));
+            }
+        for (hipEvent_t& e : c->table_ev)
+            if (!e) HIPC(c, hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        c->table_pin_cap = chunk * (W + 4);
+    }
+    NEED(c, c->gather_plan, plan.size() * 8);
+    HIPC(c, hipMemcpyAsync(c->gather_plan.p, plan.data(), plan.size() * 8, hipMemcpyHostToDevice, s));
+    struct Chunk { uint64_t r0 = 0, r1 = 0; } inflight[2];
+    uint64_t next = 0;
+    int p0 = 0;  // first partition with rows at or after `next`
+    auto launch = [&](int b) -> hipError_t {
+        inflight[b] = Chunk{next, next};
+        if (next >= total) return hipSuccess;
+        while (first[p0 + 1] <= next) p0++;
+        const int np = std::min(n - p0, kGatherParts);
+        const uint64_t r1 = std::min(std::min(next + chunk, total), first[p0 + np]);
+        GatherArgs a{};
+        a.first = c->gather_plan.as<uint64_t>() + p0;
+        a.src = c->gather_plan.as<uint64_t>() + n + 1 + p0;
+        a.n_parts = np;
+        a.keys = c->keys.p; a.keys2 = c->keys2.p;
+        a.counts = c->counts.as<uint32_t>(); a.counts2 = c->counts2.as<uint32_t>();
+        a.r0 = next; a.r1 = r1;
+        a.dst_keys = keys ? (void*)c->table_pin[b] : nullptr;
+        a.dst_counts = counts ? (uint32_t*)(c->table_pin[b] + (r1 - next) * W) : nullptr;
+        inflight[b].r1 = next = r1;
+        if (hipError_t e = launch_gather_rows(a, (int)W, s)) return e;
+        return hipEventRecord(c->table_ev[b], s);
+    };
+    for (int b = 0; b < 2; b++) HIPC(c, launch(b));
+    for (int b = 0; inflight[b].r1 > inflight[b].r0; b ^= 1) {
+        HIPC(c, hipEventSynchronize(c->table_ev[b]));
+        const uint64_t r0 = inflight[b].r0, nr = inflight[b].r1 - r0;
+        if (keys) memcpy((uint8_t*)keys + r0 * W, c->table_pin[b], nr * W);
+        if (counts) memcpy(counts + r0, c->table_pin[b] + nr * W, nr * 4);
+        HIPC(c, launch(b));
+    }
+    HIPC(c, hipStreamSynchronize(s));  // also on the way out: nothing reads `plan` any more
     return 0;
 }
 

@@ -27,6 +27,23 @@ hipError_t rowscan_u32(uint32_t* m, uint64_t* totals, int rows, uint32_t cols, h
 // out[i] = a[i] + b[i] (n entries)
 hipError_t add_u64(const uint64_t* a, const uint64_t* b, uint64_t* out, size_t n, hipStream_t s);
 
+// Rows [r0, r1) of the dense (partition after partition) table into a host buffer: of the n_parts
+// <= kGatherParts partitions that hold them, partition i has dense rows [first[i], first[i + 1]), which
+// start at row src[i] & ~(1 << 63) of the main table (bit 63 clear) or the second one. dst_keys and
+// dst_counts (either may be null) get row r at r - r0.
+constexpr int kGatherParts = 1024;
+struct GatherArgs {
+    const uint64_t* first;
+    const uint64_t* src;
+    int n_parts;
+    const void *keys, *keys2;
+    const uint32_t *counts, *counts2;
+    uint64_t r0, r1;
+    void* dst_keys;
+    uint32_t* dst_counts;
+};
+hipError_t launch_gather_rows(const GatherArgs& a, int key_bytes, hipStream_t s);
+
 // ---- phase 1 (k_phase1.hip) ------------------------------------------------------------------
 struct SegTable {
     uint32_t* seg_read = nullptr;   // read index of each segment
