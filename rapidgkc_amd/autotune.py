@@ -3,8 +3,8 @@
 Tuned (all results are identical in every setting; only the time changes):
   - `inst_cap`: k-mer instances planned per count sweep (the LDS table's work item). Small sweeps
     pay the per-sweep fixed work more often; large ones overflow the table and are split.
-  - `count_wg_per_cu`: resident workgroups per CU of the persistent count kernel (1..4; its 39 KB
-    LDS table allows four).
+  - `count_wg_per_cu`: resident workgroups per CU of the persistent count kernel (1 or 2: its 81 KB
+    of LDS allows two).
   - `p1_lists`: whether phase 1 keeps superkmer lists for its emit pass (on: one scan of the reads
     and a list region of ~1.25 B per k-mer; off: the emit pass scans the reads again).
 
@@ -14,7 +14,7 @@ each candidate timed `reps` times on the resident batch, the fastest kept. Resul
 (device, k, p, parts, log2 of the batch's k-mers) in a text file next to the library, one line per
 shape, which the standalone CLI (host/rgkc_main.cpp) reads as well:
 
-    gfx950:k31:p11:parts512:n31 inst_cap=3328 count_wg_per_cu=4 p1_lists=1
+    gfx950:k31:p11:parts512:n31 inst_cap=8192 count_wg_per_cu=2 p1_lists=1
 """
 from __future__ import annotations
 
@@ -98,7 +98,7 @@ def tune(counter: native.Counter, k: int, p: int, parts: int, n_kmers: int, cmin
     counter.set_p1_lists(0 if choice["p1_lists"] else 0xFFFFFFFF)
     counter.superkmers(k, p, parts)
     # count stage: sweep size, then workgroups per CU
-    caps = (2560, 3072, 3328, 3584, 4096) if k <= 32 else (768, 1024, 1280, 1536)
+    caps = (5504, 7168, 8192, 9472, 11008) if k <= 32 else (1600, 2048, 2304, 2688)
     best = None
     for cap in caps:
         counter.set_tuning(cap)
@@ -108,7 +108,7 @@ def tune(counter: native.Counter, k: int, p: int, parts: int, n_kmers: int, cmin
             best, choice["inst_cap"] = ms, cap
     counter.set_tuning(choice["inst_cap"])
     best = None
-    for wg in (2, 3, 4):
+    for wg in (1, 2):
         counter.set_count_workgroups(wg)
         ms = _count_ms(counter, cmin, cmax, reps)
         times[f"count_wg_per_cu={wg}"] = ms

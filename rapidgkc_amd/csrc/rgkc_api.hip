@@ -99,17 +99,19 @@ struct rgkc_ctx {
     DevBuf skm_list, skm_n;  // phase 1: superkmer lists of the count pass (n_wg x skm_cap entries)
     DevBuf totals;  // 3 x parts uint64
     DevBuf poffs;   // part_off, part_end, rec_off, rec_end, row_base, row_end: 6 x parts uint64
-    DevBuf store, side, scratch;
+    DevBuf store, side;
     DevBuf err_word, stats_dev, cursors;
     int k = 0, p = 0, parts = 0;
     std::vector<uint64_t> h_part_off, h_rec_off, h_kmers;  // parts+1 prefix arrays
     bool store_ok = false;
     // buckets
     DevBuf b_byte, b_rec, b_part;
-    DevBuf sub_start, g_hist, g_seg_bytes, sub_sinst, item_cnt, item_off, items, scan_tmp2, words, b_word;
-    DevBuf key_cnt, key_off, exp_cnt, exp_off, sub_key_off, heavy_keys, exp_items;  // heavy sub-buckets
-    DevBuf item_desc;  // count: first-sweep descriptor of each work item
-    DevBuf sub_item0, sub_key_cs, ovf_n, ovf_off, ovf_keys;  // count: exact regions of overflowed slices
+    // count stage: plan area (instances, words and records per sub-bucket, totals: zeroed together), the
+    // units' place, regrouped records, item descriptors
+    DevBuf plan_area, sub_unit, unit_cur, n_units, seg_bytes, scan_tmp2, words, desc, b_word, unit_items;
+    DevBuf key_units, key_items, key_desc, heavy_keys, ovf_n, ovf_off, ovf_keys;  // units expanded into keys
+    uint64_t* h_plan = nullptr;     // pinned: totals of the plan
+    hipEvent_t plan_ev = nullptr;   // they have arrived
     uint32_t n_buckets = 0;
     uint64_t n_items = 0;
     // table
@@ -382,6 +384,16 @@ int do_phase1(rgkc_ctx* c, int k, int p, int parts, uint32_t* mm_hist = nullptr)
     return 0;
 }
 
+// K-mer instances planned per count sweep: for 64-bit keys what fills the table (4096 of 5120 slots) at
+// one distinct key in two instances, for 128-bit ones (2150 of 3072, tried one by one) nearly all distinct.
+// Read sets are mostly below: their larger units then take fewer sweeps than planned. The count stage over
+// 5500, 7000, 8200, 9472, 11000: 13.3, 12.7, 12.9, 13.0, 13.1 ms (1.2 G k-mers at 30x), 2.40, 2.29, 2.27, 2.32,
+// 2.37 (188 M, k=25); over 1600, 1900, 2200, 2600: 11.1, 10.2, 9.6, 9.9 ms (392 M, k=55 at 10x).
+uint32_t unit_cap(const rgkc_ctx* c) {
+    const uint32_t cap = c->inst_cap ? c->inst_cap : (c->k <= 32 ? 8192u : 2304u);
+    return std::min<uint32_t>(std::max<uint32_t>(cap, 256u), 1u << 19);
+}
+
 // Count-stage working set of buckets [b0, b1) in bytes (2-bit words, record descriptors, key
 // regions, per-bucket plan arrays; plus a temporary table of one row per k-mer instance in compact
 // mode). An estimate used to cut the buckets into groups that fit the device memory.
@@ -390,52 +402,62 @@ uint64_t group_bytes(const rgkc_ctx* c, uint32_t b0, uint32_t b1, size_t W, bool
     const uint64_t nb = b1 - b0;
     const uint64_t words = (kmi + ri * (uint64_t)(c->k + 14)) / 16 * 4 + nb * 128;
     const uint64_t keys = c->heavy_mode == 0 ? (kmi + kmi / 3) * W + nb * 8192 * W : 0;
-    const uint64_t per_bucket = nb * ((uint64_t)kSubIds * 40 + (uint64_t)kGroupSegments * 2 * kGroups * 4 + 4096);
-    const uint64_t items = kmi / 512 * 88;
-    return words + ri * 8 + keys + per_bucket + items + (temp_table ? kmi * (W + 4) : 0);
+    const uint64_t per_bucket = nb * ((uint64_t)kSubIds * 22 + 4096);
+    const uint64_t items = kmi / unit_cap(c) * 192;
+    return words + ri * 4 + keys + per_bucket + items + (temp_table ? kmi * (W + 4) : 0);
 }
 
-// The count stage over buckets [b0, b1): grouping, plan, key expansion (and its overflow pass), item
-// descriptors, count. Rows go to each partition's region as set in poffs (row base and end) by the
-// caller, in `keys`/`counts`; the stage times add into c->st.
+// The count stage over buckets [b0, b1): histogram, plan, grouping, key expansion of the largest units
+// (and its overflow pass), count. Rows go to each partition's region as set in poffs (row base and end)
+// by the caller, in `keys`/`counts`; the stage times add into c->st.
 int count_buckets(rgkc_ctx* c, uint32_t b0, uint32_t b1, uint32_t cmin, uint32_t cmax, void* keys, uint32_t* counts,
                   bool first) {
     hipStream_t s = c->stream;
     const int parts = c->parts;
     const uint32_t nb = b1 - b0;
     const uint64_t R0 = c->h_rec_off[b0], R = c->h_rec_off[b1] - R0;
+    const uint64_t N = c->h_kmers[b1] - c->h_kmers[b0];
     const size_t W = c->k <= 32 ? 8 : 16;
-    // sweeps of ~2x the table capacity in instances (distinct/instance ratios of read sets are
-    // mostly below one half); the table holds 1536 (64-bit keys) or 768 (128-bit) distinct keys.
-    // Long k-mers carry more sequencing errors (higher distinct ratios): their sweeps are 4/3 of
-    // the table (a 200 Mbp k=55 set with 1% errors: 1024 instances beat 1536 by 13 ms).
-    const uint32_t cap0 = c->inst_cap ? c->inst_cap : (c->k <= 32 ? 3328u : 1024u);
-    NEEDC(c, c->scratch, R * 8 + 64);
-    NEEDC(c, c->sub_start, (size_t)nb * (kGroups + 1) * 4);
-    NEEDC(c, c->g_hist, (size_t)nb * kGroupSegments * 2 * kGroups * 4);
-    NEEDC(c, c->g_seg_bytes, (size_t)nb * (kGroupSegments + 1) * 8);
-    NEEDC(c, c->sub_sinst, (size_t)nb * kSubIds * 4);
+    const uint64_t cap = unit_cap(c);
+    if (!c->h_plan) {
+        HIPC(c, hipHostMalloc((void**)&c->h_plan, 4096, hipHostMallocDefault));
+        HIPC(c, hipEventCreateWithFlags(&c->plan_ev, hipEventDisableTiming));
+    }
     // 2-bit word regions: a record of L bases takes ceil(L / 16) words, at most (k-mers + records *
     // (k + 14)) / 16 per bucket (region record counts are upper bounds in the capacity-sized modes)
     std::vector<uint64_t> bw(nb + 1, 0);
+    uint64_t most_rec = 0, most_kmers = 0;
     for (uint32_t i = 0; i < nb; i++) {
         const uint32_t b = b0 + i;
         const uint64_t kmi = c->h_kmers[b + 1] - c->h_kmers[b], ri = c->h_rec_off[b + 1] - c->h_rec_off[b];
         bw[i + 1] = bw[i] + (kmi + ri * (uint64_t)(c->k + 14)) / 16 + 8;
+        most_rec = std::max(most_rec, ri);
+        most_kmers = std::max(most_kmers, kmi);
     }
+    // record segments per bucket, a workgroup each: one chunk's records at least, and no more than fill
+    // the device twice over
+    const uint64_t most_segs = std::max<uint64_t>(16, std::min<uint64_t>(kGroupSegments, 4096 / nb));
+    const uint32_t n_segs = (uint32_t)std::min<uint64_t>(std::max<uint64_t>((most_rec + 1023) / 1024, 1), most_segs);
+    // item bounds: two neighbouring units of a bucket hold more than `cap` instances together, an expanded
+    // unit more than kDirectSlices * cap
+    const uint64_t most_items = std::min<uint64_t>(2 * N / cap + 2 * nb, (uint64_t)nb * kSubIds);
+    const uint64_t most_kunits = N / (cap * kDirectSlices) + 1, most_kitems = (N + N / kDirectSlices) / cap + 2;
+    const size_t area = (size_t)nb * kSubIds * 12 + kPlanWords * 8;
+    NEEDC(c, c->plan_area, area);
+    NEEDC(c, c->sub_unit, (size_t)nb * kSubIds * 2);
+    NEEDC(c, c->unit_cur, (size_t)nb * kSubIds * 8);
+    NEEDC(c, c->n_units, (size_t)nb * 4);
+    NEEDC(c, c->seg_bytes, (size_t)nb * (n_segs + 1) * 8);
     NEEDC(c, c->b_word, (nb + 1) * 8);
     NEEDC(c, c->words, (bw[nb] + 16) * 4);
+    NEEDC(c, c->desc, R * 4 + 64);
+    NEEDC(c, c->unit_items, most_items * sizeof(UnitDesc) + 64);
+    if (c->heavy_mode == 0) {
+        NEEDC(c, c->key_units, most_kunits * sizeof(KeyUnit) + 64);
+        NEEDC(c, c->key_items, most_kitems * 8 + 64);
+    }
     HIPC(c, hipMemcpyAsync(c->b_word.p, bw.data(), (nb + 1) * 8, hipMemcpyHostToDevice, s));
-    NEEDC(c, c->item_cnt, ((size_t)nb + 1) * 8);
-    NEEDC(c, c->item_off, ((size_t)nb + 1) * 8);
-    NEEDC(c, c->scan_tmp2, scan_tmp_words(nb + 1) * 8);
-    HIPC(c, hipMemsetAsync(c->item_cnt.p, 0, ((size_t)nb + 1) * 8, s));
-    NEEDC(c, c->key_cnt, ((size_t)nb + 1) * 8);
-    NEEDC(c, c->key_off, ((size_t)nb + 1) * 8);
-    NEEDC(c, c->exp_cnt, ((size_t)nb + 1) * 8);
-    NEEDC(c, c->exp_off, ((size_t)nb + 1) * 8);
-    HIPC(c, hipMemsetAsync(c->key_cnt.p, 0, ((size_t)nb + 1) * 8, s));
-    HIPC(c, hipMemsetAsync(c->exp_cnt.p, 0, ((size_t)nb + 1) * 8, s));
+    HIPC(c, hipMemsetAsync(c->plan_area.p, 0, area, s));
     const uint64_t* dpo = c->poffs.as<uint64_t>();
     CountArgs a{};
     a.store = c->store.as<uint8_t>();
@@ -448,8 +470,8 @@ int count_buckets(rgkc_ctx* c, uint32_t b0, uint32_t b1, uint32_t cmin, uint32_t
         a.b_rec_end = c->b_ends.as<uint64_t>() + parts + b0;
     }
     a.n_buckets = nb;
-    a.scratch = c->scratch.as<uint64_t>();
-    a.scratch_base = R0;
+    a.n_segs = n_segs;
+    a.rec_base = R0;
     a.row_base = dpo + 4 * parts;
     a.row_end = dpo + 5 * parts;
     a.row_cursor = c->cursors.as<unsigned long long>();
@@ -457,96 +479,77 @@ int count_buckets(rgkc_ctx* c, uint32_t b0, uint32_t b1, uint32_t cmin, uint32_t
     a.out_counts = counts;
     a.k = c->k;
     a.cmin = cmin; a.cmax = cmax;
-    a.inst_cap = cap0;
+    a.unit_cap = (uint32_t)cap;
     a.count_wg_per_cu = c->count_wg_per_cu;
     a.err = c->err_word.as<uint32_t>();
     a.stats = c->stats_dev.as<unsigned long long>();
     a.part_distinct = c->part_distinct.as<unsigned long long>();
-    a.sub_start = c->sub_start.as<uint32_t>();
-    a.g_hist = c->g_hist.as<uint32_t>();
-    a.g_seg_bytes = c->g_seg_bytes.as<uint64_t>();
-    HIPC(c, hipMemsetAsync(c->sub_sinst.p, 0, (size_t)nb * kSubIds * 4, s));
-    a.sub_sinst = c->sub_sinst.as<uint32_t>();
+    a.sub_rw = c->plan_area.as<unsigned long long>();
+    a.plan_n = a.sub_rw + (size_t)nb * kSubIds;
+    a.sub_inst = (uint32_t*)(a.plan_n + kPlanWords);
+    a.sub_unit = c->sub_unit.as<uint16_t>();
+    a.seg_bytes = c->seg_bytes.as<uint64_t>();
+    a.n_units = c->n_units.as<uint32_t>();
+    a.unit_cur = c->unit_cur.as<unsigned long long>();
+    a.desc = c->desc.as<uint32_t>();
     a.words = c->words.as<uint32_t>();
     a.b_word = c->b_word.as<uint64_t>();
-    a.item_cnt = c->item_cnt.as<uint64_t>();
+    a.unit_items = c->unit_items.as<UnitDesc>();
     a.heavy_on = c->heavy_mode == 0 ? 1u : 0u;
-    a.key_cnt = c->key_cnt.as<uint64_t>();
-    a.exp_cnt = c->exp_cnt.as<uint64_t>();
+    a.key_units = c->key_units.as<KeyUnit>();
+    a.key_items = c->key_items.as<uint64_t>();
     REC(c, EV_IDX, s);
-    HIPC(c, launch_group(a, s));
-    HIPC(c, launch_plan(a, false, s));
-    HIPC(c, scan_u64(a.item_cnt, c->item_off.as<uint64_t>(), nb + 1, c->scan_tmp2.as<uint64_t>(), s));
-    uint64_t tot3[3] = {0, 0, 0};  // work items, key slots, expansion tasks
-    HIPC(c, hipMemcpyAsync(&tot3[0], c->item_off.as<uint64_t>() + nb, 8, hipMemcpyDeviceToHost, s));
-    if (a.heavy_on) {
-        HIPC(c, scan_u64(a.key_cnt, c->key_off.as<uint64_t>(), nb + 1, c->scan_tmp2.as<uint64_t>(), s));
-        HIPC(c, hipMemcpyAsync(&tot3[1], c->key_off.as<uint64_t>() + nb, 8, hipMemcpyDeviceToHost, s));
-        HIPC(c, scan_u64(a.exp_cnt, c->exp_off.as<uint64_t>(), nb + 1, c->scan_tmp2.as<uint64_t>(), s));
-        HIPC(c, hipMemcpyAsync(&tot3[2], c->exp_off.as<uint64_t>() + nb, 8, hipMemcpyDeviceToHost, s));
-    }
-    HIPC(c, hipStreamSynchronize(s));
-    const uint64_t n_items = tot3[0];
-    if (n_items > 0x7FFFFFFFull) return fail(c, RGKC_E_ARG, "too many count work items");
-    NEEDC(c, c->items, n_items * 8 + 8);
-    NEEDC(c, c->item_desc, n_items * 64 + 64);
-    a.item_desc = c->item_desc.as<uint32_t>();
-    a.item_cnt = c->item_off.as<uint64_t>();
-    a.items = c->items.as<uint64_t>();
-    a.n_items = n_items;
-    c->n_items += n_items;
-    uint64_t n_exp = 0;
-    if (a.heavy_on && tot3[2] > 0 && tot3[2] <= 0x7FFFFFFFull) {
-        // key regions (the groups were sized to hold them); if the device cannot hold them after
-        // all, the items read records instead
-        if (need_count(c, c->heavy_keys, (size_t)tot3[1] * W + 64) != hipSuccess) {
-            (void)hipGetLastError();
-            a.heavy_on = 0;
-        }
-    } else {
+    HIPC(c, launch_hist(a, s));
+    HIPC(c, launch_plan(a, s));
+    // the plan's totals arrive while the records are grouped
+    HIPC(c, hipMemcpyAsync(c->h_plan, a.plan_n, kPlanWords * 8, hipMemcpyDeviceToHost, s));
+    HIPC(c, hipEventRecord(c->plan_ev, s));
+    HIPC(c, launch_group(a, 2 * most_kmers / cap + 2 > (uint64_t)kSmallUnits, s));
+    HIPC(c, hipEventSynchronize(c->plan_ev));
+    uint64_t n_kunits = c->h_plan[kPlanKeyUnits], n_kitems = c->h_plan[kPlanKeyItems], n_items = c->h_plan[kPlanItems];
+    if (n_kunits && need_count(c, c->heavy_keys, (size_t)c->h_plan[kPlanKeySlots] * W + 64) != hipSuccess) {
+        // the key regions (the groups were sized to hold them) do not fit after all: planned again
+        // without them, every unit is counted from its records
+        (void)hipGetLastError();
         a.heavy_on = 0;
+        HIPC(c, hipMemsetAsync(a.plan_n, 0, kPlanWords * 8, s));
+        HIPC(c, launch_plan(a, s));
+        n_items += n_kunits;
+        n_kunits = n_kitems = 0;
     }
-    if (a.heavy_on) {
-        NEEDC(c, c->exp_items, tot3[2] * 8 + 8);
-        NEEDC(c, c->sub_key_off, (size_t)nb * kSubIds * 8);
-        NEEDC(c, c->sub_item0, (size_t)nb * kSubIds * 4);
-        NEEDC(c, c->sub_key_cs, (size_t)nb * kSubIds * 4);
-        a.sub_item0 = c->sub_item0.as<uint32_t>();
-        a.sub_key_cs = c->sub_key_cs.as<uint32_t>();
-        a.key_cnt = c->key_off.as<uint64_t>();
-        a.exp_cnt = c->exp_off.as<uint64_t>();
-        a.heavy_keys = c->heavy_keys.p;
-        a.exp_items = c->exp_items.as<uint64_t>();
-        a.sub_key_off = c->sub_key_off.as<uint64_t>();
-        n_exp = tot3[2];
-    }
-    c->st.heavy_groups += (uint32_t)n_exp;
-    HIPC(c, launch_plan(a, true, s));
     REC(c, EV_PLAN, s);
-    HIPC(c, launch_expand(a, n_exp, s));
-    if (a.heavy_on) {
-        // slices that received more keys than their region holds: exact regions, second pass
-        NEEDC(c, c->ovf_n, (n_items + 1) * 8);
-        NEEDC(c, c->ovf_off, (n_items + 1) * 8);
+    a.heavy_keys = c->heavy_keys.p;
+    a.n_key_items = n_kitems;
+    c->n_items += n_items + n_kitems;
+    c->st.heavy_groups += (uint32_t)n_kunits;
+    if (n_kunits) {
+        NEEDC(c, c->key_desc, n_kitems * sizeof(KeyItem) + 64);
+        NEEDC(c, c->ovf_n, (n_kitems + 1) * 8);
+        NEEDC(c, c->ovf_off, (n_kitems + 1) * 8);
+        NEEDC(c, c->scan_tmp2, scan_tmp_words(n_kitems + 1) * 8);
+        a.key_desc = c->key_desc.as<KeyItem>();
         a.ovf_n = c->ovf_n.as<uint64_t>();
-        NEEDC(c, c->scan_tmp2, scan_tmp_words(std::max<uint64_t>(n_items, nb) + 1) * 8);
+        a.ovf_off = c->ovf_off.as<uint64_t>();
+        HIPC(c, launch_expand(a, n_kunits, s));
+        // slices that received more keys than their region holds
         HIPC(c, launch_ovf_sizes(a, s));
-        HIPC(c, scan_u64(a.ovf_n, c->ovf_off.as<uint64_t>(), n_items + 1, c->scan_tmp2.as<uint64_t>(), s));
-        uint64_t n_ovf = 0;
-        HIPC(c, hipMemcpyAsync(&n_ovf, c->ovf_off.as<uint64_t>() + n_items, 8, hipMemcpyDeviceToHost, s));
-        HIPC(c, hipStreamSynchronize(s));
-        c->st.ovf_keys += n_ovf;
-        if (n_ovf) {
-            NEEDC(c, c->ovf_keys, (size_t)n_ovf * W + 64);
-            a.ovf_off = c->ovf_off.as<uint64_t>();
-            a.ovf_keys = c->ovf_keys.p;
-            HIPC(c, launch_expand_ovf(a, n_exp, s));
-        } else {
-            a.ovf_n = nullptr;
-        }
+        HIPC(c, scan_u64(a.ovf_n, a.ovf_off, n_kitems + 1, c->scan_tmp2.as<uint64_t>(), s));
+        HIPC(c, hipMemcpyAsync(c->h_plan, a.ovf_off + n_kitems, 8, hipMemcpyDeviceToHost, s));
+        HIPC(c, hipEventRecord(c->plan_ev, s));
     }
     REC(c, EV_EXP, s);
-    HIPC(c, launch_count_items(a, s));
+    HIPC(c, launch_count_units(a, s));
+    if (n_kunits) {
+        HIPC(c, hipEventSynchronize(c->plan_ev));
+        const uint64_t n_ovf = c->h_plan[0];
+        c->st.ovf_keys += n_ovf;
+        if (n_ovf) {  // exact regions, second pass
+            NEEDC(c, c->ovf_keys, (size_t)n_ovf * W + 64);
+            a.ovf_keys = c->ovf_keys.p;
+            HIPC(c, launch_expand_ovf(a, n_kunits, s));
+        }
+        HIPC(c, launch_count_keys(a, s));
+    }
     REC(c, EV_CNT, s);
     HIPC(c, hipStreamSynchronize(s));
     auto el = [&](int e0, int e1) {
@@ -678,12 +681,11 @@ int do_count_once(rgkc_ctx* c, uint32_t cmin, uint32_t cmax, bool predicted) {
     // Every count-stage buffer counts as available, so the same batch gets the same plan each time
     // and the grow-only buffers are allocated once (allocations of tens of GB cost seconds). The
     // phase-1 buffers stay: the next batch would allocate them again.
-    for (const DevBuf* d : {&c->scratch, &c->keys, &c->counts, &c->cursors, &c->stats_dev, &c->sub_start, &c->g_hist,
-                            &c->g_seg_bytes, &c->sub_sinst, &c->item_cnt, &c->item_off, &c->items, &c->scan_tmp2,
-                            &c->words, &c->b_word, &c->key_cnt, &c->key_off, &c->exp_cnt, &c->exp_off, &c->sub_key_off,
-                            &c->heavy_keys, &c->exp_items, &c->item_desc, &c->sub_item0, &c->sub_key_cs, &c->ovf_n,
-                            &c->ovf_off, &c->ovf_keys, &c->tkeys, &c->tcounts, &c->sort_segs, &c->sort_chunks,
-                            &c->sort_hist, &c->keys2, &c->counts2})
+    for (const DevBuf* d : {&c->keys, &c->counts, &c->cursors, &c->stats_dev, &c->plan_area, &c->sub_unit, &c->unit_cur,
+                            &c->n_units, &c->seg_bytes, &c->scan_tmp2, &c->words, &c->desc, &c->b_word, &c->unit_items,
+                            &c->key_units, &c->key_items, &c->key_desc, &c->heavy_keys, &c->ovf_n, &c->ovf_off,
+                            &c->ovf_keys, &c->tkeys, &c->tcounts, &c->sort_segs, &c->sort_chunks, &c->sort_hist,
+                            &c->keys2, &c->counts2})
         held += d->cap;
     const uint64_t reserve = 4ull << 30;  // other users of the device and the runtime
     uint64_t avail = (uint64_t)fr + held > reserve ? ((uint64_t)fr + held - reserve) / 100 * 92 : 0;
@@ -1071,6 +1073,8 @@ int rgkc_destroy(rgkc_ctx* c) {
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     stream_free(c);
     for (int i = 0; i < EV_N; i++) if (c->ev[i]) (void)hipEventDestroy(c->ev[i]);
+    if (c->plan_ev) (void)hipEventDestroy(c->plan_ev);
+    if (c->h_plan) (void)hipHostFree(c->h_plan);
     for (int i = 0; i < 2; i++) {
         if (c->table_ev[i]) (void)hipEventDestroy(c->table_ev[i]);
         if (c->table_pin[i]) (void)hipHostFree(c->table_pin[i]);

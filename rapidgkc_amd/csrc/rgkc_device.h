@@ -99,6 +99,18 @@ __device__ __forceinline__ uint32_t wave_incl_scan_u32(uint32_t x) {
     return x + (row >= 1 ? r0 : 0u) + (row >= 2 ? r1 : 0u) + (row >= 3 ? r2 : 0u);
 }
 
+// Loads of any alignment.
+__device__ __forceinline__ uint32_t load_u32(const uint8_t* p) {
+    uint32_t v;
+    __builtin_memcpy(&v, p, 4);
+    return v;
+}
+__device__ __forceinline__ uint32_t load_u16(const uint8_t* p) {
+    uint16_t v;
+    __builtin_memcpy(&v, p, 2);
+    return v;
+}
+
 // Workgroup-wide exclusive scan of one uint32 per thread (blockDim.x <= 1024, multiple of 64).
 // `tmp` needs blockDim.x/64 + 1 words of LDS. Returns the exclusive prefix; *total gets the sum.
 // Ends with a barrier, so `tmp` may be reused at once.

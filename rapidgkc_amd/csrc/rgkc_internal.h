@@ -9,10 +9,8 @@ constexpr int kScanTile = 4096;      // elements per workgroup tile in the devic
 constexpr int kP1Threads = 256;      // phase-1 workgroup size (one read segment per thread)
 constexpr int kSegKmers = 128;       // k-mers per read segment (long reads are cut into segments)
 constexpr int kMaxParts = 1024;      // partitions supported by the LDS histograms of phase 1
-constexpr int kSubIds = 4096;
-constexpr uint32_t kGroupSegments = 16;  // count stage: record segments per bucket in the grouping kernels
-constexpr int kGroups = 1024;         // record groups per bucket in the count stage (4 sub-buckets each)        // minimizer sub-bucket ids per partition (12 bits)
-constexpr int kCountThreads = 1024;  // count workgroup size
+constexpr int kSubIds = 4096;         // minimizer sub-bucket ids per partition (12 bits)
+constexpr uint32_t kGroupSegments = 64;  // count stage: record segments per bucket in the grouping kernels, at most
 // packed stream-mode cursor: records in the low kRecBits bits, bytes above
 constexpr int kRecBits = 28;
 constexpr unsigned long long kRecMask = (1ull << kRecBits) - 1;
@@ -117,7 +115,34 @@ hipError_t launch_batch_prep(const uint8_t* reads, const uint64_t* offs, uint64_
                              uint64_t cap_bases, int k, uint32_t* bases2, uint64_t* nseg, uint64_t* seg_off,
                              uint64_t* scan_tmp, uint32_t* seg_read, uint32_t* seg_first, hipStream_t s);
 
-// ---- count (k_count.hip) ---------------------------------------------------------------------
+// ---- count (k_group.hip, k_count.hip) ----------------------------------------------------------
+// A unit of more than this many unit_caps is expanded into keys: at 30x, 1.2 G k-mers, the count stage
+// takes 13.6 ms with 1, 13.1 with 2, 13.6 with 3 (a direct unit is read once per sweep).
+constexpr uint32_t kDirectSlices = 2;
+constexpr uint32_t kMaxKeySlices = 127; // hash slices (key regions) of an expanded unit
+constexpr int kSmallUnits = 1024;       // units of a bucket that the small grouping kernel takes
+enum { kPlanItems, kPlanKeySlots, kPlanKeyUnits, kPlanKeyItems, kPlanSeenInst, kPlanSeenDistinct, kPlanWords };
+// A unit of work: sub-buckets of one partition whose records lie together.
+struct UnitDesc {
+    uint32_t part, inst, n_rec, n_word;  // partition, k-mer instances, records, their 2-bit words
+    uint64_t desc, word;                 // first record descriptor and first word
+    uint32_t q, pad;                     // slices (expanded units)
+};
+// An expanded unit: key regions of 1 + cs slots per slice (the fill count, then keys) from slot key0 on.
+struct KeyUnit {
+    UnitDesc u;
+    uint64_t key0, item0;
+    uint32_t cs, pad;
+};
+struct KeyItem {
+    uint32_t part, n, slice, q;
+    uint64_t keys, pad;  // address of the slice's keys
+};
+// key slots of a slice region: the slice's share of instances with a margin (slices are hash slices: a
+// share above 1.25x + 256 is far in the tail; a fuller slice gets an exact region in a second pass)
+__host__ __device__ inline uint32_t key_region(uint32_t inst, uint32_t q) {
+    return ((inst + q - 1) / q / 4 * 5 + 256 + 63) & ~63u;
+}
 struct CountArgs {
     const uint8_t* store;       // superkmer records
     const uint32_t* side;       // side descriptors, one per record, in store order
@@ -127,8 +152,8 @@ struct CountArgs {
     const uint64_t* b_rec_end;
     const uint32_t* b_part;     // partition of each bucket
     uint32_t n_buckets;
-    uint64_t* scratch;          // one uint64 per record: word offset << 32 | side word, group order
-    uint64_t scratch_base;      // record index of scratch[0] (the first record of the buckets counted)
+    uint32_t n_segs;            // record segments per bucket (<= kGroupSegments)
+    uint64_t rec_base;          // record index of desc[0] (the first record of the buckets counted)
     const uint64_t* row_base;   // per partition: first row of its region
     const uint64_t* row_end;    // per partition: end of its region
     unsigned long long* row_cursor;  // per partition: rows written so far
@@ -136,44 +161,44 @@ struct CountArgs {
     uint32_t* out_counts;
     int k;
     uint32_t cmin, cmax;
-    uint32_t inst_cap;          // k-mer instances planned per sweep (distinct-capacity proxy)
-    uint32_t count_wg_per_cu;   // resident count workgroups per CU (0: four)
+    uint32_t unit_cap;          // k-mer instances planned per sweep (distinct-capacity proxy)
+    uint32_t count_wg_per_cu;   // resident count workgroups per CU (0: as many as fit)
     uint32_t* err;
     unsigned long long* stats;  // [0] sweeps, [1] overflow retries, [2] distinct (unfiltered)
     unsigned long long* part_distinct;  // per partition: distinct keys (unfiltered)
-    uint32_t* sub_start;        // [n_buckets][kGroups + 1] descriptor start of each record group
-    uint32_t* sub_sinst;        // [n_buckets][kSubIds] k-mer instances of each sub-bucket
-    uint32_t* g_hist;           // grouping: [n_buckets][segments][2][kGroups] records, words per group
-    uint64_t* g_seg_bytes;      // grouping: [n_buckets][segments + 1] store bytes per segment, then prefix
-    uint32_t* words;            // records re-encoded as word-aligned 2-bit bases, group order
+    unsigned long long* plan_n;         // [kPlanWords] totals of the plan, instances and distinct keys counted so far
+    uint32_t* sub_inst;         // [n_buckets][kSubIds] k-mer instances of each sub-bucket
+    unsigned long long* sub_rw; // [n_buckets][kSubIds] words << 32 | records of each sub-bucket
+    uint16_t* sub_unit;         // [n_buckets][kSubIds] unit of each (non-empty) sub-bucket
+    uint64_t* seg_bytes;        // [n_buckets][n_segs + 1] store bytes per record segment, then their prefix
+    uint32_t* n_units;          // [n_buckets]
+    unsigned long long* unit_cur;  // [n_buckets][kSubIds] words << 32 | records: next free place of each unit
+    uint32_t* desc;             // k-mers of each record, unit after unit
+    uint32_t* words;            // records re-encoded as word-aligned 2-bit bases, in the same order
     const uint64_t* b_word;     // [n_buckets + 1] word region of each bucket
-    uint64_t* item_cnt;         // [n_buckets + 1] work items per bucket, then their prefix
-    uint64_t* items;            // bucket << 40 | s_lo << 27 | s_hi << 14 | slice << 7 | nslices
-    uint64_t n_items;
-    // Heavy sub-buckets (more instances than one work item) are expanded into keys once: the keys
-    // of each hash slice get a region of 1 + cs key slots (slot 0 holds the fill cursor), and the
-    // work items of such a sub-bucket (s_hi field 0) read keys instead of records.
-    uint32_t heavy_on;          // 0: heavy sub-buckets are sliced over their records
-    uint64_t* key_cnt;          // [n_buckets + 1] key slots per bucket, then their prefix
-    uint64_t* exp_cnt;          // [n_buckets + 1] expansion tasks (groups) per bucket, then their prefix
-    uint64_t* sub_key_off;      // [n_buckets][kSubIds] first key slot of each heavy sub-bucket
+    UnitDesc* unit_items;       // units counted from their records (plan_n[kPlanItems] of them)
+    // Units far larger than a sweep are expanded into keys once (heavy_on), a region per hash slice:
+    uint32_t heavy_on;
+    KeyUnit* key_units;
+    uint64_t* key_items;        // unit << 8 | slice
+    KeyItem* key_desc;          // after expansion: each slice's keys
+    uint64_t n_key_items;
     void* heavy_keys;           // key slots (8 or 16 bytes)
-    uint64_t* exp_items;        // bucket << 32 | group, for each group holding a heavy sub-bucket
-    uint32_t* item_desc;        // [n_items][16] first-sweep descriptor of each work item (k_item_prep)
     // Slices whose region overflowed (a very frequent key) get an exact region in a second key area:
-    uint32_t* sub_item0;        // [n_buckets][kSubIds] first work item of each heavy sub-bucket
-    uint32_t* sub_key_cs;       // [n_buckets][kSubIds] key slots of each slice region of the sub-bucket
-    uint64_t* ovf_n;            // [n_items + 1] slots of the item's exact region (0: none), then their prefix in ovf_off
+    uint64_t* ovf_n;            // [n_key_items + 1] keys of the item's exact region (0: none), their prefix in ovf_off
     uint64_t* ovf_off;
     void* ovf_keys;
 };
-hipError_t launch_group(const CountArgs& a, hipStream_t s);
-hipError_t launch_plan(const CountArgs& a, bool fill, hipStream_t s);
-hipError_t launch_expand(const CountArgs& a, uint64_t n_exp, hipStream_t s);
-// ovf_n of every item (after launch_expand); then, with ovf_off and ovf_keys set, the exact regions
+hipError_t launch_hist(const CountArgs& a, hipStream_t s);
+hipError_t launch_plan(const CountArgs& a, hipStream_t s);
+hipError_t launch_group(const CountArgs& a, bool many, hipStream_t s);
+hipError_t launch_expand(const CountArgs& a, uint64_t n_units, hipStream_t s);
+// ovf_n of every key item (after launch_expand); then, with ovf_off and ovf_keys set, the exact regions
 hipError_t launch_ovf_sizes(const CountArgs& a, hipStream_t s);
-hipError_t launch_expand_ovf(const CountArgs& a, uint64_t n_exp, hipStream_t s);
-hipError_t launch_count_items(const CountArgs& a, hipStream_t s);
+hipError_t launch_expand_ovf(const CountArgs& a, uint64_t n_units, hipStream_t s);
+// the units counted from their records; the expanded units' slices
+hipError_t launch_count_units(const CountArgs& a, hipStream_t s);
+hipError_t launch_count_keys(const CountArgs& a, hipStream_t s);
 
 // Side descriptors for a store that lacks them (host-provided partitions): one workgroup per
 // partition finds record starts by the full/non-full byte rule and recomputes each record's
