@@ -106,6 +106,7 @@ struct rgkc_ctx {
     bool store_ok = false;
     // buckets
     DevBuf b_byte, b_rec, b_part;
+    DevBuf idx_chunks, idx_counts;  // host stores: pieces of the partitions, their record counts
     // count stage: plan area (instances, words and records per sub-bucket, totals: zeroed together), the
     // units' place, regrouped records, item descriptors
     DevBuf plan_area, sub_unit, unit_cur, n_units, seg_bytes, scan_tmp2, words, desc, b_word, unit_items;
@@ -1250,14 +1251,37 @@ int rgkc_count_host_store(rgkc_ctx* c, const uint8_t* store, const uint64_t* par
     REC(c, EV_START, s);
     if (S) HIPC(c, hipMemcpyAsync(c->store.p, store, S, hipMemcpyHostToDevice, s));
     HIPC(c, hipMemcpyAsync(c->b_byte.p, part_offs, (n_parts + 1) * 8, hipMemcpyHostToDevice, s));
+    // pieces of the partitions: the partition of each, and the first of each partition
+    std::vector<uint32_t> pieces;
+    std::vector<uint32_t> first(n_parts + 1, 0);
+    for (int i = 0; i < n_parts; i++) {
+        const uint64_t np = (part_offs[i + 1] - part_offs[i] + kIndexChunk - 1) / kIndexChunk;
+        if (pieces.size() + np > 0x7FFFFFFFull) return fail(c, RGKC_E_ARG, "store too large for one call");
+        pieces.insert(pieces.end(), (size_t)np, (uint32_t)i);
+        first[i + 1] = (uint32_t)pieces.size();
+    }
+    const size_t n_chunks = pieces.size();
+    pieces.insert(pieces.end(), first.begin(), first.end());
+    NEED(c, c->idx_chunks, pieces.size() * 4);
+    NEED(c, c->idx_counts, 2 * (n_chunks + 1) * 8);
+    NEED(c, c->scan_tmp2, scan_tmp_words(n_chunks + 1) * 8);
+    HIPC(c, hipMemcpyAsync(c->idx_chunks.p, pieces.data(), pieces.size() * 4, hipMemcpyHostToDevice, s));
+    HIPC(c, hipMemsetAsync(c->totals.p, 0, 2 * (size_t)n_parts * 8, s));
     IndexArgs ia{};
     ia.store = c->store.as<uint8_t>();
     ia.part_byte = c->b_byte.as<uint64_t>();
     ia.n_parts = (uint32_t)n_parts;
+    ia.n_chunks = (uint32_t)n_chunks;
+    ia.chunk_part = c->idx_chunks.as<uint32_t>();
+    ia.part_chunk = ia.chunk_part + n_chunks;
     ia.k = k; ia.p = p; ia.parts_total = parts_total;
+    ia.chunk_n = c->idx_counts.as<uint64_t>();
+    ia.chunk_rec = ia.chunk_n + n_chunks + 1;
     ia.rec_count = c->totals.as<uint64_t>();
     ia.err = c->err_word.as<uint32_t>();
     HIPC(c, launch_index_count(ia, s));
+    HIPC(c, scan_u64(ia.chunk_n, ia.chunk_n + n_chunks + 1, n_chunks + 1, c->scan_tmp2.as<uint64_t>(), s));
+    HIPC(c, launch_index_parts(ia, s));
     std::vector<uint64_t> rc(2 * (size_t)n_parts);
     HIPC(c, hipMemcpyAsync(rc.data(), c->totals.p, rc.size() * 8, hipMemcpyDeviceToHost, s));
     HIPC(c, hipStreamSynchronize(s));
@@ -1289,7 +1313,6 @@ int rgkc_count_host_store(rgkc_ctx* c, const uint8_t* store, const uint64_t* par
     HIPC(c, hipMemcpyAsync(c->b_rec.p, c->h_rec_off.data(), (n_parts + 1) * 8, hipMemcpyHostToDevice, s));
     HIPC(c, hipMemcpyAsync(c->b_part.p, bp.data(), n_parts * 4, hipMemcpyHostToDevice, s));
     ia.side = c->side.as<uint32_t>();
-    ia.rec_off = c->b_rec.as<uint64_t>();
     HIPC(c, launch_index_fill(ia, s));
     REC(c, EV_P1E, s);
     c->n_buckets = (uint32_t)n_parts;

@@ -111,6 +111,23 @@ __device__ __forceinline__ uint32_t load_u16(const uint8_t* p) {
     return v;
 }
 
+// The 16 bases from base t0 on of a record (cpu_funcs.cpp:219-250 layout: base t at digit (bm3 + t) % 3
+// of byte (bm3 + t) / 3, digit 0 in bits 5:4) as one LSB-first 2-bit word. Six bytes hold them; zeros
+// follow the record's last base, L - 1.
+__device__ __forceinline__ uint32_t record_word(const uint8_t* rec, uint32_t bm3, uint32_t t0, uint32_t L) {
+    const uint32_t b = bm3 + t0, j = b / 3u, r = b - 3u * j;
+    const uint32_t lo = load_u32(rec + j), hi = load_u16(rec + j + 4);
+    // the three digits of every byte reversed in place, then the bytes' six bits packed
+    auto rev = [](uint32_t x) { return ((x & 0x03030303u) << 4) | (x & 0x0C0C0C0Cu) | ((x >> 4) & 0x03030303u); };
+    auto pack = [](uint32_t x) {
+        x = (x & 0x003F003Fu) | ((x >> 2) & 0x0FC00FC0u);
+        return (x & 0xFFFu) | ((x >> 4) & 0xFFF000u);
+    };
+    const uint64_t bits = (uint64_t)pack(rev(lo)) | ((uint64_t)pack(rev(hi)) << 24);
+    const uint32_t w = (uint32_t)(bits >> (2u * r)), left = L - t0;
+    return left < 16u ? w & ((1u << (2u * left)) - 1u) : w;
+}
+
 // Workgroup-wide exclusive scan of one uint32 per thread (blockDim.x <= 1024, multiple of 64).
 // `tmp` needs blockDim.x/64 + 1 words of LDS. Returns the exclusive prefix; *total gets the sum.
 // Ends with a barrier, so `tmp` may be reused at once.

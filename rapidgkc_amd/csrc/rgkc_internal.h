@@ -200,20 +200,24 @@ hipError_t launch_expand_ovf(const CountArgs& a, uint64_t n_units, hipStream_t s
 hipError_t launch_count_units(const CountArgs& a, hipStream_t s);
 hipError_t launch_count_keys(const CountArgs& a, hipStream_t s);
 
-// Side descriptors for a store that lacks them (host-provided partitions): one workgroup per
-// partition finds record starts by the full/non-full byte rule and recomputes each record's
-// minimizer from its first k-mer.
+// Side descriptors for a store that lacks them (host-provided partitions), over pieces of kIndexChunk
+// bytes: record starts by the full/non-full byte rule, each record's minimizer from its first k-mer.
+constexpr uint64_t kIndexChunk = 8192;
 struct IndexArgs {
     const uint8_t* store;
     const uint64_t* part_byte;  // [n_parts+1]
-    uint32_t n_parts;
+    uint32_t n_parts, n_chunks;
+    const uint32_t* chunk_part; // [n_chunks] partition of each piece
+    const uint32_t* part_chunk; // [n_parts+1] first piece of each partition
     int k, p, parts_total;      // parts_total: the partition count the sub-bucket id is defined over
     uint32_t* side;             // out: one per record
-    uint64_t* rec_count;        // out: records per partition (pass 1) / used as offsets (pass 2)
-    const uint64_t* rec_off;    // pass 2: record offsets per partition
+    uint64_t* chunk_n;          // [n_chunks+1] records of each piece
+    const uint64_t* chunk_rec;  // [n_chunks+1] their prefix
+    uint64_t* rec_count;        // [n_parts][2] records, k-mers
     uint32_t* err;
 };
 hipError_t launch_index_count(const IndexArgs& a, hipStream_t s);
+hipError_t launch_index_parts(const IndexArgs& a, hipStream_t s);  // rec_count[2 * i] once chunk_rec is there
 hipError_t launch_index_fill(const IndexArgs& a, hipStream_t s);
 
 // ---- row order (k_sort.hip) ------------------------------------------------------------------
