@@ -97,10 +97,13 @@ __global__ void k_seg_count_dev(const uint64_t* __restrict__ offs, const uint64_
 
 __global__ void k_seg_fill_dev(const uint64_t* __restrict__ offs, const uint64_t* __restrict__ seg_off,
                                uint64_t* __restrict__ hdr, uint64_t cap_reads, int k, uint32_t* __restrict__ seg_read,
-                               uint32_t* __restrict__ seg_first) {
+                               uint32_t* __restrict__ seg_first, uint32_t* __restrict__ n_rescan) {
     const uint64_t n = hdr[0];
     const uint64_t gid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (gid == 0) hdr[2] = seg_off[n];
+    if (gid == 0) {
+        hdr[2] = seg_off[n];
+        if (n_rescan) *n_rescan = 0;  // of this batch's count pass (a captured graph records no memset)
+    }
     for (uint64_t r = gid; r < n && r < cap_reads; r += (uint64_t)gridDim.x * blockDim.x) {
         const uint64_t len = offs[r + 1] - offs[r];
         if (len < (uint64_t)k) continue;
@@ -292,11 +295,13 @@ __global__ __launch_bounds__(T, 3) void k_p1_count(P1Args a) {
     __shared__ uint32_t lcnt, lbad;
     const int tid = threadIdx.x;
     const uint32_t lane = (uint32_t)tid & 63u;
+    const uint64_t n_seg = a.n_seg_dev ? *a.n_seg_dev : a.n_seg;
+    const uint64_t seg_lo = (uint64_t)blockIdx.x * T;
+    const uint64_t seg_hi = min(n_seg, seg_lo + T);
+    if (seg_lo >= n_seg) return;  // batched input: the grid covers the batch capacity
     for (int i = tid; i < a.parts; i += T) { hb[i] = 0; hr[i] = 0; hk[i] = 0; }
     if (tid == 0) { lcnt = 0; lbad = 0; }
     __syncthreads();
-    const uint64_t seg_lo = (uint64_t)blockIdx.x * T;
-    const uint64_t seg_hi = min(a.n_seg, seg_lo + T);
     const uint64_t s = seg_lo + (uint64_t)tid;
     const bool has = s < seg_hi;
     uint64_t pos0 = 0;
@@ -705,7 +710,10 @@ __global__ __launch_bounds__(T) void k_p1_emit_list(P1Args a) {
     __shared__ uint32_t rpos[kReorderMax];
     __shared__ uint16_t order[kReorderMax];
     __shared__ uint32_t tmp[T / 64 + 1];
-    const uint32_t wg = xcd_tile(blockIdx.x, gridDim.x);
+    const uint64_t n_seg = a.n_seg_dev ? *a.n_seg_dev : a.n_seg;
+    const uint32_t n_tiles = (uint32_t)((n_seg + T - 1) / T);  // batched input: the grid covers the batch capacity
+    if (blockIdx.x >= n_tiles) return;
+    const uint32_t wg = xcd_tile(blockIdx.x, n_tiles);
     const uint32_t n_list = a.skm_n[wg];
     if (n_list > a.skm_cap) return;  // rescanned by the scanning emit
     const int k = a.k;
@@ -758,7 +766,7 @@ __global__ __launch_bounds__(T) void k_p1_emit_list(P1Args a) {
         }
     }
     const uint64_t seg_lo = (uint64_t)wg * T;
-    const uint64_t seg_hi = min(a.n_seg, seg_lo + T);
+    const uint64_t seg_hi = min(n_seg, seg_lo + T);
     const uint64_t s = seg_lo + threadIdx.x;
     if (s < seg_hi) {
         const uint32_t rd = a.seg_read[s];
@@ -846,7 +854,7 @@ template <int RING, int T>
 __global__ __launch_bounds__(T) void k_p1_emit_stream(P1Args a) {
     __shared__ EmitLds<RING, T> L;
     const uint64_t n_seg = *a.n_seg_dev;
-    const uint64_t tiles = a.wg_map ? a.n_map : (n_seg + T - 1) / T;
+    const uint64_t tiles = a.wg_map ? (a.n_map_dev ? *a.n_map_dev : a.n_map) : (n_seg + T - 1) / T;
     for (uint64_t t = blockIdx.x; t < tiles; t += gridDim.x)
         emit_tile<RING, T, true>(a, a.wg_map ? a.wg_map[t] : (uint32_t)t, n_seg, L);
 }
@@ -889,7 +897,8 @@ hipError_t launch_p1_count(const P1Args& a, hipStream_t s) {
 
 hipError_t launch_batch_prep(const uint8_t* reads, const uint64_t* offs, uint64_t* hdr, uint64_t cap_reads,
                              uint64_t cap_bases, int k, uint32_t* bases2, uint64_t* nseg, uint64_t* seg_off,
-                             uint64_t* scan_tmp, uint32_t* seg_read, uint32_t* seg_first, hipStream_t s) {
+                             uint64_t* scan_tmp, uint32_t* seg_read, uint32_t* seg_first, uint32_t* n_rescan,
+                             hipStream_t s) {
     const uint64_t cap_words = (cap_bases >> 4) + 2;
     hipLaunchKernelGGL(k_pack_dev, dim3((unsigned)std::min<uint64_t>((cap_words + 255) / 256, 4096)), dim3(256), 0, s,
                        (const uint4*)reads, (const uint64_t*)hdr, cap_words, bases2);
@@ -900,7 +909,7 @@ hipError_t launch_batch_prep(const uint8_t* reads, const uint64_t* offs, uint64_
     if ((e = hipGetLastError())) return e;
     if ((e = scan_u64(nseg, seg_off, cap_reads + 1, scan_tmp, s))) return e;
     hipLaunchKernelGGL(k_seg_fill_dev, dim3(g), dim3(256), 0, s, offs, (const uint64_t*)seg_off, hdr, cap_reads, k,
-                       seg_read, seg_first);
+                       seg_read, seg_first, n_rescan);
     return hipGetLastError();
 }
 
@@ -927,6 +936,21 @@ hipError_t launch_p1_emit_sized(const P1Args& a, uint32_t n_rescan, hipStream_t 
     const unsigned grid = std::min(n_rescan, 1024u);
     if (!big) hipLaunchKernelGGL((k_p1_emit_stream<32, 256>), dim3(grid), dim3(256), 0, s, b);
     else hipLaunchKernelGGL((k_p1_emit_stream<64, 128>), dim3(grid), dim3(128), 0, s, b);
+    return hipGetLastError();
+}
+
+// One batch of batched input (a.n_seg_dev segments, launched over the batch capacity a.n_wg): the count
+// pass's superkmer lists, the list emit against the region cursors, and the scanning emit over the tiles
+// whose list overflowed. The scanning emit alone scanned a batch's few tiles twice with one thread per
+// segment: 0.30 ms for 26 k segments, 9.6 ms for 32 batches.
+hipError_t launch_p1_batch(const P1Args& a, hipStream_t s) {
+    hipError_t e = launch_p1_count(a, s);
+    if (e != hipSuccess) return e;
+    const bool big = (a.k - a.p + 1) > 32;
+    if ((e = launch_list(a, big, s)) != hipSuccess) return e;
+    const unsigned grid = std::min(a.n_wg, 256u);
+    if (!big) hipLaunchKernelGGL((k_p1_emit_stream<32, 256>), dim3(grid), dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((k_p1_emit_stream<64, 128>), dim3(grid), dim3(128), 0, s, a);
     return hipGetLastError();
 }
 

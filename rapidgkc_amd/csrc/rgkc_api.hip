@@ -1554,8 +1554,9 @@ static int stream_enqueue(rgkc_ctx* c) {
     HIPC(c, launch_batch_prep(c->reads.as<uint8_t>(), c->offs.as<uint64_t>(), c->hdr.as<uint64_t>(), c->cap_reads,
                               c->cap_bases, c->k, c->bases2.as<uint32_t>(), c->nseg.as<uint64_t>(),
                               c->seg_off.as<uint64_t>(), c->scan_tmp.as<uint64_t>(), c->seg_read.as<uint32_t>(),
-                              c->seg_first.as<uint32_t>(), s));
-    HIPC(c, launch_p1_emit_stream(c->sargs, 512, s));
+                              c->seg_first.as<uint32_t>(), c->sargs.n_rescan, s));
+    if (c->sargs.skm_list) HIPC(c, launch_p1_batch(c->sargs, s));
+    else HIPC(c, launch_p1_emit_stream(c->sargs, 512, s));
     return 0;
 }
 
@@ -1703,6 +1704,22 @@ int rgkc_stream_begin(rgkc_ctx* c, int k, int p, int parts, uint64_t max_reads, 
     a.k = k; a.p = p; a.parts = parts;
     region_args(c, a);
     a.n_seg_dev = c->hdr.as<uint64_t>() + 2;
+    if (c->list_cap != 0xFFFFFFFFu) {
+        // superkmer lists and tile histograms of one batch
+        const int T1 = p1_threads(k, p);
+        const uint32_t n_wg = (uint32_t)((max_seg + T1 - 1) / T1);
+        const size_t hwords = (size_t)parts * ((size_t)n_wg + 1);
+        NEED(c, c->hist, 3 * hwords * 4);
+        a.n_seg = max_seg;
+        a.h_bytes = c->hist.as<uint32_t>();
+        a.h_recs = a.h_bytes + hwords;
+        a.h_kmers = a.h_recs + hwords;
+        a.n_wg = n_wg;
+        if (int r = setup_lists(c, a, T1, n_wg)) return r;
+        a.list_reserve = 1;
+        a.wg_map = a.wg_rescan;
+        a.n_map_dev = a.n_rescan;
+    }
     HIPC(c, hipStreamSynchronize(s));
     c->stream_graph = use_graph != 0;
     if (c->stream_graph) {

@@ -96,6 +96,7 @@ struct P1Args {
     uint32_t* n_listorder;      // list emit: tiles with too many entries for store order (written in list order)
     const uint32_t* wg_map;     // scanning emit: tile of each workgroup (nullptr: blockIdx.x)
     uint32_t n_map;             // persistent scanning emit: tiles in wg_map
+    const uint32_t* n_map_dev;  // their number on the device instead (batched input)
     uint32_t list_reserve;      // list emit: reserve each tile's runs with pos_cursor from its raw
                                 // histogram columns (capacity-sized regions) instead of exact offsets
 };
@@ -110,10 +111,12 @@ hipError_t launch_p1_emit_stream(const P1Args& a, unsigned grid, hipStream_t s);
 // the persistent scanning emit over the n_rescan tiles whose list overflowed (a.wg_map).
 hipError_t launch_p1_emit_sized(const P1Args& a, uint32_t n_rescan, hipStream_t s);
 // Batched input: pack + segment table from a device header ([0] reads, [1] bases; [2] set to the
-// segment count), all launched over the batch capacity.
+// segment count; *n_rescan cleared), all launched over the batch capacity.
 hipError_t launch_batch_prep(const uint8_t* reads, const uint64_t* offs, uint64_t* hdr, uint64_t cap_reads,
                              uint64_t cap_bases, int k, uint32_t* bases2, uint64_t* nseg, uint64_t* seg_off,
-                             uint64_t* scan_tmp, uint32_t* seg_read, uint32_t* seg_first, hipStream_t s);
+                             uint64_t* scan_tmp, uint32_t* seg_read, uint32_t* seg_first, uint32_t* n_rescan,
+                             hipStream_t s);
+hipError_t launch_p1_batch(const P1Args& a, hipStream_t s);
 
 // ---- count (k_group.hip, k_count.hip) ----------------------------------------------------------
 // A unit of more than this many unit_caps is expanded into keys: at 30x, 1.2 G k-mers, the count stage
