@@ -153,6 +153,7 @@ struct rgkc_ctx {
     uint64_t* h_offs_stage[2] = {nullptr, nullptr};
     hipEvent_t stage_ev[2] = {nullptr, nullptr};
     bool stage_ev_rec[2] = {false, false};
+    uint64_t stage_bytes = 0, stage_reads = 0;  // their capacity: read bytes, offsets
     uint64_t last_batch_bases = 0;   // bases of the batch now in the device read buffer
     hipGraph_t graph = nullptr;
     hipGraphExec_t gexec = nullptr;
@@ -1067,12 +1068,14 @@ int rgkc_create(int device, rgkc_ctx** out) {
 }
 
 static int stream_free(rgkc_ctx* c);
+static void stage_free(rgkc_ctx* c);
 
 int rgkc_destroy(rgkc_ctx* c) {
     if (!c) return 0;
     (void)hipSetDevice(c->device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     stream_free(c);
+    stage_free(c);
     for (int i = 0; i < EV_N; i++) if (c->ev[i]) (void)hipEventDestroy(c->ev[i]);
     if (c->plan_ev) (void)hipEventDestroy(c->plan_ev);
     if (c->h_plan) (void)hipHostFree(c->h_plan);
@@ -1537,15 +1540,38 @@ static int stream_free(rgkc_ctx* c) {
     (void)hipStreamSynchronize(c->stream);  // uploads from the staging sets may be in flight
     if (c->gexec) { (void)hipGraphExecDestroy(c->gexec); c->gexec = nullptr; }
     if (c->graph) { (void)hipGraphDestroy(c->graph); c->graph = nullptr; }
+    for (int i = 0; i < 2; i++) c->stage_ev_rec[i] = false;
+    (void)hipGetLastError();
+    c->stream_on = false;
+    return 0;
+}
+
+static void stage_free(rgkc_ctx* c) {
     for (int i = 0; i < 2; i++) {
         if (c->h_hdr[i]) { (void)hipHostFree(c->h_hdr[i]); c->h_hdr[i] = nullptr; }
         if (c->h_stage[i]) { (void)hipHostFree(c->h_stage[i]); c->h_stage[i] = nullptr; }
         if (c->h_offs_stage[i]) { (void)hipHostFree(c->h_offs_stage[i]); c->h_offs_stage[i] = nullptr; }
         if (c->stage_ev[i]) { (void)hipEventDestroy(c->stage_ev[i]); c->stage_ev[i] = nullptr; }
-        c->stage_ev_rec[i] = false;
     }
     (void)hipGetLastError();
-    c->stream_on = false;
+    c->stage_bytes = c->stage_reads = 0;
+}
+
+// The two pinned staging sets, kept by the context from stream to stream (grow-only like its device
+// buffers): allocated and freed with each stream, they cost up to 9 ms of a 20 ms pass over 32 batches.
+static int stage_need(rgkc_ctx* c, uint64_t bytes, uint64_t reads) {
+    if (bytes <= c->stage_bytes && reads <= c->stage_reads) return 0;
+    bytes = std::max(bytes, c->stage_bytes);
+    reads = std::max(reads, c->stage_reads);
+    stage_free(c);
+    for (int i = 0; i < 2; i++) {
+        HIPC(c, hipHostMalloc((void**)&c->h_hdr[i], 64, hipHostMallocDefault));
+        HIPC(c, hipHostMalloc((void**)&c->h_stage[i], bytes, hipHostMallocDefault));
+        HIPC(c, hipHostMalloc((void**)&c->h_offs_stage[i], reads * 8, hipHostMallocDefault));
+        HIPC(c, hipEventCreateWithFlags(&c->stage_ev[i], hipEventDisableTiming));
+    }
+    c->stage_bytes = bytes;
+    c->stage_reads = reads;
     return 0;
 }
 
@@ -1683,15 +1709,7 @@ int rgkc_stream_begin(rgkc_ctx* c, int k, int p, int parts, uint64_t max_reads, 
     HIPC(c, hipMemsetAsync(c->reads.p, 0, n_words * 16, s));
     HIPC(c, hipMemsetAsync(c->bases2.p, 0, (n_words + 2) * 4, s));
     HIPC(c, hipMemsetAsync(c->err_word.p, 0, 64, s));
-    for (int i = 0; i < 2; i++) {
-        HIPC(c, hipHostMalloc((void**)&c->h_hdr[i], 64, hipHostMallocDefault));
-        HIPC(c, hipHostMalloc((void**)&c->h_stage[i], n_words * 16, hipHostMallocDefault));
-        HIPC(c, hipHostMalloc((void**)&c->h_offs_stage[i], (max_reads + 1) * 8, hipHostMallocDefault));
-        HIPC(c, hipEventCreateWithFlags(&c->stage_ev[i], hipEventDisableTiming));
-        c->stage_ev_rec[i] = false;
-        memset(c->h_stage[i], 0, n_words * 16);
-        memset(c->h_hdr[i], 0, 64);
-    }
+    if (int r = stage_need(c, n_words * 16, max_reads + 1)) return r;
     c->last_batch_bases = 0;
     if (int r = setup_regions(c, cap_bytes, cap_recs)) return r;
     P1Args& a = c->sargs;
