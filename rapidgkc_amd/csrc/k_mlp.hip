@@ -1,6 +1,6 @@
 // Load predictor network on gfx950: a 3-layer MLP (ReLU) with BF16 weights and FP32
-// accumulation, trained with masked MSE and Adam. Small and off the counting path's critical
-// path; the kernels are plain LDS-tiled GEMMs (64x64 tiles, 4x4 per thread).
+// accumulation, trained with masked MSE and Adam. Training batches go row by row in three launches;
+// larger ones through plain LDS-tiled GEMMs (64x64 tiles, 4x4 per thread).
 //
 // Parameters (flat FP32 master copy, the BF16 copy is what the GEMMs read):
 //   W1[n_in x h1] b1[h1] W2[h1 x h2] b2[h2] W3[h2 x n_out] b3[n_out]   (row-major, x @ W)
@@ -127,6 +127,166 @@ __global__ void k_to_bf16(size_t n, const float* __restrict__ w, __hip_bfloat16*
     if (i < n) wb[i] = __float2bfloat16(w[i]);
 }
 
+// ---- batches of at most kRowBatch rows: three launches ------------------------------------------------
+// A training batch is 16 to 64 rows, so the layers are vector-matrix products whose cost is latency: as
+// GEMMs of 64 x 64 tiles over the whole K, two workgroups walked layer 1's 2563 inputs in 160 steps
+// (0.57 ms of 16 launches for the gradient of 16 rows, n_in 2563, 128 x 128 hidden, 1024 out). Instead:
+//   k_rows_in    layer 1's products, split over K: a workgroup takes kKC inputs x 64 outputs of up to 64
+//                rows and leaves partial sums (summed in a fixed order by the next kernel);
+//   k_rows_net   one workgroup per row: the rest of the forward pass, the loss and the activations'
+//                gradients, row vectors in LDS, weights read once per row (they stay in L2);
+//   k_rows_grad  a thread per parameter sums its gradient over the rows.
+// All sums in FP32 as before, in shorter chains.
+constexpr int kKC = 32;
+constexpr int kRowThreads = 1024;
+
+__global__ __launch_bounds__(256) void k_rows_in(int B, int n_in, int h1, const float* __restrict__ X,
+                                                 const __hip_bfloat16* __restrict__ W, float* __restrict__ part) {
+    __shared__ float xs[kKC][65];
+    __shared__ float ws[kKC][64];
+    const int n0 = blockIdx.x * 64, k0 = blockIdx.y * kKC, b0 = blockIdx.z * 64;
+    const int kn = min(kKC, n_in - k0), bn = min(64, B - b0);
+    for (int i = threadIdx.x; i < 64 * kKC; i += 256) {
+        const int b = i / kKC, kk = i % kKC;
+        xs[kk][b] = (b < bn && kk < kn) ? X[(size_t)(b0 + b) * n_in + k0 + kk] : 0.f;
+        const int n = i % 64, kw = i / 64;
+        ws[kw][n] = (n0 + n < h1 && kw < kn) ? __bfloat162float(W[(size_t)(k0 + kw) * h1 + n0 + n]) : 0.f;
+    }
+    __syncthreads();
+    const int n = threadIdx.x & 63, r0 = threadIdx.x >> 6;
+    float acc[16] = {};
+    for (int kk = 0; kk < kKC; kk++) {
+        const float w = ws[kk][n];
+#pragma unroll
+        for (int i = 0; i < 16; i++)
+            if (4 * i < bn) acc[i] = fmaf(xs[kk][r0 + 4 * i], w, acc[i]);
+    }
+    if (n0 + n >= h1) return;
+#pragma unroll
+    for (int i = 0; i < 16; i++)
+        if (r0 + 4 * i < bn) part[((size_t)blockIdx.y * B + b0 + r0 + 4 * i) * h1 + n0 + n] = acc[i];
+}
+
+// out[n] = sum_k f(k, n) for n < N, k < K; all threads call it. With fewer outputs than threads, groups of
+// threads share K and their sums are added in group order. `red` holds kRowThreads floats.
+template <typename F, typename O>
+__device__ __forceinline__ void row_sum(int K, int N, float* red, F f, O out) {
+    const int G = N < kRowThreads ? max(1, min(K, kRowThreads / N)) : 1;
+    for (int n0 = 0; n0 < N; n0 += kRowThreads) {
+        const int nn = min(N - n0, kRowThreads);
+        const int n = (int)threadIdx.x % nn, g = (int)threadIdx.x / nn;
+        if (g < G) {
+            float s = 0.f;
+#pragma unroll 8
+            for (int k = g; k < K; k += G) s += f(k, n0 + n);
+            red[threadIdx.x] = s;
+        }
+        __syncthreads();
+        if ((int)threadIdx.x < nn) {
+            float s = red[threadIdx.x];
+            for (int q = 1; q < G; q++) s += red[q * nn + (int)threadIdx.x];
+            out(n0 + (int)threadIdx.x, s);
+        }
+        __syncthreads();
+    }
+}
+
+// out(j, sum_n W[j][n] v[n]) for j < J, a wave per j
+template <typename O>
+__device__ __forceinline__ void row_dot(int J, int N, const __hip_bfloat16* W, const float* v, O out) {
+    for (int j = threadIdx.x >> 6; j < J; j += kRowThreads / 64) {
+        float s = 0.f;
+#pragma unroll 8
+        for (int n = threadIdx.x & 63; n < N; n += 64) s = fmaf(__bfloat162float(W[(size_t)j * N + n]), v[n], s);
+        for (int o = 32; o > 0; o >>= 1) s += __shfl_down(s, o, 64);
+        if ((threadIdx.x & 63) == 0) out(j, s);
+    }
+    __syncthreads();
+}
+
+// T null: forward only. row_loss[b] receives the row's share of the masked MSE.
+__global__ __launch_bounds__(kRowThreads) void k_rows_net(MlpDims d, int B, int S, const __hip_bfloat16* __restrict__ W,
+                                                          const float* __restrict__ w32, const float* __restrict__ part,
+                                                          const float* __restrict__ T, const float* __restrict__ mask,
+                                                          float inv_cnt, float* __restrict__ H1, float* __restrict__ H2,
+                                                          float* __restrict__ Y, float* __restrict__ dY,
+                                                          float* __restrict__ dH1, float* __restrict__ dH2,
+                                                          float* __restrict__ row_loss) {
+    extern __shared__ float dyn[];
+    float *const red = dyn, *const v1 = red + kRowThreads, *const v2 = v1 + d.h1, *const vo = v2 + d.h2;
+    const size_t b = blockIdx.x;
+    const __hip_bfloat16 *const W2 = W + d.off_W2(), *const W3 = W + d.off_W3();
+    const float *const b1 = w32 + d.off_b1(), *const b2 = w32 + d.off_b2(), *const b3 = w32 + d.off_b3();
+    row_sum(S, d.h1, red, [&](int s, int n) { return part[((size_t)s * B + b) * d.h1 + n]; },
+            [&](int n, float x) {
+                x += b1[n];
+                v1[n] = x > 0.f ? x : 0.f;
+                H1[b * d.h1 + n] = v1[n];
+            });
+    row_sum(d.h1, d.h2, red, [&](int k, int n) { return v1[k] * __bfloat162float(W2[(size_t)k * d.h2 + n]); },
+            [&](int n, float x) {
+                x += b2[n];
+                v2[n] = x > 0.f ? x : 0.f;
+                H2[b * d.h2 + n] = v2[n];
+            });
+    float l = 0.f;
+    row_sum(d.h2, d.n_out, red, [&](int k, int n) { return v2[k] * __bfloat162float(W3[(size_t)k * d.n_out + n]); },
+            [&](int n, float x) {
+                const size_t i = b * d.n_out + n;
+                x += b3[n];
+                Y[i] = x;
+                if (T) {
+                    const float e = (x - T[i]) * (mask ? mask[i] : 1.f);
+                    vo[n] = 2.f * e * inv_cnt;
+                    dY[i] = vo[n];
+                    l += e * e * inv_cnt;
+                }
+            });
+    if (!T) return;
+    red[threadIdx.x] = l;
+    __syncthreads();
+    for (int o = kRowThreads / 2; o > 0; o >>= 1) {
+        if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) row_loss[b] = red[0];
+    row_dot(d.h2, d.n_out, W3, vo, [&](int j, float x) {
+        v2[j] = v2[j] > 0.f ? x : 0.f;
+        dH2[b * d.h2 + j] = v2[j];
+    });
+    row_dot(d.h1, d.h2, W2, v2, [&](int j, float x) { dH1[b * d.h1 + j] = v1[j] > 0.f ? x : 0.f; });
+}
+
+__global__ __launch_bounds__(256) void k_rows_grad(MlpDims d, int B, const float* __restrict__ X, const float* __restrict__ H1,
+                                                   const float* __restrict__ H2, const float* __restrict__ dY,
+                                                   const float* __restrict__ dH1, const float* __restrict__ dH2,
+                                                   const float* __restrict__ row_loss, float* __restrict__ G,
+                                                   float* __restrict__ loss) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i == 0) {
+        float l = 0.f;
+        for (int b = 0; b < B; b++) l += row_loss[b];
+        *loss = l;
+    }
+    if (i >= d.total()) return;
+    // the parameter's layer: inputs A (ones for a bias), output gradients D of width N
+    const float *A, *D;
+    size_t o;
+    int K, N;
+    if (i < d.off_W2()) { A = X; D = dH1; o = i; K = d.n_in; N = d.h1; }
+    else if (i < d.off_W3()) { A = H1; D = dH2; o = i - d.off_W2(); K = d.h1; N = d.h2; }
+    else { A = H2; D = dY; o = i - d.off_W3(); K = d.h2; N = d.n_out; }
+    const int kk = (int)(o / N), n = (int)(o % N);
+    float s = 0.f;
+    if (kk < K) {
+#pragma unroll 8
+        for (int b = 0; b < B; b++) s = fmaf(A[(size_t)b * K + kk], D[(size_t)b * N + n], s);
+    } else {
+        for (int b = 0; b < B; b++) s += D[(size_t)b * N + n];
+    }
+    G[i] = s;
+}
+
 template <bool TA, bool TB, typename BT>
 hipError_t gemm(int M, int N, int K, const float* A, int lda, const BT* B, int ldb, float* C, int ldc, const float* bias,
                 bool relu, bool acc, hipStream_t s) {
@@ -143,6 +303,30 @@ inline unsigned nblk(size_t n) { return (unsigned)((n + 255) / 256); }
 // ---- host-side operations on device buffers (called by the C ABI layer) --------------------
 hipError_t mlp_to_bf16(const float* w, void* wb, size_t n, hipStream_t s) {
     hipLaunchKernelGGL(k_to_bf16, dim3(nblk(n)), dim3(256), 0, s, n, w, (__hip_bfloat16*)wb);
+    return hipGetLastError();
+}
+
+// Batches that go row by row: up to kRowBatch rows whose vectors fit a workgroup's LDS.
+constexpr int kRowBatch = 1024;
+static size_t row_lds(const MlpDims& d) { return ((size_t)kRowThreads + d.h1 + d.h2 + d.n_out) * 4; }
+bool mlp_by_rows(const MlpDims& d, int B) { return B <= kRowBatch && row_lds(d) <= 60 * 1024; }
+size_t mlp_part_floats(const MlpDims& d, int B) { return (size_t)((d.n_in + kKC - 1) / kKC) * B * d.h1; }
+
+hipError_t mlp_rows_forward(const MlpDims& d, const void* wb, const float* w32, const float* X, int B, float* part,
+                            const float* T, const float* mask, float mask_sum, float* H1, float* H2, float* Y, float* dY,
+                            float* dH1, float* dH2, float* row_loss, hipStream_t s) {
+    const __hip_bfloat16* W = (const __hip_bfloat16*)wb;
+    const int S = (d.n_in + kKC - 1) / kKC;
+    hipLaunchKernelGGL(k_rows_in, dim3((d.h1 + 63) / 64, S, (B + 63) / 64), dim3(256), 0, s, B, d.n_in, d.h1, X, W + d.off_W1(),
+                       part);
+    hipLaunchKernelGGL(k_rows_net, dim3(B), dim3(kRowThreads), row_lds(d), s, d, B, S, W, w32, (const float*)part, T, mask,
+                       1.f / (mask_sum > 1.f ? mask_sum : 1.f), H1, H2, Y, dY, dH1, dH2, row_loss);
+    return hipGetLastError();
+}
+
+hipError_t mlp_rows_grad(const MlpDims& d, const float* X, int B, const float* H1, const float* H2, const float* dY,
+                         const float* dH1, const float* dH2, const float* row_loss, float* G, float* loss, hipStream_t s) {
+    hipLaunchKernelGGL(k_rows_grad, dim3(nblk(d.total())), dim3(256), 0, s, d, B, X, H1, H2, dY, dH1, dH2, row_loss, G, loss);
     return hipGetLastError();
 }
 

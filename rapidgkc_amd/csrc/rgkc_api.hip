@@ -1879,7 +1879,7 @@ int rgkc_sample_features(rgkc_ctx* c, int k, int p, int parts, uint32_t* hist, u
 struct rgkc_mlp {
     rgkc_ctx* c = nullptr;
     MlpDims d;
-    DevBuf w32, wb, g, m1, m2, X, T, M, H1, H2, Y, dY, dH1, dH2, loss;
+    DevBuf w32, wb, g, m1, m2, X, T, M, H1, H2, Y, dY, dH1, dH2, loss, part;
     int step = 0;
 };
 
@@ -1934,16 +1934,50 @@ int rgkc_mlp_get_params(rgkc_mlp* m, float* p) {
     return 0;
 }
 
-static int mlp_stage_fwd(rgkc_mlp* m, const float* x, int B) {
+// Inputs to the device and the forward pass; with targets (and an optional mask), the backward pass as well.
+static int mlp_stage(rgkc_mlp* m, const float* x, const float* t, const float* mask, int B, float* loss) {
     rgkc_ctx* c = m->c;
     const MlpDims& d = m->d;
+    hipStream_t s = c->stream;
+    const size_t nY = (size_t)B * d.n_out;
+    const bool rows = mlp_by_rows(d, B);
     NEED(c, m->X, (size_t)B * d.n_in * 4);
     NEED(c, m->H1, (size_t)B * d.h1 * 4);
     NEED(c, m->H2, (size_t)B * d.h2 * 4);
-    NEED(c, m->Y, (size_t)B * d.n_out * 4);
-    HIPC(c, hipMemcpyAsync(m->X.p, x, (size_t)B * d.n_in * 4, hipMemcpyHostToDevice, c->stream));
-    HIPC(c, mlp_forward(d, m->wb.p, m->w32.as<float>(), m->X.as<float>(), B, m->H1.as<float>(), m->H2.as<float>(),
-                        m->Y.as<float>(), c->stream));
+    NEED(c, m->Y, nY * 4);
+    if (rows) NEED(c, m->part, (mlp_part_floats(d, B) + B) * 4);
+    HIPC(c, hipMemcpyAsync(m->X.p, x, (size_t)B * d.n_in * 4, hipMemcpyHostToDevice, s));
+    float msum = (float)nY;
+    if (t) {
+        NEED(c, m->T, nY * 4);
+        NEED(c, m->dY, nY * 4);
+        NEED(c, m->dH1, (size_t)B * d.h1 * 4);
+        NEED(c, m->dH2, (size_t)B * d.h2 * 4);
+        if (mask) {
+            NEED(c, m->M, nY * 4);
+            double sm = 0;
+            for (size_t i = 0; i < nY; i++) sm += mask[i];
+            msum = (float)sm;
+            HIPC(c, hipMemcpyAsync(m->M.p, mask, nY * 4, hipMemcpyHostToDevice, s));
+        }
+        HIPC(c, hipMemcpyAsync(m->T.p, t, nY * 4, hipMemcpyHostToDevice, s));
+    }
+    float *const X = m->X.as<float>(), *const H1 = m->H1.as<float>(), *const H2 = m->H2.as<float>();
+    float *const dY = m->dY.as<float>(), *const dH1 = m->dH1.as<float>(), *const dH2 = m->dH2.as<float>();
+    const float* const T = t ? m->T.as<float>() : nullptr;
+    const float* const M = t && mask ? m->M.as<float>() : nullptr;
+    if (rows) {
+        float* const row_loss = m->part.as<float>() + mlp_part_floats(d, B);
+        HIPC(c, mlp_rows_forward(d, m->wb.p, m->w32.as<float>(), X, B, m->part.as<float>(), T, M, msum, H1, H2,
+                                 m->Y.as<float>(), dY, dH1, dH2, row_loss, s));
+        if (t) HIPC(c, mlp_rows_grad(d, X, B, H1, H2, dY, dH1, dH2, row_loss, m->g.as<float>(), m->loss.as<float>(), s));
+    } else {
+        HIPC(c, mlp_forward(d, m->wb.p, m->w32.as<float>(), X, B, H1, H2, m->Y.as<float>(), s));
+        if (t)
+            HIPC(c, mlp_backward(d, m->wb.p, X, B, H1, H2, m->Y.as<float>(), T, M, msum, dY, dH1, dH2, m->g.as<float>(),
+                                 m->loss.as<float>(), s));
+    }
+    if (t && loss) HIPC(c, hipMemcpyAsync(loss, m->loss.p, 4, hipMemcpyDeviceToHost, s));
     return 0;
 }
 
@@ -1952,33 +1986,9 @@ int rgkc_mlp_forward(rgkc_mlp* m, const float* x, int B, float* y) {
     rgkc_ctx* c = m->c;
     (void)hipGetLastError();
     HIPC(c, hipSetDevice(c->device));
-    if (int r = mlp_stage_fwd(m, x, B)) return r;
+    if (int r = mlp_stage(m, x, nullptr, nullptr, B, nullptr)) return r;
     HIPC(c, hipMemcpyAsync(y, m->Y.p, (size_t)B * m->d.n_out * 4, hipMemcpyDeviceToHost, c->stream));
     HIPC(c, hipStreamSynchronize(c->stream));
-    return 0;
-}
-
-static int mlp_stage_bwd(rgkc_mlp* m, const float* t, const float* mask, int B, float* loss) {
-    rgkc_ctx* c = m->c;
-    const MlpDims& d = m->d;
-    const size_t nY = (size_t)B * d.n_out;
-    NEED(c, m->T, nY * 4);
-    NEED(c, m->dY, nY * 4);
-    NEED(c, m->dH1, (size_t)B * d.h1 * 4);
-    NEED(c, m->dH2, (size_t)B * d.h2 * 4);
-    float msum = (float)nY;
-    if (mask) {
-        NEED(c, m->M, nY * 4);
-        double sm = 0;
-        for (size_t i = 0; i < nY; i++) sm += mask[i];
-        msum = (float)sm;
-        HIPC(c, hipMemcpyAsync(m->M.p, mask, nY * 4, hipMemcpyHostToDevice, c->stream));
-    }
-    HIPC(c, hipMemcpyAsync(m->T.p, t, nY * 4, hipMemcpyHostToDevice, c->stream));
-    HIPC(c, mlp_backward(d, m->wb.p, m->X.as<float>(), B, m->H1.as<float>(), m->H2.as<float>(), m->Y.as<float>(),
-                         m->T.as<float>(), mask ? m->M.as<float>() : nullptr, msum, m->dY.as<float>(),
-                         m->dH1.as<float>(), m->dH2.as<float>(), m->g.as<float>(), m->loss.as<float>(), c->stream));
-    if (loss) HIPC(c, hipMemcpyAsync(loss, m->loss.p, 4, hipMemcpyDeviceToHost, c->stream));
     return 0;
 }
 
@@ -1987,8 +1997,7 @@ int rgkc_mlp_grad(rgkc_mlp* m, const float* x, const float* t, const float* mask
     rgkc_ctx* c = m->c;
     (void)hipGetLastError();
     HIPC(c, hipSetDevice(c->device));
-    if (int r = mlp_stage_fwd(m, x, B)) return r;
-    if (int r = mlp_stage_bwd(m, t, mask, B, loss)) return r;
+    if (int r = mlp_stage(m, x, t, mask, B, loss)) return r;
     if (grad) HIPC(c, hipMemcpyAsync(grad, m->g.p, m->d.total() * 4, hipMemcpyDeviceToHost, c->stream));
     HIPC(c, hipStreamSynchronize(c->stream));
     return 0;
@@ -2000,8 +2009,7 @@ int rgkc_mlp_train_step(rgkc_mlp* m, const float* x, const float* t, const float
     rgkc_ctx* c = m->c;
     (void)hipGetLastError();
     HIPC(c, hipSetDevice(c->device));
-    if (int r = mlp_stage_fwd(m, x, B)) return r;
-    if (int r = mlp_stage_bwd(m, t, mask, B, loss)) return r;
+    if (int r = mlp_stage(m, x, t, mask, B, loss)) return r;
     m->step++;
     HIPC(c, mlp_adam(m->d.total(), m->w32.as<float>(), m->wb.p, m->g.as<float>(), m->m1.as<float>(),
                      m->m2.as<float>(), lr, m->step, wd, c->stream));

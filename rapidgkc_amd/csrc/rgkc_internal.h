@@ -256,13 +256,13 @@ hipError_t launch_sort_scatter(const SortArgs& a, uint32_t n_chunks, int key_byt
 // Flat parameter layout: W1[n_in x h1] b1[h1] W2[h1 x h2] b2[h2] W3[h2 x n_out] b3[n_out].
 struct MlpDims {
     int n_in = 0, h1 = 0, h2 = 0, n_out = 0;
-    size_t off_W1() const { return 0; }
-    size_t off_b1() const { return (size_t)n_in * h1; }
-    size_t off_W2() const { return off_b1() + h1; }
-    size_t off_b2() const { return off_W2() + (size_t)h1 * h2; }
-    size_t off_W3() const { return off_b2() + h2; }
-    size_t off_b3() const { return off_W3() + (size_t)h2 * n_out; }
-    size_t total() const { return off_b3() + n_out; }
+    __host__ __device__ size_t off_W1() const { return 0; }
+    __host__ __device__ size_t off_b1() const { return (size_t)n_in * h1; }
+    __host__ __device__ size_t off_W2() const { return off_b1() + h1; }
+    __host__ __device__ size_t off_b2() const { return off_W2() + (size_t)h1 * h2; }
+    __host__ __device__ size_t off_W3() const { return off_b2() + h2; }
+    __host__ __device__ size_t off_b3() const { return off_W3() + (size_t)h2 * n_out; }
+    __host__ __device__ size_t total() const { return off_b3() + n_out; }
 };
 hipError_t mlp_to_bf16(const float* w, void* wb, size_t n, hipStream_t s);
 hipError_t mlp_forward(const MlpDims& d, const void* wb, const float* w32, const float* X, int B, float* H1, float* H2,
@@ -270,6 +270,16 @@ hipError_t mlp_forward(const MlpDims& d, const void* wb, const float* w32, const
 hipError_t mlp_backward(const MlpDims& d, const void* wb, const float* X, int B, const float* H1, const float* H2,
                         const float* Y, const float* T, const float* mask, float mask_sum, float* dY, float* dH1,
                         float* dH2, float* G, float* loss, hipStream_t s);
+// The same for batches that go row by row (mlp_by_rows): `part` holds mlp_part_floats, row_loss B floats.
+// T null: forward only; else the activations' gradients and each row's loss too, from which mlp_rows_grad
+// makes the parameters' gradients and the loss.
+bool mlp_by_rows(const MlpDims& d, int B);
+size_t mlp_part_floats(const MlpDims& d, int B);
+hipError_t mlp_rows_forward(const MlpDims& d, const void* wb, const float* w32, const float* X, int B, float* part,
+                            const float* T, const float* mask, float mask_sum, float* H1, float* H2, float* Y, float* dY,
+                            float* dH1, float* dH2, float* row_loss, hipStream_t s);
+hipError_t mlp_rows_grad(const MlpDims& d, const float* X, int B, const float* H1, const float* H2, const float* dY,
+                         const float* dH1, const float* dH2, const float* row_loss, float* G, float* loss, hipStream_t s);
 hipError_t mlp_adam(size_t n, float* w, void* wb, const float* g, float* m1, float* m2, float lr, int step, float wd,
                     hipStream_t s);
 
