@@ -43,8 +43,8 @@ typedef struct {
     uint32_t fallbacks;         /* partitions whose predicted table region overflowed (counted again, exactly) */
     uint32_t err_bits;
     uint32_t p1_rescans;        /* phase-1 tiles whose superkmer list overflowed (rescanned by the emit pass) */
-    uint32_t heavy_groups;      /* count: record groups whose heavy sub-buckets were expanded into keys */
-    float expand_ms;            /* count: key expansion of heavy sub-buckets (k_expand); count_ms is k_count_items */
+    uint32_t heavy_groups;      /* count: heavy sub-buckets expanded into keys */
+    float expand_ms;            /* count: key expansion of heavy sub-buckets (k_expand); count_ms is the count kernels */
     uint32_t p1_list_order;     /* phase-1 tiles with too many superkmers to write in store order (list order) */
     uint64_t ovf_keys;          /* count: key slots of the exact second-pass regions (slices that overflowed) */
     uint32_t count_groups;      /* count: partition groups counted one after another to fit the device memory */
@@ -154,8 +154,7 @@ int rgkc_stream_end(rgkc_ctx* ctx, uint64_t* part_bytes, uint64_t* skm_cnt, uint
  * at every limit. */
 int rgkc_set_memory_limit(rgkc_ctx* ctx, uint64_t bytes);
 
-/* Tunables (0 = default): resident workgroups per CU of the persistent count kernel (1..4; its LDS
- * table allows four). Chosen by the autotuner (rapidgkc_amd/autotune.py). */
+/* Accepted and without effect: one workgroup of the count kernel takes a CU's LDS (per_cu 0..4). */
 int rgkc_set_count_workgroups(rgkc_ctx* ctx, uint32_t per_cu);
 
 /* Tunables (0 = default): instances planned per count sweep. */
@@ -166,10 +165,10 @@ int rgkc_set_tuning(rgkc_ctx* ctx, uint32_t inst_per_sweep);
  * random sequence gives), UINT32_MAX = no lists (the emit pass always scans). Lists that would
  * take more than half the free device memory are skipped by themselves. */
 int rgkc_set_p1_lists(rgkc_ctx* ctx, uint32_t list_cap);
-/* Heavy sub-buckets (more k-mer instances than one count work item; no counterpart in the
- * reference): mode 0 (default) extracts their keys once into per-hash-slice regions when half the
- * free device memory holds them, so each slice's sweep reads keys instead of every record of the
- * sub-bucket; mode 1 always reads records. */
+/* Heavy sub-buckets (more k-mer instances than two count sweeps; no counterpart in the reference):
+ * mode 0 (default) extracts their keys once into per-hash-slice regions when the device memory holds
+ * them, so each slice's sweep reads keys instead of every record of the sub-bucket; mode 1 always
+ * reads records. */
 int rgkc_set_heavy_expand(rgkc_ctx* ctx, int mode);
 
 /* Features of a read sample for the learned sizing (no counterpart in the reference): runs phase 1

@@ -3,18 +3,17 @@
 Tuned (all results are identical in every setting; only the time changes):
   - `inst_cap`: k-mer instances planned per count sweep (the LDS table's work item). Small sweeps
     pay the per-sweep fixed work more often; large ones overflow the table and are split.
-  - `count_wg_per_cu`: resident workgroups per CU of the persistent count kernel (1 or 2: its 81 KB
-    of LDS allows two).
   - `p1_lists`: whether phase 1 keeps superkmer lists for its emit pass (on: one scan of the reads
     and a list region of ~1.25 B per k-mer; off: the emit pass scans the reads again).
 
-The search is coordinate-wise: phase-1 lists on the phase-1 time, then the sweep size and the
-workgroups per CU on the count stage's time (grouping + plan + expansion + count, HIP events),
-each candidate timed `reps` times on the resident batch, the fastest kept. Results are cached per
-(device, k, p, parts, log2 of the batch's k-mers) in a text file next to the library, one line per
-shape, which the standalone CLI (host/rgkc_main.cpp) reads as well:
+The search is coordinate-wise: phase-1 lists on the phase-1 time, then the sweep size on the count
+stage's time (grouping + plan + expansion + count, HIP events), each candidate timed `reps` times on
+the resident batch, the fastest kept. (`count_wg_per_cu` stays 0: one workgroup of the count kernel
+takes a CU's LDS.) Results are cached per (device, k, p, parts, log2 of the batch's k-mers) in a text
+file next to the library, one line per shape, which the standalone CLI (host/rgkc_main.cpp) reads as
+well. The 2 in the shape's name is the count kernel's: sweep sizes tuned for another one are not read.
 
-    gfx950:k31:p11:parts512:n31 inst_cap=8192 count_wg_per_cu=2 p1_lists=1
+    gfx950.2:k31:p11:parts512:n31 inst_cap=16384 count_wg_per_cu=0 p1_lists=1
 """
 from __future__ import annotations
 
@@ -27,7 +26,7 @@ CACHE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "autotune_cache
 
 
 def shape_key(k: int, p: int, parts: int, n_kmers: int) -> str:
-    return f"gfx950:k{k}:p{p}:parts{parts}:n{max(0, int(math.log2(max(n_kmers, 1))))}"
+    return f"gfx950.2:k{k}:p{p}:parts{parts}:n{max(0, int(math.log2(max(n_kmers, 1))))}"
 
 
 def load(path: str = CACHE) -> dict:
@@ -97,8 +96,8 @@ def tune(counter: native.Counter, k: int, p: int, parts: int, n_kmers: int, cmin
             best_p1, choice["p1_lists"] = ms, lists
     counter.set_p1_lists(0 if choice["p1_lists"] else 0xFFFFFFFF)
     counter.superkmers(k, p, parts)
-    # count stage: sweep size, then workgroups per CU
-    caps = (5504, 7168, 8192, 9472, 11008) if k <= 32 else (1600, 2048, 2304, 2688)
+    # count stage: sweep size
+    caps = (9216, 11264, 13312, 16384, 18432, 20480) if k <= 32 else (2304, 3072, 3840, 4224, 4608, 4992)
     best = None
     for cap in caps:
         counter.set_tuning(cap)
@@ -107,13 +106,6 @@ def tune(counter: native.Counter, k: int, p: int, parts: int, n_kmers: int, cmin
         if best is None or ms < best:
             best, choice["inst_cap"] = ms, cap
     counter.set_tuning(choice["inst_cap"])
-    best = None
-    for wg in (1, 2):
-        counter.set_count_workgroups(wg)
-        ms = _count_ms(counter, cmin, cmax, reps)
-        times[f"count_wg_per_cu={wg}"] = ms
-        if best is None or ms < best:
-            best, choice["count_wg_per_cu"] = ms, wg
     apply(counter, choice)
     if log:
         log(f"[autotune] {shape_key(k, p, parts, n_kmers)}: {choice} ({', '.join(f'{a} {b:.2f}' for a, b in times.items())})")

@@ -1,14 +1,14 @@
 // Count stage, second half, on gfx950: exact (k-mer, count) tables from the units that k_group.hip
 // laid out.
 //
-//  1. k_count_items<RECORDS>, persistent: a workgroup takes units b, b + G, b + 2G, ... and counts each in
+//  1. k_count_units, persistent: a workgroup takes units b, b + G, b + 2G, ... and counts each in
 //     one or more sweeps over its records: chunks of records have their 2-bit words copied into LDS, the
 //     k-mers are taken from there four at a time and counted in an open-addressing LDS table. A unit with
 //     more distinct keys than the table holds is counted in hash slices, one sweep each, that read the
 //     records again; their number follows the ratio of distinct keys to instances seen so far, and a sweep
 //     that overflows all the same is cut further.
 //  2. A unit of more than kDirectSlices sweeps would be read too often: k_expand extracts its k-mers once
-//     and scatters their canonical keys to one region per hash slice, and k_count_items<KEYS> counts a
+//     and scatters their canonical keys to one region per hash slice, and k_count_keys counts a
 //     slice from its region. A slice that received more keys than its margin (a very frequent k-mer) gets
 //     an exact region in a second key area, filled by a second pass (k_ovf_sizes, k_expand<OVF>).
 //  3. A sweep's distinct keys with min <= count <= max (utilities.hpp:190) are appended to the partition's
@@ -25,22 +25,23 @@
 namespace rgkc {
 namespace {
 
-constexpr int kItemThreads = 512;  // count workgroup size (two per CU)
+constexpr int kItemThreads = 1024; // count workgroup size (one per CU)
 constexpr int kStack = 128;        // pending sweeps of one unit
 constexpr uint32_t kMaxCut = 8;    // slices an overflowing sweep is cut into, at most
 constexpr uint32_t kMaxSlices = 1u << 20;
 constexpr int kProbes = 64;        // table probes a key may take
 constexpr uint32_t kPiece = 4;     // consecutive k-mers of a record that one thread takes
 constexpr int kBatch = 2;          // of them inserted together
-constexpr uint32_t kStageW = 2560; // 2-bit words of a chunk
-constexpr uint32_t kPieces = 2048; // pieces of a chunk
-constexpr uint32_t kSame = 1024;   // slots of the chunk's record set
-constexpr uint32_t kLongPieces = 128;  // a record of more pieces is not cut into the chunk's piece map
-static_assert(kStageW <= 4096 && kItemThreads <= 512 && kLongPieces <= 128, "packed record and piece fields");
+constexpr uint32_t kStageW = 4096; // 2-bit words of a chunk
+constexpr uint32_t kPieces = 4096; // pieces of a chunk
+constexpr uint32_t kSame = 2048;   // slots of the chunk's record set
+constexpr uint32_t kLongPieces = 64;  // a record of more pieces is not cut into the chunk's piece map
+static_assert(kStageW <= 4096 && kItemThreads <= 1024 && kLongPieces <= 64, "packed record and piece fields");
 static_assert(kStageW % kItemThreads == 0, "whole words per thread");
 
-// LDS table: 5120 x (8 + 4) or 3072 x (16 + 4) bytes, 60 KiB either way: with the staging areas two
-// workgroups share a CU's 160 KiB.
+// LDS table: 10240 x (8 + 4) or 6144 x (16 + 4) bytes, 120 KiB either way: with the staging areas one
+// workgroup of 16 waves takes a CU. (Two workgroups of 8 waves with half the table each were 4% slower on 1.2 G
+// k-mers: twice the sweeps, more units in several slices, fewer equal records found.)
 //
 // Hash: a 32-bit multiply per key word, its high half rotated down before the next word joins, and the
 // high half folded into the low one at the end (two multiplies for 64-bit keys; a 64-bit multiply takes
@@ -58,14 +59,14 @@ __device__ __forceinline__ uint32_t place(uint32_t h, uint32_t n) { return __umu
 
 template <typename K> struct KT;
 template <> struct KT<uint64_t> {
-    static constexpr uint32_t H = 5120;
+    static constexpr uint32_t H = 10240;
     static __device__ __forceinline__ uint64_t empty() { return ~0ull; }
     static __device__ __forceinline__ uint32_t hash(uint64_t x) {
         return mix((mix_in((uint32_t)x) ^ (uint32_t)(x >> 32)));
     }
 };
 template <> struct KT<u128> {
-    static constexpr uint32_t H = 3072;
+    static constexpr uint32_t H = 6144;
     static __device__ __forceinline__ u128 empty() { return ~(u128)0; }
     static __device__ __forceinline__ uint32_t hash(u128 v) {
         const uint64_t lo = (uint64_t)v, hi = (uint64_t)(v >> 64);
@@ -156,83 +157,92 @@ template <typename K> __device__ __forceinline__ K key_mask(int k) {
 // a slot holding a key keeps it for the whole sweep; a key that finds neither itself nor an empty slot
 // among kProbes flags the sweep (*ovf = 1).
 //
-// 64-bit keys: groups of four slots (32 bytes, two 16-byte reads); the groups of all N keys are read, then
-// the claims of all N keys made, so their latencies overlap. A key is claimed with a CAS at its group's
-// first empty slot, so a group's keys are always a prefix of it; the CAS's old value decides, and every
-// lane inserting a key tries the same slots in the same order: a key is never held twice. (One CAS per
-// slot in turn executed some lane's CAS for all four slots of every wave.)
+// 64-bit keys: groups of four slots (32 bytes, two 16-byte reads). A key is claimed with a CAS at its
+// group's first empty slot, so a group's keys are always a prefix of it; the CAS's old value decides, and
+// every lane inserting a key tries the same slots in the same order: a key is never held twice. (One CAS
+// per slot in turn executed some lane's CAS for all four slots of every wave.)
+constexpr uint32_t kGroupsOf4 = KT<uint64_t>::H / 4u;
+// the slot of a group that holds the key, else 4; its first empty slot (4: none). Compares and selects
+// that do not wait for one another.
+__device__ __forceinline__ uint32_t find(ulonglong2 x, ulonglong2 y, uint64_t k, uint32_t& empty) {
+    const uint32_t e0 = x.x == ~0ull ? 0u : 4u, e1 = x.y == ~0ull ? 1u : 4u, e2 = y.x == ~0ull ? 2u : 4u,
+                   e3 = y.y == ~0ull ? 3u : 4u;
+    const uint32_t i0 = x.x == k ? 0u : 4u, i1 = x.y == k ? 1u : 4u, i2 = y.x == k ? 2u : 4u, i3 = y.y == k ? 3u : 4u;
+    empty = min(min(e0, e1), min(e2, e3));
+    return min(min(i0, i1), min(i2, i3));
+}
+// One try for each of N keys; returns the keys that lost a claim to another key, or whose group is full.
 template <int N>
-__device__ __forceinline__ void insert(uint64_t* tk, uint32_t* tc, const uint64_t* key, const uint32_t* h, uint32_t valid,
-                                       uint32_t w, uint32_t* ovf) {
-    constexpr uint32_t NG = KT<uint64_t>::H / 4u;
-    uint32_t g[N];
+__device__ __forceinline__ uint32_t insert_first(uint64_t* tk, uint32_t* tc, const uint64_t* key, const uint32_t* h,
+                                                 uint32_t valid, uint32_t w) {
+    uint32_t g[N], pend = 0;
     ulonglong2 q0[N], q1[N];
 #pragma unroll
     for (int u = 0; u < N; u++) {
-        g[u] = place(h[u], NG);
+        g[u] = place(h[u], kGroupsOf4);
         const ulonglong2* const gs = (const ulonglong2*)&tk[4u * g[u]];
         q0[u] = gs[0];
         q1[u] = gs[1];
     }
-    // the slot that holds the key, else 4; the first empty slot (4: none)
-    auto find = [](ulonglong2 x, ulonglong2 y, uint64_t k, uint32_t& empty) -> uint32_t {
-        uint32_t i = 4u;
-        i = y.y == k ? 3u : i;
-        i = y.x == k ? 2u : i;
-        i = x.y == k ? 1u : i;
-        i = x.x == k ? 0u : i;
-        empty = (x.x != ~0ull) + (x.y != ~0ull) + (y.x != ~0ull) + (y.y != ~0ull);
-        return i;
-    };
-    uint32_t pend = 0;  // keys that lost a claim to another key, or whose group is full
 #pragma unroll
     for (int u = 0; u < N; u++) {
+        const uint32_t v = (valid >> u) & 1u;
         uint32_t e;
         uint32_t i = find(q0[u], q1[u], key[u], e);
-        if (i == 4u && e < 4u && ((valid >> u) & 1u)) {
+        if (((i >> 2) & v) && e < 4u) {
             const unsigned long long o = atomicCAS((unsigned long long*)&tk[4u * g[u] + e], ~0ull, (unsigned long long)key[u]);
-            if (o == ~0ull || o == key[u]) i = e;
+            i = (o == ~0ull) | (o == key[u]) ? e : 4u;
         }
-        if ((valid >> u) & 1u) {
-            if (i < 4u) atomicAdd(&tc[4u * g[u] + i], w);
-            else pend |= 1u << u;
-        }
+        pend |= ((i >> 2) & v) << u;
+        if (v & ~(i >> 2)) atomicAdd(&tc[4u * g[u] + i], w);
     }
-    // they go on in one loop for all N keys (a lane's next key as soon as one has its slot): nearly every
-    // wave has some, few lanes more than one
-    if (pend) {
-        uint64_t kk = 0;
-        uint32_t gg = 0;
-        auto take = [&]() {
-            const uint32_t u = (uint32_t)__builtin_ctz(pend);
+    return pend;
+}
+// The keys `pend` of N, on from their groups, in one loop (a lane's next key as soon as one has its slot):
+// nearly every wave has some, few lanes more than one.
+template <int N>
+__device__ __forceinline__ void insert_rest(uint64_t* tk, uint32_t* tc, const uint64_t* key, const uint32_t* h, uint32_t pend,
+                                            uint32_t w, uint32_t* ovf) {
+    if (!pend) return;
+    uint64_t kk = 0;
+    uint32_t gg = 0;
+    auto take = [&]() {
+        const uint32_t u = (uint32_t)__builtin_ctz(pend);
+        uint32_t hh = 0;
 #pragma unroll
-            for (int j = 0; j < N; j++)
-                if (u == (uint32_t)j) { kk = key[j]; gg = g[j]; }
-        };
-        take();
-        for (int tries = 0;;) {
-            const ulonglong2* const gs = (const ulonglong2*)&tk[4u * gg];
-            uint32_t e;
-            uint32_t i = find(gs[0], gs[1], kk, e);
-            if (i == 4u && e < 4u) {
-                const unsigned long long o = atomicCAS((unsigned long long*)&tk[4u * gg + e], ~0ull, (unsigned long long)kk);
-                if (o == ~0ull || o == kk) i = e;
-            }
-            if (i < 4u) {
-                atomicAdd(&tc[4u * gg + i], w);
-                pend &= pend - 1u;
-                if (!pend) break;
-                take();
-                tries = 0;
-            } else {
-                if (e == 4u) gg = gg + 1u == NG ? 0u : gg + 1u;
-                if (++tries == kProbes) {
-                    *ovf = 1u;
-                    break;
-                }
+        for (int j = 0; j < N; j++)
+            if (u == (uint32_t)j) { kk = key[j]; hh = h[j]; }
+        gg = place(hh, kGroupsOf4);
+    };
+    take();
+#pragma unroll 1
+    for (int tries = 0;;) {
+        const ulonglong2* const gs = (const ulonglong2*)&tk[4u * gg];
+        uint32_t e;
+        uint32_t i = find(gs[0], gs[1], kk, e);
+        if ((i >> 2) && e < 4u) {
+            const unsigned long long o = atomicCAS((unsigned long long*)&tk[4u * gg + e], ~0ull, (unsigned long long)kk);
+            i = (o == ~0ull) | (o == kk) ? e : 4u;
+        }
+        if (i < 4u) {
+            atomicAdd(&tc[4u * gg + i], w);
+            pend &= pend - 1u;
+            if (!pend) break;
+            take();
+            tries = 0;
+        } else {
+            if (e == 4u) gg = gg + 1u == kGroupsOf4 ? 0u : gg + 1u;
+            if (++tries == kProbes) {
+                *ovf = 1u;
+                break;
             }
         }
     }
+}
+template <int N>
+__device__ __forceinline__ void insert(uint64_t* tk, uint32_t* tc, const uint64_t* key, const uint32_t* h, uint32_t valid,
+                                       uint32_t w, uint32_t* ovf) {
+    insert_rest<N>(tk, tc, key, h, insert_first<N>(tk, tc, key, h, valid, w), w, ovf);
 }
 // 128-bit keys: slot = {lo, hi}; hi == ~0 empty, ~0-1 busy (being published); keys have hi < 2^62.
 // The winner of the claim publishes in straight-line code before anyone waits, and a full fence keeps
@@ -454,335 +464,443 @@ __global__ void k_key_desc(CountArgs a) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// 1. / 3. Persistent count kernel. RECORDS: workgroup b takes units b, b + G, ... (G = grid size) and
-//     reads their records; else it takes expanded slices and reads their keys. A unit's sweeps are its
-//     initial hash slices in order, each followed by the slices it was cut into if it overflowed.
-//     Bound by VALU issue in the insert (about 120 instructions a wave of keys) and by LDS (random
-//     32-byte reads, CAS and count atomics). For 1.2 G k-mers at 30x (360 M distinct): 9.4 ms with the
-//     0.9 ms expansion of the largest units, where expanding every k-mer took 6.5 and counting the keys
-//     6.0; 187 M k-mers with k=25 1.4 + 0.35 ms, before 1.2 + 0.9; 392 M 128-bit keys 7.9 + 0.6 ms, before 5.3 + 7.0.
+// 1. / 3. The two persistent count kernels: workgroup b takes units (or expanded slices) b, b + G, ...
+//     (G = grid size), each in one or more sweeps.
 struct Cut {
     uint32_t slice, n;
 };
-template <typename K, bool RECORDS>
-__global__ __launch_bounds__(kItemThreads, 4) void k_count_items(CountArgs a) {
-    constexpr int TC = kItemThreads, NW = TC / 64;
-    constexpr uint32_t H = KT<K>::H;
-    constexpr int SPT = (int)H / TC;  // table slots per thread
-    static_assert(H % TC == 0, "whole slots per thread");
-    __shared__ __align__(16) K tkeys[H];
-    __shared__ uint32_t tcnt[H];
-    __shared__ uint32_t stw[RECORDS ? kStageW + 8 : 1];
+
+// A sweep's end: every thread takes its table slots into registers and clears them. `occ` and `keep` are
+// the wave's occupied slots and those that pass [cmin, cmax].
+template <typename K> struct Slots {
+    static constexpr int SPT = (int)KT<K>::H / kItemThreads;
+    static_assert(KT<K>::H % kItemThreads == 0, "whole slots per thread");
+    K key[SPT];
+    uint32_t cnt[SPT];
+    __device__ __forceinline__ bool kept(const CountArgs& a, int j) const {
+        return key[j] != KT<K>::empty() && cnt[j] >= a.cmin && cnt[j] <= a.cmax;
+    }
+    __device__ __forceinline__ void take(const CountArgs& a, K* tkeys, uint32_t* tcnt, uint32_t& occ, uint32_t& keep) {
+        occ = keep = 0;
+#pragma unroll
+        for (int j = 0; j < SPT; j++) {
+            const uint32_t s = threadIdx.x + (uint32_t)j * kItemThreads;
+            key[j] = tkeys[s];
+            cnt[j] = tcnt[s];
+            tkeys[s] = KT<K>::empty();
+            tcnt[s] = 0;
+        }
+#pragma unroll
+        for (int j = 0; j < SPT; j++) {
+            occ += (uint32_t)__popcll(__ballot(key[j] != KT<K>::empty()));
+            keep += (uint32_t)__popcll(__ballot(kept(a, j)));
+        }
+    }
+    // The wave's kept rows from row `row` on, straight from registers: the kept ones of 64 slots go to
+    // consecutive rows, so they leave in nearly whole lines.
+    __device__ __forceinline__ void store(const CountArgs& a, uint64_t row) const {
+#pragma unroll
+        for (int j = 0; j < SPT; j++) {
+            const bool keeps = kept(a, j);
+            const uint64_t kb = __ballot(keeps);
+            if (keeps) {
+                const uint64_t r = row + __builtin_amdgcn_mbcnt_hi((uint32_t)(kb >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)kb, 0u));
+                if constexpr (sizeof(K) == 8) ((uint64_t*)a.out_keys)[r] = (uint64_t)key[j];
+                else ((ulonglong2*)a.out_keys)[r] = make_ulonglong2((uint64_t)key[j], (uint64_t)((u128)key[j] >> 64));
+                a.out_counts[r] = cnt[j];
+            }
+            row += (uint32_t)__popcll(kb);
+        }
+    }
+};
+// the workgroup's totals and the kept rows of the waves before this one, from each wave's in wtot
+__device__ __forceinline__ void slot_totals(const uint32_t* wtot, uint32_t wave, uint32_t& nd, uint32_t& kept, uint32_t& before) {
+    nd = kept = before = 0;
+#pragma unroll
+    for (int w = 0; w < kItemThreads / 64; w++) {
+        const uint32_t t = wtot[w];
+        nd += t & 0xFFFFu;
+        if ((uint32_t)w < wave) before += t >> 16;
+        kept += t >> 16;
+    }
+}
+// Cuts an overflowing sweep: f slices of it onto the stack, from the distinct keys held when it stopped and
+// the share of its records or keys read until then. False (and an error) if it cannot be cut.
+__device__ __forceinline__ bool cut_sweep(const CountArgs& a, uint32_t ovf, Cut c, uint32_t nd, float frac, float fill, Cut* stack,
+                                          uint32_t& n_stack) {
+    uint32_t f = (uint32_t)ceilf(1.2f * (float)nd / (fminf(frac, 1.0f) * fill));
+    f = max(2u, min(f, kMaxCut));
+    if (ovf >= 2u || (uint64_t)c.n * f > kMaxSlices || n_stack + f > (uint32_t)kStack) {
+        raise_err(a.err, RGKC_ERR_COUNT_FAIL);
+        return false;
+    }
+    for (uint32_t j = 0; j < f; j++) stack[n_stack++] = Cut{c.slice * f + j, c.n * f};
+    return true;
+}
+// Row reservation of a sweep (thread 0): the rows its partition had before, and its first row from them
+// (apart, so that the atomic's latency can pass in between).
+__device__ __forceinline__ uint64_t reserve_rows(const CountArgs& a, uint32_t part, uint32_t kept, uint32_t nd) {
+    uint64_t rows = 0;
+    if (kept) rows = atomicAdd(&a.row_cursor[part], (unsigned long long)kept);
+    if (nd) atomicAdd(&a.part_distinct[part], (unsigned long long)nd);
+    return rows;
+}
+__device__ __forceinline__ uint64_t first_row(const CountArgs& a, uint32_t part, uint64_t rows, uint32_t kept) {
+    const uint64_t row = a.row_base[part] + rows;
+    if (row + kept > a.row_end[part]) raise_err(a.err, RGKC_ERR_ROW_OVERFLOW);
+    return row;
+}
+
+// Units, from their records: chunk after chunk of up to kItemThreads records. A chunk is staged (record
+// sizes scanned, words and record info to LDS) from registers whose loads were issued while the chunk
+// before it was counted, across the ends of sweeps and units as well; a sweep's rows leave only after the
+// next chunk is staged, so the row reservation's latency passes under the staging and the stores' under
+// the next chunk's counting. (With the loads of a sweep's first chunk and its row stores in line, staging
+// and row output took a third of the kernel.)
+// Bound by LDS in the insert (random 32-byte reads, CAS and count atomics: a third of the time at three
+// quarters of its rate) and by VALU issue around it. 1.2 G k-mers at 30x (360 M distinct): 9.1 ms, where
+// expanding every k-mer took 6.5 and counting the keys 6.0; 188 M (k=25) 1.35 ms, before 1.2 + 0.85; 392 M
+// 128-bit keys 7.5 ms, before 5.3 + 7.0.
+template <typename K>
+__global__ __launch_bounds__(kItemThreads, 4) void k_count_units(CountArgs a) {
+    constexpr int TC = kItemThreads, NW = TC / 64, WPT = (int)kStageW / TC;
+    __shared__ __align__(16) K tkeys[KT<K>::H];
+    __shared__ uint32_t tcnt[KT<K>::H];
+    __shared__ uint32_t stw[kStageW + 8];
     // a chunk's records: first word | k-mers << 12, how many equal ones; the hash set of the records, then
-    // the pieces (record | piece of it << 9)
-    __shared__ uint32_t rinfo[RECORDS ? TC : 1], rmul[RECORDS ? TC : 1];
-    __shared__ union { uint32_t same[RECORDS ? kSame : 1]; uint16_t pmap[RECORDS ? kPieces : 1]; } mp;
-    uint32_t* const same = mp.same;
-    uint16_t* const pmap = mp.pmap;
+    // the pieces (record | piece of it << 10)
+    __shared__ uint32_t rinfo[TC], rmul[TC];
+    __shared__ union { uint32_t same[kSame]; uint16_t pmap[kPieces]; } mp;
     __shared__ Cut stack[kStack];
     __shared__ uint32_t tmp2[2 * NW], wtot[NW];
     __shared__ unsigned long long sh_in;  // chunk: records << 20 | words
-    __shared__ uint32_t sh_np, sh_long;
     __shared__ uint64_t sh_row_base;
-    __shared__ uint32_t sh_ovf, sh_nstack, sh_first, sh_q0;
+    __shared__ uint32_t sh_ovf, sh_np, sh_long, sh_nstack, sh_first, sh_q0, sh_next;
     __shared__ Cut cur;
+    uint32_t* const same = mp.same;
+    uint16_t* const pmap = mp.pmap;
 
     const int k = a.k;
     const K m = key_mask<K>(k);
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    const uint64_t G = gridDim.x, it_end = RECORDS ? a.plan_n[kPlanItems] : a.n_key_items;
+    const uint64_t G = gridDim.x, it_end = a.plan_n[kPlanItems];
+    uint64_t it = blockIdx.x;
+    if (it >= it_end) return;
     // the workgroup's sweep, retry and distinct totals, added to the global counters once at the end;
     // instances and distinct keys of its sweeps are added to the shared totals every few sweeps
     unsigned long long n_sweeps = 0, n_retries = 0, n_distinct = 0, seen_i = 0, seen_d = 0;
-    for (uint32_t i = threadIdx.x; i < H; i += TC) { tkeys[i] = KT<K>::empty(); tcnt[i] = 0; }
-    unsigned long long est_i = 0, est_d = 0;  // read one unit ahead, by thread 0
+    unsigned long long est_i = 0, est_d = 0;  // the shared totals, read one unit ahead by thread 0
+    for (uint32_t i = threadIdx.x; i < KT<K>::H; i += TC) { tkeys[i] = KT<K>::empty(); tcnt[i] = 0; }
+
     // descriptors: lane i of every wave loads word i one unit ahead, and the fields are wave-uniform
-    constexpr uint32_t DW = (RECORDS ? sizeof(UnitDesc) : sizeof(KeyItem)) / 4;
+    constexpr uint32_t DW = sizeof(UnitDesc) / 4;
     static_assert(DW <= 64, "a lane per word");
-    const uint32_t* const items = RECORDS ? (const uint32_t*)a.unit_items : (const uint32_t*)a.key_desc;
-    uint32_t ahead = (blockIdx.x < it_end && lane < DW) ? items[blockIdx.x * (uint64_t)DW + lane] : 0u;
-    for (uint64_t it = blockIdx.x; it < it_end; it += G) {
-        auto word = [&](int i) { return (uint32_t)__builtin_amdgcn_readlane((int)ahead, i); };
-        auto word2 = [&](int i) { return (uint64_t)word(i) | ((uint64_t)word(i + 1) << 32); };
-        UnitDesc ud{};
-        KeyItem kd{};
-        if (RECORDS) {
-            ud.part = word(0); ud.inst = word(1); ud.n_rec = word(2); ud.n_word = word(3);
-            ud.desc = word2(4); ud.word = word2(6);
-        } else {
-            kd.part = word(0); kd.n = word(1); kd.slice = word(2); kd.q = word(3);
-            kd.keys = word2(4);
+    const uint32_t* const items = (const uint32_t*)a.unit_items;
+    auto fetch = [&](uint64_t i) { return (i < it_end && lane < DW) ? items[i * DW + lane] : 0u; };
+    auto unit = [&](uint32_t v) {
+        auto word = [&](int i) { return (uint32_t)__builtin_amdgcn_readlane((int)v, i); };
+        UnitDesc d;
+        d.part = word(0); d.inst = word(1); d.n_rec = word(2); d.n_word = word(3);
+        d.desc = (uint64_t)word(4) | ((uint64_t)word(5) << 32);
+        d.word = (uint64_t)word(6) | ((uint64_t)word(7) << 32);
+        d.q = d.pad = 0;
+        return d;
+    };
+    UnitDesc ud = unit(fetch(it));
+    uint32_t ahead = fetch(it + G);
+    // initial hash slices of a unit (thread 0): what its distinct keys should take by the ratio seen so far
+    auto slices = [&](uint32_t inst) {
+        const float ratio = est_i > 4ull * a.unit_cap ? (float)est_d / (float)est_i : kFill<K> / (float)a.unit_cap;
+        uint32_t q = (uint32_t)ceilf(1.1f * (float)inst * fminf(ratio, 1.0f) / kFill<K>);
+        q = max(1u, min(q, kMaxSlices));
+        if ((float)inst <= kFill<K>) q = 1u;
+        est_i = __hip_atomic_load(&a.plan_n[kPlanSeenInst], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        est_d = __hip_atomic_load(&a.plan_n[kPlanSeenDistinct], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return q;
+    };
+    if (threadIdx.x == 0) {
+        sh_nstack = 0;
+        sh_q0 = slices(ud.inst);
+        sh_first = 1;
+        cur = Cut{0, sh_q0};
+        sh_ovf = 0;
+    }
+
+    uint32_t dn, wn[WPT];  // the next chunk's descriptor and words of this thread
+    auto load = [&](const UnitDesc& d, uint32_t c, uint32_t w) {
+        dn = c + threadIdx.x < d.n_rec ? a.desc[d.desc + c + threadIdx.x] : 0u;
+#pragma unroll
+        for (int u = 0; u < WPT; u++) {
+            const uint32_t i = w + threadIdx.x + (uint32_t)u * TC;
+            wn[u] = i < d.n_word ? a.words[d.word + i] : 0u;
         }
-        if (it + G < it_end && lane < DW) ahead = items[(it + G) * DW + lane];
-        const uint32_t part = RECORDS ? ud.part : kd.part;
-        const uint32_t inst = RECORDS ? ud.inst : kd.n;
+    };
+    uint32_t km, nw, np, exW;
+    bool in;
+    // stages the loaded chunk (records c ... of the unit); `publish` runs in thread 0 before its last barrier
+    auto stage = [&](uint32_t c, auto&& publish) {
+        const bool has = c + threadIdx.x < ud.n_rec;
+        km = dn;
+        nw = has ? rec_words(km, k) : 0u;
+        np = (km + kPiece - 1u) / kPiece;
+        if (threadIdx.x == 0) { sh_in = 0; sh_np = 0; sh_long = 0; }
+        uint32_t exP, totW, totP;
+        wg_exscan2_u32(nw, np, tmp2, exW, exP, totW, totP);
+        in = has && (exW + nw <= kStageW) && (exP + np <= kPieces);
+        const uint64_t bal = __ballot(in);
+        if (in && (bal >> lane) == 1ull)
+            atomicMax(&sh_in, ((unsigned long long)(threadIdx.x + 1u) << 20) | (exW + nw));
+        rinfo[threadIdx.x] = exW | (km << 12);
+        rmul[threadIdx.x] = 1u;
+#pragma unroll
+        for (int u = 0; u < WPT; u++) stw[threadIdx.x + (uint32_t)u * TC] = wn[u];
+        for (uint32_t i = threadIdx.x; i < kSame; i += TC) same[i] = 0;
+        if (threadIdx.x == 0) publish();
+        __syncthreads();
+    };
+    load(ud, 0, 0);
+    stage(0, [] {});
+    uint32_t c0 = 0, w0 = 0;  // the staged chunk's first record and word in its unit
+    for (;;) {
+        const uint32_t n = (uint32_t)(sh_in >> 20), slice = cur.slice, ns = cur.n;
+        const bool filt = ns > 1;
+        // n == 0: the first record alone exceeds the staging area
+        const uint32_t c1 = c0 + max(n, 1u), w1 = w0 + (n ? (uint32_t)sh_in & 0xFFFFFu : rec_words(rinfo[0] >> 12, k));
+        const bool last = c1 >= ud.n_rec;
+        // the next chunk's loads: this sweep's, the unit's next sweep's, or the next unit's
+        const bool again = sh_nstack > 0 || sh_first < sh_q0;
+        if (!last) load(ud, c1, w1);
+        else if (again) load(ud, 0, 0);
+        else load(unit(ahead), 0, 0);
+        auto single = [&](const uint32_t* bw, uint32_t g) {
+            Window<K> w;
+            w.load(bw, g);
+            const K key = w.key(0, k, m);
+            const uint32_t h = KT<K>::hash(key);
+            insert<1>(tkeys, tcnt, &key, &h, !filt || slice_of(h, ns) == slice ? 1u : 0u, 1u, &sh_ovf);
+        };
+        if (n == 0) {
+            const uint32_t km1 = rinfo[0] >> 12;  // its k-mers straight from HBM
+            for (uint32_t x = threadIdx.x; x < km1 && !sh_ovf; x += TC) single(a.words + ud.word + w0, x);
+        } else {
+            // Equal records (reads of one place without errors give equal records but for their ends: two in
+            // five at 30x and 1% errors) are counted once, with their number: a hash set of the chunk's
+            // records, compared word by word.
+            bool uniq = in;
+            if (in && nw <= 16u) {
+                uint32_t h = km;
+                for (uint32_t i = 0; i < nw; i++) h = mix_in(h) ^ stw[exW + i];
+                h = mix(h);
+                const uint32_t entry = (threadIdx.x + 1u) | (h << 16);
+                for (uint32_t s = h >> 16, tries = 0; tries < 8u; s++, tries++) {
+                    const uint32_t o = atomicCAS(&same[s % kSame], 0u, entry);
+                    if (o == 0) break;
+                    if ((o ^ entry) >> 16) continue;
+                    const uint32_t other = (o & 0xFFFFu) - 1u, oi = rinfo[other];
+                    if (oi >> 12 != km) continue;
+                    uint32_t diff = 0;
+                    for (uint32_t i = 0; i < nw; i++) diff |= stw[(oi & 0xFFFu) + i] ^ stw[exW + i];
+                    if (diff) continue;
+                    atomicAdd(&rmul[other], 1u);
+                    uniq = false;
+                    break;
+                }
+            }
+            __syncthreads();
+            // pieces of the records that remain; a record of more than kLongPieces apart
+            {
+                const bool big = np > kLongPieces;
+                const uint32_t mine = uniq && !big ? np : 0u;
+                const uint32_t incl = wave_incl_scan_u32(mine);
+                uint32_t wb = 0;
+                if (lane == 63u) wb = atomicAdd(&sh_np, incl);
+                uint32_t e = (uint32_t)__builtin_amdgcn_readlane((int)wb, 63) + incl - mine;
+                for (uint32_t i = 0; i < mine; i++) pmap[e++] = (uint16_t)(threadIdx.x | (i << 10));
+                if (uniq && big) sh_long = 1;
+            }
+            __syncthreads();
+            const uint32_t npc = sh_np;
+            for (uint32_t x = threadIdx.x; x < npc; x += TC) {
+                const uint32_t e = pmap[x], rec = e & 1023u, j = e >> 10, info = rinfo[rec], mul = rmul[rec];
+                const uint32_t c = min(kPiece, (info >> 12) - kPiece * j);
+                Window<K> w;
+                w.load(stw, (info & 0xFFFu) * 16u + kPiece * j);
+                K key[kPiece];
+                uint32_t h[kPiece], valid = (1u << c) - 1u, pend = 0;
+#pragma unroll
+                for (int t0 = 0; t0 < (int)kPiece; t0 += kBatch) {
+#pragma unroll
+                    for (int t = t0; t < t0 + kBatch; t++) {
+                        key[t] = w.key(t, k, m);
+                        h[t] = KT<K>::hash(key[t]);
+                        if (filt) valid &= ~((uint32_t)(slice_of(h[t], ns) != slice) << t);
+                    }
+                    if constexpr (sizeof(K) == 8)
+                        pend |= insert_first<kBatch>(tkeys, tcnt, key + t0, h + t0, valid >> t0, mul) << t0;
+                    else
+                        insert<kBatch>(tkeys, tcnt, key + t0, h + t0, valid >> t0, mul, &sh_ovf);
+                }
+                if constexpr (sizeof(K) == 8) insert_rest<(int)kPiece>(tkeys, tcnt, key, h, pend, mul, &sh_ovf);
+            }
+            if (sh_long)
+                for (uint32_t q = 0; q < n; q++) {
+                    const uint32_t info = rinfo[q], kq = info >> 12;
+                    if ((kq + kPiece - 1u) / kPiece > kLongPieces)
+                        for (uint32_t x = threadIdx.x; x < kq; x += TC) single(stw, (info & 0xFFFu) * 16u + x);
+                }
+        }
+        __syncthreads();
+        const uint32_t ovf = sh_ovf;
+        if (!last && !ovf) {
+            c0 = c1;
+            w0 = w1;
+            stage(c0, [] {});
+            continue;
+        }
+        // ---- the sweep ends: its slots to registers, its rows reserved, the next sweep chosen and its first
+        // chunk staged, then the rows stored
+        Slots<K> sl;
+        uint32_t occ, keep;
+        sl.take(a, tkeys, tcnt, occ, keep);
+        if (lane == 0) wtot[wave] = occ | (keep << 16);
+        __syncthreads();
+        uint32_t nd, kept, before;
+        slot_totals(wtot, wave, nd, kept, before);
+        const uint32_t part = ud.part;
+        uint64_t row0 = 0;
+        if (threadIdx.x == 0) {
+            if (ovf) {  // cut: the rest of its records is skipped
+                n_retries++;
+                cut_sweep(a, ovf, cur, nd, (float)c1 / (float)ud.n_rec, kFill<K>, stack, sh_nstack);
+            } else {
+                row0 = reserve_rows(a, part, kept, nd);
+                n_sweeps++;
+                n_distinct += nd;
+                seen_i += ud.inst / ns;
+                seen_d += nd;
+                if (n_sweeps <= 2 || (n_sweeps & 7u) == 0) {
+                    atomicAdd(&a.plan_n[kPlanSeenInst], seen_i);
+                    atomicAdd(&a.plan_n[kPlanSeenDistinct], seen_d);
+                    seen_i = seen_d = 0;
+                }
+            }
+            sh_ovf = 0;
+            if (sh_nstack > 0) {
+                cur = stack[--sh_nstack];
+                sh_next = 0;
+            } else if (sh_first < sh_q0) {
+                cur = Cut{sh_first++, sh_q0};
+                sh_next = 0;
+            } else {
+                sh_next = 1;
+                if (it + G < it_end) {
+                    sh_q0 = slices((uint32_t)__builtin_amdgcn_readlane((int)ahead, 1));
+                    sh_first = 1;
+                    cur = Cut{0, sh_q0};
+                }
+            }
+        }
+        __syncthreads();
+        const bool next_unit = sh_next != 0;
+        // what was loaded ahead is the next sweep's, unless this one was cut
+        const bool reload = ovf != 0;
+        if (next_unit) {
+            it += G;
+            if (it >= it_end) {
+                if (threadIdx.x == 0 && !ovf) sh_row_base = first_row(a, part, row0, kept);
+                __syncthreads();
+                if (!ovf && sh_row_base + kept <= a.row_end[part]) sl.store(a, sh_row_base + before);
+                break;
+            }
+            ud = unit(ahead);
+            ahead = fetch(it + G);
+        }
+        if (reload) load(ud, 0, 0);
+        c0 = w0 = 0;
+        stage(0, [&] {
+            if (!ovf) sh_row_base = first_row(a, part, row0, kept);
+        });
+        if (!ovf && sh_row_base + kept <= a.row_end[part]) sl.store(a, sh_row_base + before);
+    }
+    if (threadIdx.x == 0) {
+        if (n_sweeps) atomicAdd(&a.stats[0], n_sweeps);
+        if (n_retries) atomicAdd(&a.stats[1], n_retries);
+        if (n_distinct) atomicAdd(&a.stats[2], n_distinct);
+    }
+}
+
+// Expanded slices, from their keys.
+template <typename K>
+__global__ __launch_bounds__(kItemThreads, 4) void k_count_keys(CountArgs a) {
+    constexpr int TC = kItemThreads, NW = TC / 64, KB = 4;
+    __shared__ __align__(16) K tkeys[KT<K>::H];
+    __shared__ uint32_t tcnt[KT<K>::H];
+    __shared__ Cut stack[kStack];
+    __shared__ uint32_t wtot[NW];
+    __shared__ uint64_t sh_row_base;
+    __shared__ uint32_t sh_ovf, sh_nstack;
+    __shared__ Cut cur;
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    unsigned long long n_sweeps = 0, n_retries = 0, n_distinct = 0;
+    for (uint32_t i = threadIdx.x; i < KT<K>::H; i += TC) { tkeys[i] = KT<K>::empty(); tcnt[i] = 0; }
+    for (uint64_t it = blockIdx.x; it < a.n_key_items; it += gridDim.x) {
+        const KeyItem kd = a.key_desc[it];
+        const K* const kreg = (const K*)kd.keys;
         __syncthreads();
         if (threadIdx.x == 0) {
-            // sweeps that the unit's distinct keys should take, by the ratio seen so far
-            uint32_t q = 1;
-            if (RECORDS) {
-                const float ratio = est_i > 4ull * a.unit_cap ? (float)est_d / (float)est_i : kFill<K> / (float)a.unit_cap;
-                q = (uint32_t)ceilf(1.1f * (float)inst * fminf(ratio, 1.0f) / kFill<K>);
-                q = max(1u, min(q, kMaxSlices));
-                if ((float)inst <= kFill<K>) q = 1u;
-                est_i = __hip_atomic_load(&a.plan_n[kPlanSeenInst], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                est_d = __hip_atomic_load(&a.plan_n[kPlanSeenDistinct], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
-            sh_nstack = 0;
-            sh_first = 0;  // next initial slice
-            sh_q0 = RECORDS ? q : 1u;
+            stack[0] = Cut{kd.slice, kd.q};
+            sh_nstack = 1;
         }
         __syncthreads();
         for (;;) {
             if (threadIdx.x == 0) {
                 cur.n = 0;
                 if (sh_nstack > 0) cur = stack[--sh_nstack];
-                else if (sh_first < sh_q0) {
-                    if (RECORDS) cur = Cut{sh_first, sh_q0};
-                    else cur = Cut{kd.slice, kd.q};
-                    sh_first++;
-                }
                 sh_ovf = 0;
             }
             __syncthreads();
             const uint32_t slice = cur.slice, ns = cur.n;
             if (ns == 0) break;
-            uint32_t scanned = 0;  // records or keys read
-            if constexpr (RECORDS) {
-                const bool filt = ns > 1;
-                const uint32_t* const desc = a.desc + ud.desc;
-                const uint32_t* words = a.words + ud.word;  // the chunk's first word
-                uint32_t words_left = ud.n_word;
-                // a chunk's descriptors and words are loaded while the chunk before it is counted
-                constexpr int WPT = (int)kStageW / TC;
-                uint32_t dn = threadIdx.x < ud.n_rec ? desc[threadIdx.x] : 0u, wn[WPT];
+            const bool filt = ns != kd.q;  // a region holds exactly its slice: only a finer one filters its keys
+            uint32_t scanned = 0;
+            K v[KB];
 #pragma unroll
-                for (int u = 0; u < WPT; u++) {
-                    const uint32_t i = threadIdx.x + (uint32_t)u * TC;
-                    wn[u] = i < words_left ? words[i] : 0u;
+            for (int u = 0; u < KB; u++) v[u] = threadIdx.x + (uint32_t)u * TC < kd.n ? kreg[threadIdx.x + (uint32_t)u * TC] : (K)0;
+            for (uint32_t x0 = 0; x0 < kd.n; x0 += (uint32_t)(KB * TC)) {
+                K key[KB];
+                uint32_t h[KB], valid = 0;
+#pragma unroll
+                for (int u = 0; u < KB; u++) {
+                    const uint32_t x = x0 + threadIdx.x + (uint32_t)u * TC, y = x + (uint32_t)(KB * TC);
+                    key[u] = v[u];
+                    v[u] = y < kd.n ? kreg[y] : (K)0;  // the next batch, in flight while this one is counted
+                    h[u] = KT<K>::hash(key[u]);
+                    if (x < kd.n && (!filt || slice_of(h[u], ns) == slice)) valid |= 1u << u;
                 }
-                auto single = [&](const uint32_t* bw, uint32_t g) {
-                    Window<K> w;
-                    w.load(bw, g);
-                    const K key = w.key(0, k, m);
-                    const uint32_t h = KT<K>::hash(key);
-                    insert<1>(tkeys, tcnt, &key, &h, !filt || slice_of(h, ns) == slice ? 1u : 0u, 1u, &sh_ovf);
-                };
-                for (uint32_t c0 = 0; c0 < ud.n_rec;) {
-                    const uint32_t r = c0 + threadIdx.x;
-                    const uint32_t km = dn;
-                    const uint32_t nw = r < ud.n_rec ? rec_words(km, k) : 0u, np = (km + kPiece - 1u) / kPiece;
-                    if (threadIdx.x == 0) { sh_in = 0; sh_np = 0; sh_long = 0; }
-                    uint32_t exW, exP, totW, totP;
-                    wg_exscan2_u32(nw, np, tmp2, exW, exP, totW, totP);
-                    const bool in = (r < ud.n_rec) && (exW + nw <= kStageW) && (exP + np <= kPieces);
-                    const uint64_t bal = __ballot(in);
-                    if (in && (bal >> lane) == 1ull)
-                        atomicMax(&sh_in, ((unsigned long long)(threadIdx.x + 1u) << 20) | (exW + nw));
-                    rinfo[threadIdx.x] = exW | (km << 12);
-                    rmul[threadIdx.x] = 1u;
-#pragma unroll
-                    for (int u = 0; u < WPT; u++) stw[threadIdx.x + (uint32_t)u * TC] = wn[u];
-                    for (uint32_t i = threadIdx.x; i < kSame; i += TC) same[i] = 0;
-                    __syncthreads();
-                    const uint32_t n = (uint32_t)(sh_in >> 20);
-                    if (n == 0) {
-                        // the first record alone exceeds the staging area: its k-mers straight from HBM
-                        const uint32_t km1 = rinfo[0] >> 12, nw1 = rec_words(km1, k);
-                        for (uint32_t x = threadIdx.x; x < km1 && !sh_ovf; x += TC) single(words, x);
-                        scanned = c0 + 1;
-                        c0 += 1;
-                        words += nw1;
-                        words_left -= nw1;
-                    } else {
-                        const uint32_t nwc = (uint32_t)sh_in & 0xFFFFFu;
-                        c0 += n;
-                        words += nwc;
-                        words_left -= nwc;
-                    }
-                    dn = c0 + threadIdx.x < ud.n_rec ? desc[c0 + threadIdx.x] : 0u;
-#pragma unroll
-                    for (int u = 0; u < WPT; u++) {
-                        const uint32_t i = threadIdx.x + (uint32_t)u * TC;
-                        wn[u] = i < words_left ? words[i] : 0u;
-                    }
-                    if (n > 0) {
-                        // Equal records (reads of one place without errors give equal records but for their
-                        // ends: half of them at 30x and 1% errors) are counted once, with their number: a hash
-                        // set of the chunk's records, compared word by word.
-                        bool uniq = in;
-                        if (in && nw <= 16u) {
-                            uint32_t h = km;
-                            for (uint32_t i = 0; i < nw; i++) h = mix_in(h) ^ stw[exW + i];
-                            h = mix(h);
-                            const uint32_t entry = (threadIdx.x + 1u) | (h << 16);
-                            for (uint32_t s = h >> 16, tries = 0; tries < 8u; s++, tries++) {
-                                const uint32_t o = atomicCAS(&same[s % kSame], 0u, entry);
-                                if (o == 0) break;
-                                if ((o ^ entry) >> 16) continue;
-                                const uint32_t other = (o & 0xFFFFu) - 1u, oi = rinfo[other];
-                                if (oi >> 12 != km) continue;
-                                uint32_t diff = 0;
-                                for (uint32_t i = 0; i < nw; i++) diff |= stw[(oi & 0xFFFu) + i] ^ stw[exW + i];
-                                if (diff) continue;
-                                atomicAdd(&rmul[other], 1u);
-                                uniq = false;
-                                break;
-                            }
-                        }
-                        __syncthreads();
-                        // pieces of the records that remain; a record of more than kLongPieces apart
-                        {
-                            const bool big = np > kLongPieces;
-                            const uint32_t mine = uniq && !big ? np : 0u;
-                            const uint32_t incl = wave_incl_scan_u32(mine);
-                            uint32_t wb = 0;
-                            if (lane == 63u) wb = atomicAdd(&sh_np, incl);
-                            uint32_t e = (uint32_t)__builtin_amdgcn_readlane((int)wb, 63) + incl - mine;
-                            for (uint32_t i = 0; i < mine; i++) pmap[e++] = (uint16_t)(threadIdx.x | (i << 9));
-                            if (uniq && big) sh_long = 1;
-                        }
-                        __syncthreads();
-                        const uint32_t npc = sh_np;
-                        auto piece = [&](uint32_t info, uint32_t mul, uint32_t j) {
-                            const uint32_t c = min(kPiece, (info >> 12) - kPiece * j);
-                            Window<K> w;
-                            w.load(stw, (info & 0xFFFu) * 16u + kPiece * j);
-#pragma unroll
-                            for (int t0 = 0; t0 < (int)kPiece; t0 += kBatch) {
-                                K key[kBatch];
-                                uint32_t h[kBatch], valid = 0;
-#pragma unroll
-                                for (int t = 0; t < kBatch; t++) {
-                                    key[t] = w.key(t0 + t, k, m);
-                                    h[t] = KT<K>::hash(key[t]);
-                                    if ((uint32_t)(t0 + t) < c && (!filt || slice_of(h[t], ns) == slice)) valid |= 1u << t;
-                                }
-                                insert<kBatch>(tkeys, tcnt, key, h, valid, mul, &sh_ovf);
-                            }
-                        };
-                        for (uint32_t x = threadIdx.x; x < npc; x += TC) {
-                            const uint32_t e = pmap[x], rec = e & 511u;
-                            piece(rinfo[rec], rmul[rec], e >> 9);
-                        }
-                        if (sh_long)
-                            for (uint32_t q = 0; q < n; q++) {
-                                const uint32_t info = rinfo[q], kq = info >> 12;
-                                if ((kq + kPiece - 1u) / kPiece > kLongPieces)
-                                    for (uint32_t x = threadIdx.x; x < kq; x += TC) single(stw, (info & 0xFFFu) * 16u + x);
-                            }
-                        scanned = c0;  // records read
-                    }
-                    __syncthreads();
-                    if (sh_ovf) break;  // the sweep will be cut: skip its remaining records
-                }
-            } else {
-                const bool filt = ns != kd.q;
-                const K* const kreg = (const K*)kd.keys;
-                constexpr int KB = 4;
-                K v[KB];
-#pragma unroll
-                for (int u = 0; u < KB; u++) v[u] = threadIdx.x + (uint32_t)u * TC < kd.n ? kreg[threadIdx.x + (uint32_t)u * TC] : (K)0;
-                for (uint32_t x0 = 0; x0 < kd.n; x0 += (uint32_t)(KB * TC)) {
-                    K key[KB];
-                    uint32_t h[KB], valid = 0;
-#pragma unroll
-                    for (int u = 0; u < KB; u++) {
-                        const uint32_t x = x0 + threadIdx.x + (uint32_t)u * TC, y = x + (uint32_t)(KB * TC);
-                        key[u] = v[u];
-                        v[u] = y < kd.n ? kreg[y] : (K)0;  // the next batch, in flight while this one is counted
-                        h[u] = KT<K>::hash(key[u]);
-                        if (x < kd.n && (!filt || slice_of(h[u], ns) == slice)) valid |= 1u << u;
-                    }
-                    insert<KB>(tkeys, tcnt, key, h, valid, 1u, &sh_ovf);
-                    scanned += (uint32_t)(KB * TC);
-                    if (sh_ovf) break;
-                }
+                insert<KB>(tkeys, tcnt, key, h, valid, 1u, &sh_ovf);
+                scanned += (uint32_t)(KB * TC);
+                if (sh_ovf) break;
             }
             __syncthreads();
-            // ---- finalize: every thread takes its slots and clears them; the kept rows of a wave's slots go
-            // to consecutive places, so the rows leave from registers in nearly whole lines
-            K kr[SPT];
-            uint32_t cr[SPT], occ = 0, keep = 0;  // of the wave
-            auto kept_row = [&](int j) { return kr[j] != KT<K>::empty() && cr[j] >= a.cmin && cr[j] <= a.cmax; };
-#pragma unroll
-            for (int j = 0; j < SPT; j++) {
-                const uint32_t s = threadIdx.x + (uint32_t)j * TC;
-                kr[j] = tkeys[s];
-                cr[j] = tcnt[s];
-                tkeys[s] = KT<K>::empty();
-                tcnt[s] = 0;
-            }
-#pragma unroll
-            for (int j = 0; j < SPT; j++) {
-                occ += (uint32_t)__popcll(__ballot(kr[j] != KT<K>::empty()));
-                keep += (uint32_t)__popcll(__ballot(kept_row(j)));
-            }
+            Slots<K> sl;
+            uint32_t occ, keep, nd, kept, before;
+            sl.take(a, tkeys, tcnt, occ, keep);
             if (lane == 0) wtot[wave] = occ | (keep << 16);
             __syncthreads();
-            uint32_t nd = 0, kept = 0, before = 0;
-#pragma unroll
-            for (int w = 0; w < NW; w++) {
-                const uint32_t t = wtot[w];
-                nd += t & 0xFFFFu;
-                if ((uint32_t)w < wave) before += t >> 16;
-                kept += t >> 16;
-            }
+            slot_totals(wtot, wave, nd, kept, before);
             const uint32_t ovf = sh_ovf;
-            if (ovf) {
-                if (threadIdx.x == 0) {
-                    n_retries++;
-                    // distinct keys of this sweep, estimated from the keys held when it stopped and the
-                    // share of the unit read until then
-                    const float frac = fminf((float)max(scanned, 1u) / (float)max(RECORDS ? ud.n_rec : kd.n, 1u), 1.0f);
-                    uint32_t f = (uint32_t)ceilf(1.2f * (float)nd / (frac * kFill<K>));
-                    f = max(2u, min(f, kMaxCut));
-                    if (ovf >= 2u || (uint64_t)ns * f > kMaxSlices || sh_nstack + f > (uint32_t)kStack)
-                        raise_err(a.err, RGKC_ERR_COUNT_FAIL);
-                    else
-                        for (uint32_t j = 0; j < f; j++) stack[sh_nstack++] = Cut{slice * f + j, ns * f};
-                }
-                __syncthreads();
-                continue;
-            }
             if (threadIdx.x == 0) {
-                uint64_t base = 0;
-                if (kept) base = atomicAdd(&a.row_cursor[part], (unsigned long long)kept);
-                sh_row_base = a.row_base[part] + base;
-                if (sh_row_base + kept > a.row_end[part]) raise_err(a.err, RGKC_ERR_ROW_OVERFLOW);
-                n_sweeps++;
-                n_distinct += nd;
-                if (nd) atomicAdd(&a.part_distinct[part], (unsigned long long)nd);
-                if (RECORDS) {
-                    seen_i += inst / ns;
-                    seen_d += nd;
-                    if (n_sweeps <= 2 || (n_sweeps & 7u) == 0) {
-                        atomicAdd(&a.plan_n[kPlanSeenInst], seen_i);
-                        atomicAdd(&a.plan_n[kPlanSeenDistinct], seen_d);
-                        seen_i = seen_d = 0;
-                    }
+                if (ovf) {
+                    n_retries++;
+                    cut_sweep(a, ovf, cur, nd, (float)scanned / (float)kd.n, kFill<K>, stack, sh_nstack);
+                } else {
+                    sh_row_base = first_row(a, kd.part, reserve_rows(a, kd.part, kept, nd), kept);
+                    n_sweeps++;
+                    n_distinct += nd;
                 }
             }
             __syncthreads();
-            const uint64_t rb = sh_row_base;
-            if (rb + kept <= a.row_end[part]) {
-                uint64_t row = rb + before;
-#pragma unroll
-                for (int j = 0; j < SPT; j++) {
-                    const bool keeps = kept_row(j);
-                    const uint64_t kb = __ballot(keeps);
-                    if (keeps) {
-                        const uint64_t r = row + __builtin_amdgcn_mbcnt_hi((uint32_t)(kb >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)kb, 0u));
-                        if constexpr (sizeof(K) == 8) {
-                            ((uint64_t*)a.out_keys)[r] = (uint64_t)kr[j];
-                        } else {
-                            ((ulonglong2*)a.out_keys)[r] = make_ulonglong2((uint64_t)kr[j], (uint64_t)((u128)kr[j] >> 64));
-                        }
-                        a.out_counts[r] = cr[j];
-                    }
-                    row += (uint32_t)__popcll(kb);
-                }
-            }
+            if (!ovf && sh_row_base + kept <= a.row_end[kd.part]) sl.store(a, sh_row_base + before);
         }
     }
     if (threadIdx.x == 0) {
@@ -815,32 +933,32 @@ hipError_t launch_expand_ovf(const CountArgs& a, uint64_t n_units, hipStream_t s
     return hipGetLastError();
 }
 
-// up to two resident workgroups per CU (the LDS table allows two), each looping over units
-static unsigned count_grid(const CountArgs& a) {
+// one resident workgroup per CU (its table and staging areas take the LDS), looping over units
+static unsigned count_grid() {
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
         cus <= 0)
         cus = 256;
-    return (unsigned)cus * (a.count_wg_per_cu ? std::min<uint32_t>(a.count_wg_per_cu, 2u) : 2u);
+    return (unsigned)cus;
 }
 
 hipError_t launch_count_units(const CountArgs& a, hipStream_t s) {
-    const unsigned grid = count_grid(a);
-    if (a.k <= 32) hipLaunchKernelGGL((k_count_items<uint64_t, true>), dim3(grid), dim3(kItemThreads), 0, s, a);
-    else hipLaunchKernelGGL((k_count_items<u128, true>), dim3(grid), dim3(kItemThreads), 0, s, a);
+    const unsigned grid = count_grid();
+    if (a.k <= 32) hipLaunchKernelGGL(k_count_units<uint64_t>, dim3(grid), dim3(kItemThreads), 0, s, a);
+    else hipLaunchKernelGGL(k_count_units<u128>, dim3(grid), dim3(kItemThreads), 0, s, a);
     return hipGetLastError();
 }
 
 hipError_t launch_count_keys(const CountArgs& a, hipStream_t s) {
     if (!a.n_key_items) return hipSuccess;
     const unsigned pb = (unsigned)((a.n_key_items + 255) / 256);
-    const unsigned grid = (unsigned)std::min<uint64_t>(a.n_key_items, count_grid(a));
+    const unsigned grid = (unsigned)std::min<uint64_t>(a.n_key_items, count_grid());
     if (a.k <= 32) {
         hipLaunchKernelGGL(k_key_desc<uint64_t>, dim3(pb), dim3(256), 0, s, a);
-        hipLaunchKernelGGL((k_count_items<uint64_t, false>), dim3(grid), dim3(kItemThreads), 0, s, a);
+        hipLaunchKernelGGL(k_count_keys<uint64_t>, dim3(grid), dim3(kItemThreads), 0, s, a);
     } else {
         hipLaunchKernelGGL(k_key_desc<u128>, dim3(pb), dim3(256), 0, s, a);
-        hipLaunchKernelGGL((k_count_items<u128, false>), dim3(grid), dim3(kItemThreads), 0, s, a);
+        hipLaunchKernelGGL(k_count_keys<u128>, dim3(grid), dim3(kItemThreads), 0, s, a);
     }
     return hipGetLastError();
 }

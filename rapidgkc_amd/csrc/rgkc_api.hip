@@ -131,7 +131,6 @@ struct rgkc_ctx {
     hipEvent_t table_ev[2] = {nullptr, nullptr};
     bool table_ok = false;
     uint32_t inst_cap = 0;
-    uint32_t count_wg_per_cu = 0;  // count kernel: resident workgroups per CU (0: four)
     uint64_t mem_limit = 0;  // count stage: device memory to plan with (0: what is free)
     bool compact_active = false;  // a count in compact mode holds its temporary table in tkeys/tcounts
     bool recount_active = false;  // the predicted path's recount writes keys2/counts2
@@ -386,13 +385,13 @@ int do_phase1(rgkc_ctx* c, int k, int p, int parts, uint32_t* mm_hist = nullptr)
     return 0;
 }
 
-// K-mer instances planned per count sweep: for 64-bit keys what fills the table (4096 of 5120 slots) at
-// one distinct key in two instances, for 128-bit ones (2150 of 3072, tried one by one) nearly all distinct.
+// K-mer instances planned per count sweep: for 64-bit keys what fills the table (8192 of 10240 slots) at
+// one distinct key in two instances, for 128-bit ones (4300 of 6144, tried one by one) nearly all distinct.
 // Read sets are mostly below: their larger units then take fewer sweeps than planned. The count stage over
-// 5500, 7000, 8200, 9472, 11000: 13.3, 12.7, 12.9, 13.0, 13.1 ms (1.2 G k-mers at 30x), 2.40, 2.29, 2.27, 2.32,
-// 2.37 (188 M, k=25); over 1600, 1900, 2200, 2600: 11.1, 10.2, 9.6, 9.9 ms (392 M, k=55 at 10x).
+// 13000, 15000, 16384, 18432: 12.2, 12.0, 12.1, 12.0 ms (1.2 G k-mers at 30x), 2.10, 2.05, 1.96, 2.00 (188 M,
+// k=25); over 3800, 4200, 4608, 5000: 9.4, 9.2, 9.1, 9.2 ms (392 M, k=55 at 10x).
 uint32_t unit_cap(const rgkc_ctx* c) {
-    const uint32_t cap = c->inst_cap ? c->inst_cap : (c->k <= 32 ? 8192u : 2304u);
+    const uint32_t cap = c->inst_cap ? c->inst_cap : (c->k <= 32 ? 16384u : 4608u);
     return std::min<uint32_t>(std::max<uint32_t>(cap, 256u), 1u << 19);
 }
 
@@ -482,7 +481,6 @@ int count_buckets(rgkc_ctx* c, uint32_t b0, uint32_t b1, uint32_t cmin, uint32_t
     a.k = c->k;
     a.cmin = cmin; a.cmax = cmax;
     a.unit_cap = (uint32_t)cap;
-    a.count_wg_per_cu = c->count_wg_per_cu;
     a.err = c->err_word.as<uint32_t>();
     a.stats = c->stats_dev.as<unsigned long long>();
     a.part_distinct = c->part_distinct.as<unsigned long long>();
@@ -1826,7 +1824,7 @@ int rgkc_set_sizing(rgkc_ctx* c, const double* distinct_pred, int parts, float m
 int rgkc_set_count_workgroups(rgkc_ctx* c, uint32_t per_cu) {
     if (!c) return RGKC_E_ARG;
     if (per_cu > 4) return fail(c, RGKC_E_ARG, "at most four count workgroups fit a CU");
-    c->count_wg_per_cu = per_cu;
+    // one workgroup of the count kernel takes a CU's LDS
     return 0;
 }
 

@@ -119,8 +119,8 @@ hipError_t launch_batch_prep(const uint8_t* reads, const uint64_t* offs, uint64_
 hipError_t launch_p1_batch(const P1Args& a, hipStream_t s);
 
 // ---- count (k_group.hip, k_count.hip) ----------------------------------------------------------
-// A unit of more than this many unit_caps is expanded into keys: at 30x, 1.2 G k-mers, the count stage
-// takes 13.6 ms with 1, 13.1 with 2, 13.6 with 3 (a direct unit is read once per sweep).
+// A unit of more than this many unit_caps is expanded into keys: the count stage takes 12.5 ms with 1 and
+// 12.1 with 2 (1.2 G k-mers at 30x), 2.43 and 1.96 (188 M, k=25): a unit is read once per sweep.
 constexpr uint32_t kDirectSlices = 2;
 constexpr uint32_t kMaxKeySlices = 127; // hash slices (key regions) of an expanded unit
 constexpr int kSmallUnits = 1024;       // units of a bucket that the small grouping kernel takes
@@ -165,7 +165,6 @@ struct CountArgs {
     int k;
     uint32_t cmin, cmax;
     uint32_t unit_cap;          // k-mer instances planned per sweep (distinct-capacity proxy)
-    uint32_t count_wg_per_cu;   // resident count workgroups per CU (0: as many as fit)
     uint32_t* err;
     unsigned long long* stats;  // [0] sweeps, [1] overflow retries, [2] distinct (unfiltered)
     unsigned long long* part_distinct;  // per partition: distinct keys (unfiltered)

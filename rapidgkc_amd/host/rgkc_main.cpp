@@ -299,7 +299,7 @@ void apply_tuning(rgkc_ctx* c, const Params& P) {
     FILE* f = fopen((dir + "/../autotune_cache.txt").c_str(), "r");
     if (!f) return;
     char prefix[128];
-    snprintf(prefix, sizeof prefix, "gfx950:k%d:p%d:parts%d:n", P.K, P.P, P.parts);
+    snprintf(prefix, sizeof prefix, "gfx950.2:k%d:p%d:parts%d:n", P.K, P.P, P.parts);
     const int want = (int)std::log2((double)std::max<long long>(P.gpu_batch_bases, 1));
     char line[512];
     int best_d = 1 << 30, cap = 0, wg = 0, lists = 1;

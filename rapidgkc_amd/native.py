@@ -239,7 +239,7 @@ class Counter:
         self._chk(self._L.rgkc_set_tuning(self._h, inst_per_sweep))
 
     def set_count_workgroups(self, per_cu: int = 0):
-        """Resident workgroups per CU of the persistent count kernel (0: four)."""
+        """Accepted and without effect: one workgroup of the count kernel takes a CU's LDS."""
         self._chk(self._L.rgkc_set_count_workgroups(self._h, per_cu))
 
     def set_memory_limit(self, nbytes: int = 0):
