@@ -465,37 +465,51 @@ __global__ __launch_bounds__(T, 3) void k_p1_count(P1Args a) {
     }
 }
 
+// Four record bytes 11|b0|b1|b2 from 12 LSB-first bases (the low 24 bits of x).
+__device__ __forceinline__ uint32_t record_bytes4(uint32_t x) {
+    uint32_t t = (x & 0xFFFu) | ((x & 0xFFF000u) << 4);
+    t = (t & 0x003F003Fu) | ((t & 0x0FC00FC0u) << 2);
+    return 0xC0C0C0C0u | ((t & 0x03030303u) << 4) | (t & 0x0C0C0C0Cu) | ((t >> 4) & 0x03030303u);
+}
+
 // Write record bytes [0, nb) of superkmer [b, e) of a read into dst (cpu_funcs.cpp:238-244).
 // Record byte x is packed-read byte m = b/3 + x: 11|b0|b1|b2 for a full group, the read's tail
-// byte (len%3)<<6 with its bases high, or 0 when len%3 == 0; then the first and last indicators
-// are patched. Ten bytes (30 bases) come from one 64-bit window of the 2-bit words.
+// byte (len%3)<<6 with its bases high, or 0 when len%3 == 0 (only the record's last byte can be that
+// one); then the first and last indicators are patched. Four bytes at a time, from one word pair: a byte
+// at a time took 43 instructions a byte, and the list emit was bound by them.
 __device__ __forceinline__ void write_record(const BaseSrc& src, uint64_t R0, uint32_t len, uint32_t b, uint32_t e, int k,
                                              uint32_t nb, uint8_t* dst) {
     const uint32_t m0 = b / 3u;
-    const uint32_t last_ind = ((e - 1u + (uint32_t)k) % 3u) << 6;
-    for (uint32_t x0 = 0; x0 < nb; x0 += 10u) {
-        const uint64_t pos = R0 + 3ull * (m0 + x0);
-        const uint64_t wi = pos >> 4;
-        const uint32_t sh = 2u * (uint32_t)(pos & 15);
-        uint64_t win = ((uint64_t)src.word(wi) | ((uint64_t)src.word(wi + 1) << 32)) >> sh;
-        if (sh) win |= (uint64_t)src.word(wi + 2) << (64u - sh);
-        const uint32_t xe = min(nb, x0 + 10u);
-        for (uint32_t x = x0; x < xe; x++) {
-            const uint32_t d = (uint32_t)(win >> (6u * (x - x0))) & 63u;  // b0 | b1 << 2 | b2 << 4
-            const uint32_t grp = ((d & 3u) << 4) | (d & 0xCu) | (d >> 4);  // b0 << 4 | b1 << 2 | b2
-            const uint32_t m = m0 + x;
-            uint32_t byte;
-            if (3u * m + 3u <= len) {
-                byte = 0xC0u | grp;
-            } else {
-                const uint32_t rem = len - 3u * m;  // 0, 1 or 2 (the read's tail byte)
-                byte = (rem << 6) | (grp & (rem == 2u ? 0x3Cu : rem == 1u ? 0x30u : 0u));
+    const uint64_t pos = R0 + 3ull * m0;
+    const uint32_t first_ind = (3u - (b - 3u * m0)) << 6, last_ind = ((e - 1u + (uint32_t)k) % 3u) << 6;
+    const int32_t rem = (int32_t)(len - 3u * (m0 + nb - 1u));  // of the read's bases from the last byte's first on
+    const uint32_t last_mask = rem >= 3 ? 0x3Fu : rem == 2 ? 0x3Cu : rem == 1 ? 0x30u : 0u;
+    auto bytes = [&](auto word, uint32_t p) {  // p: the record's first base, relative to word(0)
+        uint32_t x = 0;
+        for (;; x += 4u, p += 12u) {
+            uint32_t v = record_bytes4(__builtin_amdgcn_alignbit(word((p >> 4) + 1u), word(p >> 4), 2u * (p & 15u)));
+            if (x == 0) v = (v & ~0xC0u) | first_ind;
+            if (x + 4u < nb) {
+                __builtin_memcpy(dst + x, &v, 4);
+                continue;
             }
-            if (x == 0) byte = (byte & 0x3Fu) | ((3u - b % 3u) << 6);
-            if (x == nb - 1u) byte = (byte & 0x3Fu) | last_ind;
-            dst[x] = (uint8_t)byte;
+            // the last one to four bytes, the record's last byte patched
+            const uint32_t n = nb - x, sh = 8u * (n - 1u);
+            v = (v & ((1u << sh) - 1u)) | (((((v >> sh) & last_mask) | last_ind)) << sh);
+            if (n == 4u) {
+                __builtin_memcpy(dst + x, &v, 4);
+            } else {
+                if (n & 2u) { const uint16_t h = (uint16_t)v; __builtin_memcpy(dst + x, &h, 2); v >>= 16; }
+                if (n & 1u) dst[x + (n & 2u)] = (uint8_t)v;
+            }
+            break;
         }
-    }
+    };
+    // a record whose words are all staged is read from LDS (its first byte can begin up to two bases, and
+    // so a word, before the tile's first one: d is then past src.nw)
+    const uint64_t w = pos >> 4, d = w - src.w0;
+    if (d < src.nw && d + ((3u * nb + 15u) >> 4) + 2u < src.nw) bytes([&](uint32_t i) { return src.l[i]; }, (uint32_t)d * 16u + (uint32_t)(pos & 15u));
+    else bytes([&](uint32_t i) { return src.g[w + i]; }, (uint32_t)(pos & 15u));
 }
 
 // emit pass: records staged in LDS grouped by partition, then copied out in contiguous runs;
@@ -690,37 +704,48 @@ __device__ __forceinline__ uint32_t xcd_tile(uint32_t b, uint32_t n) {
 
 // Emit from the count pass's superkmer lists (exact mode): one workgroup per count-pass tile whose
 // list fit. Each list entry is one record: its slot in the tile's partition run comes from an LDS
-// cursor, and its side descriptor and bytes go straight to their place in HBM (the tile's runs
-// hold its records only, so nothing is staged). A small LDS footprint keeps several tiles per CU.
-// LDS of the list emit is sized so that three 256-thread workgroups share a CU (~51 KB each with
-// partition tables for up to 512 partitions)
+// cursor, the entry moves to its place in store order in LDS, and lane i writes the tile's i-th record
+// straight to its place in HBM, so the lanes of one store cover neighbouring records.
+// A tile's loads (its entries, run starts, segments) all start before anything waits, and two threads
+// per segment take the entries: with one, entries loaded in each pass from HBM and the records written a
+// byte at a time, the kernel took 3.5 ms for 114 M records (1.65 GB of store, 0.46 GB of side words) on
+// 12 waves a CU; written four bytes at a time 2.9, and so 2.4.
 constexpr uint32_t kListStageW = 2560;  // staged 2-bit words per tile (the rest read from HBM)
-constexpr uint32_t kReorderMax = 3840;  // list entries a tile can put in store order (more: list order)
+constexpr uint32_t kReorderMax = 3840;  // list entries a tile of 256 segments can put in store order (more: list order)
 
-template <int T, int PMAX>  // PMAX: partition-table size (parts <= PMAX)
-__global__ __launch_bounds__(T) void k_p1_emit_list(P1Args a) {
+template <int T, int TE, int PMAX>  // segments per tile, threads, partition-table size (parts <= PMAX)
+__global__ __launch_bounds__(TE) void k_p1_emit_list(P1Args a) {
+    constexpr uint32_t RM = kReorderMax * T / 256;
+    constexpr int EPT = (int)((RM + TE - 1) / TE);
+    static_assert(T <= TE, "a thread per segment");
     __shared__ uint32_t lw[kListStageW];
     __shared__ uint64_t seg_r0[T];
     __shared__ uint32_t seg_len[T], seg_s0[T];
     __shared__ uint64_t gbyte[PMAX], grec[PMAX];
     __shared__ unsigned long long pcur[PMAX];
-    // store order of the tile's records: roff[p] = records of partitions < p, then each entry's
-    // byte position in its run and the entry at each store-order place
-    __shared__ uint32_t roff[PMAX];
-    __shared__ uint32_t rpos[kReorderMax];
-    __shared__ uint16_t order[kReorderMax];
-    __shared__ uint32_t tmp[T / 64 + 1];
+    __shared__ uint32_t roff[PMAX];  // records of the tile's partitions before each
+    __shared__ uint64_t ent[RM];     // the tile's entries in store order, and each one's byte position in its run
+    __shared__ uint32_t epos[RM];
+    __shared__ uint32_t tmp[TE / 64 + 1];
     const uint64_t n_seg = a.n_seg_dev ? *a.n_seg_dev : a.n_seg;
     const uint32_t n_tiles = (uint32_t)((n_seg + T - 1) / T);  // batched input: the grid covers the batch capacity
     if (blockIdx.x >= n_tiles) return;
     const uint32_t wg = xcd_tile(blockIdx.x, n_tiles);
     const uint32_t n_list = a.skm_n[wg];
     if (n_list > a.skm_cap) return;  // rescanned by the scanning emit
+    const uint64_t* const lst = a.skm_list + (size_t)wg * a.skm_cap;
+    const bool reorder = n_list <= RM;
+    uint64_t v[EPT];
+#pragma unroll
+    for (int j = 0; j < EPT; j++) {
+        const uint32_t x = threadIdx.x + (uint32_t)j * TE;
+        v[j] = reorder && x < n_list ? lst[x] : 0ull;
+    }
     const int k = a.k;
     const uint32_t parts = (uint32_t)a.parts;
     const FastDivU32 pdiv = FastDivU32::make(parts);
     const size_t stride = (size_t)a.n_wg + 1;
-    for (uint32_t i = threadIdx.x; i < parts; i += T) {
+    for (uint32_t i = threadIdx.x; i < parts; i += TE) {
         uint64_t bo, ro;
         uint32_t nbp, nrp;
         if (a.list_reserve) {
@@ -752,23 +777,10 @@ __global__ __launch_bounds__(T) void k_p1_emit_list(P1Args a) {
         pcur[i] = 0;
         roff[i] = nrp;
     }
-    const bool reorder = n_list <= kReorderMax;
-    if (reorder) {
-        __syncthreads();
-        uint32_t carry = 0;
-        for (uint32_t c0 = 0; c0 < parts; c0 += T) {
-            const uint32_t i = c0 + threadIdx.x;
-            const uint32_t v = i < parts ? roff[i] : 0u;
-            uint32_t tot;
-            const uint32_t ex = wg_exscan_u32(v, tmp, &tot);
-            if (i < parts) roff[i] = carry + ex;
-            carry += tot;
-        }
-    }
     const uint64_t seg_lo = (uint64_t)wg * T;
     const uint64_t seg_hi = min(n_seg, seg_lo + T);
     const uint64_t s = seg_lo + threadIdx.x;
-    if (s < seg_hi) {
+    if (threadIdx.x < (uint32_t)T && s < seg_hi) {
         const uint32_t rd = a.seg_read[s];
         const uint64_t R0 = a.offs[rd];
         seg_r0[threadIdx.x] = R0;
@@ -776,45 +788,55 @@ __global__ __launch_bounds__(T) void k_p1_emit_list(P1Args a) {
         seg_s0[threadIdx.x] = a.seg_first[s];
     }
     BaseSrc src;
-    stage_bases<T>(a, lw, kListStageW, src, seg_lo, seg_hi);  // ends with a barrier
-    const uint64_t* lst = a.skm_list + (size_t)wg * a.skm_cap;
+    stage_bases<TE>(a, lw, kListStageW, src, seg_lo, seg_hi);  // ends with a barrier
+    const uint32_t n_here = (uint32_t)(seg_hi - seg_lo);
     if (reorder) {
-        // pass 1: slots; pass 2: lane i writes the tile's i-th record in store order, so the
-        // lanes of one store cover neighbouring records instead of 64 unrelated places. Every
-        // store-order place is filled when the count pass's histograms match its list; a place
-        // left at the 0xFFFF mark means they do not, and is reported instead of read.
-        for (uint32_t i = threadIdx.x; i < n_list; i += T) order[i] = 0xFFFFu;
+        {
+            uint32_t carry = 0;
+            for (uint32_t c0 = 0; c0 < parts; c0 += TE) {
+                const uint32_t i = c0 + threadIdx.x;
+                const uint32_t nr = i < parts ? roff[i] : 0u;
+                uint32_t tot;
+                const uint32_t ex = wg_exscan_u32(nr, tmp, &tot);
+                if (i < parts) roff[i] = carry + ex;
+                carry += tot;
+            }
+        }
+        // Every store-order place is filled when the count pass's histograms match its list; a place
+        // left at the mark means they do not, and is reported instead of read.
+        for (uint32_t i = threadIdx.x; i < n_list; i += TE) ent[i] = ~0ull;
         __syncthreads();
-        for (uint32_t x = threadIdx.x; x < n_list; x += T) {
-            const uint64_t v = lst[x];
-            const uint32_t t = (uint32_t)(v >> 32) & 0xFFu;
-            const uint32_t b = seg_s0[t] + ((uint32_t)(v >> 40) & 0x7Fu);
-            if ((uint64_t)b + (v >> 47) + (uint64_t)k - 1u > seg_len[t]) {  // not a superkmer of its read
+#pragma unroll
+        for (int j = 0; j < EPT; j++) {
+            if (threadIdx.x + (uint32_t)j * TE >= n_list) break;
+            const uint32_t t = (uint32_t)(v[j] >> 32) & 0xFFu;
+            const uint32_t b = t < n_here ? seg_s0[t] + ((uint32_t)(v[j] >> 40) & 0x7Fu) : 0u;
+            if (t >= n_here || (uint64_t)b + (v[j] >> 47) + (uint64_t)k - 1u > seg_len[t]) {  // not a superkmer of its read
                 raise_err(a.err, RGKC_ERR_BAD_STORE);
-                rpos[x] = 0;
                 continue;
             }
-            const uint32_t part = pdiv.mod(~(uint32_t)v);
-            const uint32_t nb = skm_nbytes(b % 3u, (uint32_t)(v >> 47) + (uint32_t)k - 1u);
+            const uint32_t part = pdiv.mod(~(uint32_t)v[j]);
+            const uint32_t nb = skm_nbytes(b % 3u, (uint32_t)(v[j] >> 47) + (uint32_t)k - 1u);
             const unsigned long long old = atomicAdd(&pcur[part], ((unsigned long long)nb << 32) | 1ull);
-            rpos[x] = (uint32_t)(old >> 32);
             const uint32_t oi = roff[part] + (uint32_t)old;  // < n_list: the count pass counted these records
-            if (oi < n_list) order[oi] = (uint16_t)x;
-            else raise_err(a.err, RGKC_ERR_BAD_STORE);
+            if (oi < n_list) {
+                ent[oi] = v[j];
+                epos[oi] = (uint32_t)(old >> 32);
+            } else {
+                raise_err(a.err, RGKC_ERR_BAD_STORE);
+            }
         }
         __syncthreads();
-        for (uint32_t i = threadIdx.x; i < n_list; i += T) {
-            const uint32_t x = order[i];
-            if (x >= n_list) {  // an unfilled place (0xFFFF): histograms and list disagree
+        for (uint32_t i = threadIdx.x; i < n_list; i += TE) {
+            const uint64_t e = ent[i];
+            if (e == ~0ull) {  // an unfilled place: histograms and list disagree
                 raise_err(a.err, RGKC_ERR_BAD_STORE);
                 continue;
             }
-            const uint64_t v = lst[x];
-            const uint32_t t = (uint32_t)(v >> 32) & 0xFFu;
-            const uint32_t b = seg_s0[t] + ((uint32_t)(v >> 40) & 0x7Fu);
-            const uint32_t kmers = (uint32_t)(v >> 47);
-            if ((uint64_t)b + kmers + (uint64_t)k - 1u > seg_len[t]) continue;  // reported by pass 1
-            const uint32_t nmm = ~(uint32_t)v;
+            const uint32_t t = (uint32_t)(e >> 32) & 0xFFu;
+            const uint32_t b = seg_s0[t] + ((uint32_t)(e >> 40) & 0x7Fu);
+            const uint32_t kmers = (uint32_t)(e >> 47);
+            const uint32_t nmm = ~(uint32_t)e;
             const uint32_t q = pdiv.div(nmm);
             const uint32_t part = nmm - q * parts;
             const uint32_t sub = q % (uint32_t)kSubIds;
@@ -822,21 +844,21 @@ __global__ __launch_bounds__(T) void k_p1_emit_list(P1Args a) {
             if (grec[part] != ~0ull)
                 a.side[grec[part] + (i - roff[part])] = side_pack(sub, kmers > 0x3FFFFu ? 0x3FFFFu : kmers, b % 3u);
             if (gbyte[part] != ~0ull)
-                write_record(src, seg_r0[t], seg_len[t], b, b + kmers, k, nb, a.store + gbyte[part] + rpos[x]);
+                write_record(src, seg_r0[t], seg_len[t], b, b + kmers, k, nb, a.store + gbyte[part] + epos[i]);
         }
         return;
     }
     if (threadIdx.x == 0 && a.n_listorder) atomicAdd(a.n_listorder, 1u);  // tile written in list order
-    for (uint32_t x = threadIdx.x; x < n_list; x += T) {
-        const uint64_t v = lst[x];
-        const uint32_t t = (uint32_t)(v >> 32) & 0xFFu;
-        const uint32_t b = seg_s0[t] + ((uint32_t)(v >> 40) & 0x7Fu);
-        const uint32_t kmers = (uint32_t)(v >> 47);
-        if ((uint64_t)b + kmers + (uint64_t)k - 1u > seg_len[t]) {  // not a superkmer of its read
+    for (uint32_t x = threadIdx.x; x < n_list; x += TE) {
+        const uint64_t e = lst[x];
+        const uint32_t t = (uint32_t)(e >> 32) & 0xFFu;
+        const uint32_t b = t < n_here ? seg_s0[t] + ((uint32_t)(e >> 40) & 0x7Fu) : 0u;
+        const uint32_t kmers = (uint32_t)(e >> 47);
+        if (t >= n_here || (uint64_t)b + kmers + (uint64_t)k - 1u > seg_len[t]) {  // not a superkmer of its read
             raise_err(a.err, RGKC_ERR_BAD_STORE);
             continue;
         }
-        const uint32_t nmm = ~(uint32_t)v;
+        const uint32_t nmm = ~(uint32_t)e;
         const uint32_t q = pdiv.div(nmm);
         const uint32_t part = nmm - q * parts;
         const uint32_t sub = q % (uint32_t)kSubIds;
@@ -913,15 +935,17 @@ hipError_t launch_batch_prep(const uint8_t* reads, const uint64_t* offs, uint64_
     return hipGetLastError();
 }
 
-// The list emit over all tiles, with partition tables sized for a.parts.
+// The list emit over all tiles, with partition tables sized for a.parts: two workgroups of 512 threads share
+// a CU with tables for 512 partitions (75 KB of LDS), one of 1024 takes it with the full ones; tiles of 128
+// segments (49 KB) three of 256.
 static hipError_t launch_list(const P1Args& a, bool big, hipStream_t s) {
     const bool small = a.parts <= 512;
     if (!big) {
-        if (small) hipLaunchKernelGGL((k_p1_emit_list<256, 512>), dim3(a.n_wg), dim3(256), 0, s, a);
-        else hipLaunchKernelGGL((k_p1_emit_list<256, kMaxParts>), dim3(a.n_wg), dim3(256), 0, s, a);
+        if (small) hipLaunchKernelGGL((k_p1_emit_list<256, 512, 512>), dim3(a.n_wg), dim3(512), 0, s, a);
+        else hipLaunchKernelGGL((k_p1_emit_list<256, 1024, kMaxParts>), dim3(a.n_wg), dim3(1024), 0, s, a);
     } else {
-        if (small) hipLaunchKernelGGL((k_p1_emit_list<128, 512>), dim3(a.n_wg), dim3(128), 0, s, a);
-        else hipLaunchKernelGGL((k_p1_emit_list<128, kMaxParts>), dim3(a.n_wg), dim3(128), 0, s, a);
+        if (small) hipLaunchKernelGGL((k_p1_emit_list<128, 256, 512>), dim3(a.n_wg), dim3(256), 0, s, a);
+        else hipLaunchKernelGGL((k_p1_emit_list<128, 512, kMaxParts>), dim3(a.n_wg), dim3(512), 0, s, a);
     }
     return hipGetLastError();
 }
