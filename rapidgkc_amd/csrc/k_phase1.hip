@@ -265,18 +265,33 @@ __device__ __forceinline__ void stage_bases(const P1Args& a, uint32_t* lds_w, ui
     __syncthreads();
 }
 
+// Hardware places workgroup b on XCD b % 8: give each XCD one contiguous range of tiles, so the
+// partition runs of neighbouring tiles (adjacent in the store) meet in one L2.
+__device__ __forceinline__ uint32_t xcd_tile(uint32_t b, uint32_t n) {
+    const uint32_t x = b % 8u, q = n / 8u, r = n % 8u;
+    return x * q + min(x, r) + b / 8u;
+}
+
 // ---------------------------------------------------------------------------------------------
 // count pass: per-(partition, workgroup) histograms of record bytes, records and k-mers, and
 // (when a.skm_list is set) the workgroup's superkmer list for the emit pass.
 //
-// The lanes of a wave step together: at step j every lane reads base i0 + j of its own segment
+// The lanes of a wave step together: at step j every lane ends a p-mer at base i0 + j of its own segment
 // (i0: the segment's first k-mer, or the one before it as look-back), so the window ring index, the
 // warm-up and the block ends of the window minimum are the same in all lanes. Each lane reads its
-// bases from HBM as 16-base words realigned to its segment, loaded two words ahead of use. A minimizer
+// bases from HBM as 16-base words realigned to its segment, loaded two words ahead of use. A p-mer and its
+// reverse complement are cut out of the words (no step depends on the one before), and which of them the
+// minimizer filter drops is worked out for 16 steps at once, a bit each. A minimizer
 // change is only noted in a per-lane LDS queue (its k-mer step and minimizer) by straight-line
 // code; the queue is drained by the whole wave at once every few steps, where each lane turns its
 // complete superkmers into histogram counts and list entries. So the per-superkmer work runs once
-// per superkmer instead of once per step of any lane that emits.
+// per superkmer instead of once per step of any lane that emits. Steps that no lane of the wave has near
+// its segment's end skip the rules for it.
+//
+// Bound by instructions: 10 M reads of 150 bp (k = 31, p = 11, 24 M wave steps) took 3.2 ms at 50 vector and 46
+// scalar ones a step, with p-mers shifted in base by base and tested one by one; so 2.2 ms, on 12 waves a CU (the
+// ring and the queue fill LDS). Tiles go to the XCDs in ranges as in the emit pass, or the three histogram
+// columns that neighbouring tiles write meet in no L2: 3.4 ms before that.
 constexpr int kEvQ = 8;      // queued events per lane
 constexpr int kEvChunk = 4;  // steps between queue checks (a lane adds at most one event per step)
 
@@ -296,16 +311,18 @@ __global__ __launch_bounds__(T, 3) void k_p1_count(P1Args a) {
     const int tid = threadIdx.x;
     const uint32_t lane = (uint32_t)tid & 63u;
     const uint64_t n_seg = a.n_seg_dev ? *a.n_seg_dev : a.n_seg;
-    const uint64_t seg_lo = (uint64_t)blockIdx.x * T;
+    const uint32_t n_tiles = (uint32_t)((n_seg + T - 1) / T);
+    if (blockIdx.x >= n_tiles) return;  // batched input: the grid covers the batch capacity
+    const uint32_t wg = xcd_tile(blockIdx.x, n_tiles);
+    const uint64_t seg_lo = (uint64_t)wg * T;
     const uint64_t seg_hi = min(n_seg, seg_lo + T);
-    if (seg_lo >= n_seg) return;  // batched input: the grid covers the batch capacity
     for (int i = tid; i < a.parts; i += T) { hb[i] = 0; hr[i] = 0; hk[i] = 0; }
     if (tid == 0) { lcnt = 0; lbad = 0; }
     __syncthreads();
     const uint64_t s = seg_lo + (uint64_t)tid;
     const bool has = s < seg_hi;
     uint64_t pos0 = 0;
-    uint32_t s0 = 0, i0 = 0, jend = 0, js1 = 0;
+    uint32_t s0 = 0, i0 = 0, jend = 0xFFFFFFFFu, js1 = 0xFFFFFFFFu;
     if (has) {
         const uint32_t rd = a.seg_read[s];
         const uint64_t R0 = a.offs[rd];
@@ -318,21 +335,84 @@ __global__ __launch_bounds__(T, 3) void k_p1_count(P1Args a) {
         jend = len - i0;                     // step after the read's last k-mer
         js1 = s1 - i0 + (uint32_t)k - 1u;   // step of k-mer s1 (the next segment's first)
     }
-    // raw words wi, wi + 1, ... of the 2-bit stream (clamped to the array) realigned by sh
+    uint32_t jfast = min(js1, jend);  // before this step no lane of the wave ends
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) jfast = min(jfast, (uint32_t)__shfl_xor((int)jfast, d));
+    jfast = (uint32_t)__builtin_amdgcn_readfirstlane((int)jfast);
+    // The lane's bases as aligned words: block m holds the steps j = k + 16 m + jj, jj in [0, 16), whose
+    // p-mers end at base 15 + jj of the word pair (prev, cur). The first block is the one of step p - 1; its
+    // words may begin before the read (and the array: the clamp), no p-mer does.
     const uint32_t* const g = a.bases2;
-    const uint64_t last_w = (a.n_bases >> 4) + 1;
-    uint64_t wi = pos0 >> 4;
-    const uint32_t sh = 2u * (uint32_t)(pos0 & 15);
-    auto raw = [&](uint64_t i) __attribute__((always_inline)) { return g[i < last_w ? i : last_w]; };
-    uint32_t r_lo = raw(wi), r_hi = raw(wi + 1), r_nx = raw(wi + 2);
-    wi += 3;
-    const uint32_t pmask = (p >= 16) ? 0xFFFFFFFFu : ((1u << (2 * p)) - 1u);
-    const uint32_t rsh = 2u * (uint32_t)(p - 1);
+    const int64_t last_w = (int64_t)(a.n_bases >> 4) + 1;
+    const int64_t first = (int64_t)pos0 + k - 15 - 16 * (int64_t)((w + 15u) / 16u);
+    int64_t wi = (first >> 4) - 1;  // one word more: p = 16 reaches back to base -1 of prev
+    const uint32_t sh = 2u * (uint32_t)(first & 15);
+    auto raw = [&](int64_t i) __attribute__((always_inline)) { return g[i < 0 ? 0 : i < last_w ? i : last_w]; };
+    uint32_t r_lo, r_hi, r_nx, prev_w, cur_w, vpp, vprev, vcur;  // v*: the words with base 0 on top
+    auto turn = [](uint32_t x) __attribute__((always_inline)) {
+        x = __builtin_bitreverse32(x);
+        return ((x >> 1) & 0x55555555u) | ((x << 1) & 0xAAAAAAAAu);
+    };
+    {
+        const uint32_t x0 = raw(wi), x1 = raw(wi + 1), x2 = raw(wi + 2);
+        r_lo = x2;
+        r_hi = raw(wi + 3);
+        r_nx = raw(wi + 4);
+        wi += 5;
+        prev_w = __builtin_amdgcn_alignbit(x1, x0, sh);
+        cur_w = __builtin_amdgcn_alignbit(x2, x1, sh);
+        vprev = turn(prev_w);
+        vcur = turn(cur_w);
+        vpp = vprev;
+    }
+    // The block's words: the p-mer that ends at step jj is the top 2p bits of (fc:fn) << 2 (jj + 1), its reverse
+    // complement of (nc:np) >> 2 jj; bits 2 jj + 1 of bad_f and bad_r say which the filter drops.
+    uint32_t fc = 0, fn = 0, np = 0, nc = 0, bad_f = 0, bad_r = 0;
+    const uint32_t sa = 2u * (uint32_t)(15 - (p < 16 ? p : 15));
+    auto block = [&]() __attribute__((always_inline)) {
+        vpp = vprev;
+        vprev = vcur;
+        const uint32_t pp_w = prev_w;
+        prev_w = cur_w;
+        cur_w = __builtin_amdgcn_alignbit(r_hi, r_lo, sh);
+        r_lo = r_hi;
+        r_hi = r_nx;
+        r_nx = raw(wi++);
+        vcur = turn(cur_w);
+        uint32_t wc, wn;  // (wc:wn): from base 15 - p of (prev:cur), where the p-mer of step -1 starts
+        if (p == 16) {
+            fc = __builtin_amdgcn_alignbit(vpp, vprev, 2);
+            fn = __builtin_amdgcn_alignbit(vprev, vcur, 2);
+            wc = __builtin_amdgcn_alignbit(prev_w, pp_w, 30);
+            wn = __builtin_amdgcn_alignbit(cur_w, prev_w, 30);
+        } else {
+            fc = sa ? __builtin_amdgcn_alignbit(vprev, vcur, 32u - sa) : vprev;
+            fn = vcur << sa;
+            wc = __builtin_amdgcn_alignbit(cur_w, prev_w, sa);
+            wn = cur_w >> sa;
+        }
+        np = ~prev_w;
+        nc = ~cur_w;
+        // bases e, e - 1, e - 2 of each step's p-mer [s, e], and s, s + 1, s + 2
+        const uint32_t y0 = __builtin_amdgcn_alignbit(cur_w, prev_w, 30), y1 = __builtin_amdgcn_alignbit(cur_w, prev_w, 28),
+                       y2 = __builtin_amdgcn_alignbit(cur_w, prev_w, 26);
+        const uint32_t z0 = __builtin_amdgcn_alignbit(wn, wc, 2), z1 = __builtin_amdgcn_alignbit(wn, wc, 4),
+                       z2 = __builtin_amdgcn_alignbit(wn, wc, 6);
+        const uint32_t t = y0 | y1 | y2, u = z0 & z1 & z2;
+        bad_f = ~((t | (t << 1)) & (z0 | z1 | z2 | (z2 << 1)));  // ends in AAA, or starts with [AC][AC]A
+        bad_r = (y0 & y1 & y2 & (y2 << 1)) | (u & (u << 1));     // the same of the reverse complement
+    };
+    const uint32_t mm_sh = 32u - 2u * (uint32_t)p, top = 0xFFFFFFFFu << mm_sh;
+    // the smaller of the step's p-mer and its reverse complement, top-justified (all ones if both are dropped)
+    auto pmer = [&](uint32_t jj) __attribute__((always_inline)) {
+        const uint32_t f = __builtin_amdgcn_alignbit(fc, fn, 30u - 2u * jj) | (uint32_t)__builtin_amdgcn_sbfe((int)bad_f, 2u * jj + 1u, 1u);
+        const uint32_t r = __builtin_amdgcn_alignbit(nc, np, 2u * jj) | (uint32_t)__builtin_amdgcn_sbfe((int)bad_r, 2u * jj + 1u, 1u);
+        return (f < r ? f : r) & top;
+    };
     const FastDivU32 pdiv = FastDivU32::make((uint32_t)a.parts);
-    uint64_t* const lst = a.skm_list ? a.skm_list + (size_t)blockIdx.x * a.skm_cap : nullptr;
+    uint64_t* const lst = a.skm_list ? a.skm_list + (size_t)wg * a.skm_cap : nullptr;
     bool done = !has, open = false;
-    uint32_t qn = 0, f = 0, r = 0, pm = 0, prev = 0, W = 0;
-    uint32_t bu = w - 1u;  // ring slot of the current p-mer within its block (the same in every lane)
+    uint32_t qn = 0;
     unsigned long long* const myq = evq + tid;
     // superkmer [b, e) with minimizer mm, list slot li
     auto record = [&](uint32_t b, uint32_t e, uint32_t mm, uint32_t li) __attribute__((always_inline)) {
@@ -367,7 +447,7 @@ __global__ __launch_bounds__(T, 3) void k_p1_count(P1Args a) {
             const unsigned long long e1 = myq[(size_t)(t + 1) * T];
             const uint32_t b = kb + ((uint32_t)(e0 >> 32) & 0x7FFFFFFFu);
             const uint32_t e = kb + ((uint32_t)(e1 >> 32) & 0x7FFFFFFFu);
-            record(b, e, (uint32_t)e0, li + t);
+            record(b, e, (uint32_t)e0 >> mm_sh, li + t);
             e0 = e1;
         }
         if (qn) {
@@ -375,77 +455,105 @@ __global__ __launch_bounds__(T, 3) void k_p1_count(P1Args a) {
             else qn = 0;
         }
     };
+    // Window minimum over blocks of w p-mers (van Herk / Gil-Werman): pm is the prefix minimum of the current
+    // block; at a block's end its ring slots are rewritten with suffix minima, and a window that starts in
+    // the previous block is min(suffix there, pm). Slot w is all ones: the last window of a block.
     uint32_t* const rbase = ring + tid;
-    for (uint32_t j0 = 0;; j0 += kEvChunk) {
-        if ((j0 & 15u) == 0u) {  // next word; fetch the one after it
-            W = __builtin_amdgcn_alignbit(r_hi, r_lo, sh);
-            r_lo = r_hi;
-            r_hi = r_nx;
-            r_nx = raw(wi++);
-        }
+    uint32_t* slot = rbase;
+    uint32_t pm = 0xFFFFFFFFu, bu = 0, sfx;
+    rbase[(size_t)w * T] = 0xFFFFFFFFu;
+    auto advance = [&]() __attribute__((always_inline)) {  // to the next step's slot; its suffix is loaded ahead of use
+        slot += T;
+        if (++bu == w) {
+            uint32_t sm = 0xFFFFFFFFu;
+            uint32_t* q = rbase + (size_t)(w - 1u) * T;
+            int sl = (int)w - 1;
+            for (; sl >= 8; sl -= 8, q -= 8 * T) {
+                uint32_t x[8];
 #pragma unroll
-        for (int t = 0; t < kEvChunk; t++) {
-            const uint32_t j = j0 + (uint32_t)t;
-            const uint32_t c = (W >> (2u * (j & 15u))) & 3u;
-            f = ((f << 2) | c) & pmask;
-            r = (r >> 2) | ((3u - c) << rsh);
-            if (j + 1u < (uint32_t)p) continue;
-            // window minimum over blocks of w p-mers (van Herk / Gil-Werman): pm is the prefix
-            // minimum of the current block; at a block end the block's ring slots are rewritten
-            // with suffix minima, and a window that starts in the previous block is
-            // min(suffix there, pm)
-            bu = (bu + 1u == w) ? 0u : bu + 1u;
-            uint32_t* const slot = rbase + (size_t)bu * T;
-            const uint32_t sfx = slot[T];
-            const uint32_t vf = pmer_valid(f, p) ? f : pmask;
-            const uint32_t vr = pmer_valid(r, p) ? r : pmask;
-            const uint32_t v = vf < vr ? vf : vr;
-            pm = bu == 0u ? v : (v < pm ? v : pm);
-            const bool bend = bu + 1u == w;
-            const uint32_t mm = bend ? pm : (sfx < pm ? sfx : pm);
-            slot[0] = v;
-            if (bend) {
-                uint32_t sm = 0xFFFFFFFFu;
-                int sl = (int)w - 1;
-                for (; sl >= 3; sl -= 4) {
-                    uint32_t* const q = rbase + (size_t)sl * T;
-                    uint32_t x0 = q[0], x1 = q[-T], x2 = q[-2 * T], x3 = q[-3 * T];
-                    x0 = x0 < sm ? x0 : sm;
-                    x1 = x1 < x0 ? x1 : x0;
-                    x2 = x2 < x1 ? x2 : x1;
-                    x3 = x3 < x2 ? x3 : x2;
-                    q[0] = x0; q[-T] = x1; q[-2 * T] = x2; q[-3 * T] = x3;
-                    sm = x3;
-                }
-                for (; sl >= 0; sl--) {
-                    uint32_t* const q = rbase + (size_t)sl * T;
-                    const uint32_t x = q[0] < sm ? q[0] : sm;
-                    q[0] = x;
-                    sm = x;
-                }
+                for (int i = 0; i < 8; i++) x[i] = q[-i * T];
+#pragma unroll
+                for (int i = 0; i < 8; i++) q[-i * T] = sm = min(x[i], sm);
             }
-            if (j + 1u < (uint32_t)k) continue;
-            // events, without branches: the entry is written to queue slot qn in every step and
-            // kept (qn advanced) only when it is one
-            bool ev, term;
-            if (j + 1u == (uint32_t)k) {  // k-mer i0: a start when the segment begins the read, else the look-back
-                ev = !done && s0 == 0u;
-                term = false;
-                open = ev;
-            } else {
+            if (sl & 4) {
+                uint32_t x[4];
+#pragma unroll
+                for (int i = 0; i < 4; i++) x[i] = q[-i * T];
+#pragma unroll
+                for (int i = 0; i < 4; i++) q[-i * T] = sm = min(x[i], sm);
+                q -= 4 * T;
+            }
+            for (sl &= 3; sl > 0; sl--, q -= T) q[0] = sm = min(q[0], sm);
+            bu = 0;
+            slot = rbase;
+            pm = 0xFFFFFFFFu;
+        }
+        sfx = slot[T];
+    };
+    // the first window: steps p - 1 .. k - 1
+    uint32_t prev;
+    {
+        uint32_t jj = (uint32_t)(16 - (int)(w & 15u)) & 15u;
+        block();
+        for (uint32_t t = 0;; jj++) {
+            if (jj == 16u) {
+                block();
+                jj = 0;
+            }
+            const uint32_t v = pmer(jj);
+            pm = min(pm, v);
+            *slot = v;
+            if (++t == w) break;
+            slot += T;
+        }
+        prev = pm;
+        bu = w - 1u;
+        advance();
+        // k-mer i0: a start when the segment begins the read, else the look-back
+        if (!done && s0 == 0u) {
+            open = true;
+            myq[0] = (unsigned long long)prev | ((unsigned long long)(uint32_t)(k - 1) << 32);
+            qn = 1;
+        }
+    }
+    for (uint32_t j0 = (uint32_t)k, jb = 0;; j0 += kEvChunk, jb = (jb + kEvChunk) & 15u) {
+        if (jb == 0u) block();
+        if (j0 + (uint32_t)kEvChunk <= jfast) {
+#pragma unroll
+            for (int t = 0; t < kEvChunk; t++) {
+                const uint32_t v = pmer(jb + (uint32_t)t);
+                pm = min(pm, v);
+                const uint32_t mm = min(sfx, pm);
+                *slot = v;
+                advance();
+                // events, without branches: the entry is written to queue slot qn in every step and
+                // kept (qn advanced) only when it is one
+                const bool chg = !done && mm != prev;
+                open = open || chg;
+                myq[(size_t)qn * T] = (unsigned long long)mm | ((unsigned long long)(j0 + (uint32_t)t) << 32);
+                qn += chg ? 1u : 0u;
+                prev = mm;
+            }
+        } else {
+            for (int t = 0; t < kEvChunk; t++) {
+                const uint32_t j = j0 + (uint32_t)t;
+                const uint32_t v = pmer(jb + (uint32_t)t);
+                pm = min(pm, v);
+                const uint32_t mm = min(sfx, pm);
+                *slot = v;
+                advance();
                 const bool past = j >= js1;  // k-mer index >= s1
                 const bool stop = !done && past && !open;
                 const bool rend = !done && !stop && j >= jend;
                 const bool chg = !done && !stop && !rend && mm != prev;
-                ev = (rend && open) || chg;
-                term = rend || (chg && past);
+                const bool ev = (rend && open) || chg;
+                const bool term = rend || (chg && past);
                 open = open || (chg && !past);
                 done = done || stop || rend || (chg && past);
+                myq[(size_t)qn * T] = (unsigned long long)mm | ((unsigned long long)(term ? j | 0x80000000u : j) << 32);
+                qn += ev ? 1u : 0u;
+                prev = mm;
             }
-            myq[(size_t)qn * T] = term ? ((unsigned long long)(j | 0x80000000u) << 32)
-                                       : ((unsigned long long)mm | ((unsigned long long)j << 32));
-            qn += ev ? 1u : 0u;
-            prev = mm;
         }
         const bool any_left = __ballot(!done) != 0ull;
         if (!any_left || __ballot(qn + (uint32_t)kEvChunk >= (uint32_t)kEvQ) != 0ull) drain();
@@ -454,14 +562,14 @@ __global__ __launch_bounds__(T, 3) void k_p1_count(P1Args a) {
     __syncthreads();
     if (a.skm_list && threadIdx.x == 0) {
         const bool over = lbad || lcnt > a.skm_cap;
-        a.skm_n[blockIdx.x] = over ? a.skm_cap + 1u : lcnt;
-        if (over) a.wg_rescan[atomicAdd(a.n_rescan, 1u)] = blockIdx.x;
+        a.skm_n[wg] = over ? a.skm_cap + 1u : lcnt;
+        if (over) a.wg_rescan[atomicAdd(a.n_rescan, 1u)] = wg;
     }
     const size_t stride = (size_t)a.n_wg + 1;
     for (int i = threadIdx.x; i < a.parts; i += T) {
-        a.h_bytes[(size_t)i * stride + blockIdx.x] = hb[i];
-        a.h_recs[(size_t)i * stride + blockIdx.x] = hr[i];
-        a.h_kmers[(size_t)i * stride + blockIdx.x] = hk[i];
+        a.h_bytes[(size_t)i * stride + wg] = hb[i];
+        a.h_recs[(size_t)i * stride + wg] = hr[i];
+        a.h_kmers[(size_t)i * stride + wg] = hk[i];
     }
 }
 
@@ -693,13 +801,6 @@ template <int RING, int T>
 __global__ __launch_bounds__(T) void k_p1_emit(P1Args a) {
     __shared__ EmitLds<RING, T> L;
     emit_tile<RING, T, false>(a, a.wg_map ? a.wg_map[blockIdx.x] : blockIdx.x, a.n_seg, L);
-}
-
-// Hardware places workgroup b on XCD b % 8: give each XCD one contiguous range of tiles, so the
-// partition runs of neighbouring tiles (adjacent in the store) meet in one L2.
-__device__ __forceinline__ uint32_t xcd_tile(uint32_t b, uint32_t n) {
-    const uint32_t x = b % 8u, q = n / 8u, r = n % 8u;
-    return x * q + min(x, r) + b / 8u;
 }
 
 // Emit from the count pass's superkmer lists (exact mode): one workgroup per count-pass tile whose

@@ -2,7 +2,7 @@
 or 2 bases past a byte, first bytes at each of a read's three phases, records of each length modulo four,
 short reads (a tile's words all staged) and long ones (only some of them), 1 partition and both table sizes,
 tiles of 256 and of 128 segments, and windows so short that a tile has more records than it can put in
-order. Bytes: equal to the oracle's."""
+order; and the minimizers that cut them. Bytes: equal to the oracle's."""
 import numpy as np
 import pytest
 
@@ -28,4 +28,25 @@ def test_list_records(k, p, parts, long):
     c.set_reads(chars, offs)
     for _ in range(2):
         check_store(c, chars, offs, k, p, parts)
+    c.close()
+
+
+@pytest.mark.parametrize("k,p", [(8, 8), (8, 3), (16, 16), (17, 16), (31, 16), (32, 16), (33, 16), (31, 15), (31, 14), (22, 7),
+                                 (24, 9), (25, 9), (39, 8), (40, 9), (42, 11), (63, 16), (63, 4), (63, 3)])
+def test_minimizers(k, p):
+    """p-mers cut out of the packed words: every phase of a window to the 16-base words (w = k - p + 1 from 1 to
+    61, blocks of 8, 4 and 1 suffix minima), p = 16 (one word back), reads that start anywhere in a word,
+    and reads of which the filter drops all p-mers, those of one strand, or many."""
+    from rapidgkc_amd import native
+    print(f"[gpu] case minimizers k{k} p{p}", flush=True)
+    rng = np.random.default_rng(1000 * k + p)
+    reads = [rng.choice(np.frombuffer(b"ACGT", dtype=np.uint8), int(n)) for n in rng.integers(k, 330, 1500)]
+    reads += [rng.choice(np.frombuffer(alpha, dtype=np.uint8), int(n)) for alpha in (b"A", b"T", b"AC", b"GT", b"AT", b"AAAAAAAC",
+              b"TTTTTTTG", b"CG") for n in (k, k + 1, k + 17, 200, 500)]
+    offs = np.zeros(len(reads) + 1, dtype=np.uint64)
+    np.cumsum([len(r) for r in reads], out=offs[1:])
+    chars = np.concatenate(reads)
+    c = native.Counter(0)
+    c.set_reads(chars, offs)
+    check_store(c, chars, offs, k, p, 31)
     c.close()
