@@ -97,7 +97,7 @@ def tune(counter: native.Counter, k: int, p: int, parts: int, n_kmers: int, cmin
     counter.set_p1_lists(0 if choice["p1_lists"] else 0xFFFFFFFF)
     counter.superkmers(k, p, parts)
     # count stage: sweep size
-    caps = (9216, 11264, 13312, 16384, 18432, 20480) if k <= 32 else (2304, 3072, 3840, 4224, 4608, 4992)
+    caps = (9216, 11264, 13312, 16384, 18432, 20480) if k <= 32 else (3072, 3840, 4608, 5376, 6144, 7168)
     best = None
     for cap in caps:
         counter.set_tuning(cap)

@@ -75,9 +75,8 @@ template <> struct KT<u128> {
         return mix(mix_in(h) ^ (uint32_t)(hi >> 32));
     }
 };
-// distinct keys a sweep is planned for: 80% of the slots where they are tried in groups of four, 70%
-// where one by one (a run of 64 full slots flags the sweep)
-template <typename K> constexpr float kFill = (sizeof(K) == 8 ? 0.80f : 0.70f) * (float)KT<K>::H;
+// distinct keys a sweep is planned for: 80% of the slots (a run of 64 full groups flags the sweep)
+template <typename K> constexpr float kFill = 0.80f * (float)KT<K>::H;
 
 // Hash slice of a key among n. Slice s of n is the union of the slices s * f ... s * f + f - 1 of n * f.
 __device__ __forceinline__ uint32_t slice_of(uint32_t h, uint32_t n) {
@@ -244,49 +243,138 @@ __device__ __forceinline__ void insert(uint64_t* tk, uint32_t* tc, const uint64_
                                        uint32_t w, uint32_t* ovf) {
     insert_rest<N>(tk, tc, key, h, insert_first<N>(tk, tc, key, h, valid, w), w, ovf);
 }
-// 128-bit keys: slot = {lo, hi}; hi == ~0 empty, ~0-1 busy (being published); keys have hi < 2^62.
-// The winner of the claim publishes in straight-line code before anyone waits, and a full fence keeps
-// the compiler from sinking the publish below the wait: a lane that waits on a slot claimed by a lane of
-// its own wave must never run first.
+// 128-bit keys (126 bits at most) as two words of 63, neither ever ~0: the table holds the lower halves in groups
+// of four, then the upper ones. A claim is a CAS of the lower half; the claimer writes the upper one next, and a
+// key that meets its own lower half reads the upper one: ~0 until it is written, when the key tries again. Keys
+// that differ in the lower half (the k-mer's last 31 bases), nearly all that share a group, never wait for each
+// other. A slot of both words, marked busy until both were there and tried one by one: 392 M 128-bit keys
+// 7.3 ms, now 5.8.
+// The claimer writes in straight-line code before any lane of its wave tries again, and a full fence keeps the
+// compiler from moving the write past the tries.
+__device__ __forceinline__ uint64_t half0(u128 key) { return (uint64_t)key & (~0ull >> 1); }
+__device__ __forceinline__ uint64_t half1(u128 key) { return (uint64_t)(key >> 63); }
+constexpr uint32_t kGroups128 = KT<u128>::H / 4u;
+__device__ __forceinline__ uint64_t load_half1(const uint64_t* ta, uint32_t s) {
+    return __hip_atomic_load(ta + KT<u128>::H + s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ __forceinline__ void store_half1(uint64_t* ta, uint32_t s, uint64_t v) {
+    __hip_atomic_store(ta + KT<u128>::H + s, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+template <int N>
+__device__ __forceinline__ uint32_t insert_first(u128* tk, uint32_t* tc, const u128* key, const uint32_t* h, uint32_t valid,
+                                                 uint32_t w) {
+    uint64_t* const ta = (uint64_t*)tk;
+    uint32_t g[N], at[N], pend = 0;
+    ulonglong2 q0[N], q1[N];
+#pragma unroll
+    for (int u = 0; u < N; u++) {
+        g[u] = 4u * place(h[u], kGroups128);
+        const ulonglong2* const gs = (const ulonglong2*)&ta[g[u]];
+        q0[u] = gs[0];
+        q1[u] = gs[1];
+    }
+#pragma unroll
+    for (int u = 0; u < N; u++) {
+        const uint32_t v = (valid >> u) & 1u;
+        const uint64_t ka = half0(key[u]);
+        uint32_t e;
+        uint32_t i = find(q0[u], q1[u], ka, e);
+        if (((i >> 2) & v) && e < 4u) {
+            const unsigned long long o = atomicCAS((unsigned long long*)&ta[g[u] + e], ~0ull, (unsigned long long)ka);
+            if (o == ~0ull) store_half1(ta, g[u] + e, half1(key[u]));
+            i = (o == ~0ull) | (o == ka) ? e : 4u;
+        }
+        at[u] = v ? i : 8u;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+    uint64_t kb[N];
+#pragma unroll
+    for (int u = 0; u < N; u++) kb[u] = load_half1(ta, g[u] + (at[u] & 3u));
+#pragma unroll
+    for (int u = 0; u < N; u++) {
+        const bool hit = at[u] < 4u && kb[u] == half1(key[u]);
+        if (hit) atomicAdd(&tc[g[u] + at[u]], w);
+        pend |= (uint32_t)(!hit && at[u] < 8u) << u;
+    }
+    return pend;
+}
+template <int N>
+__device__ __forceinline__ void insert_rest(u128* tk, uint32_t* tc, const u128* key, const uint32_t* h, uint32_t pend,
+                                            uint32_t w, uint32_t* ovf) {
+    if (!pend) return;
+    uint64_t* const ta = (uint64_t*)tk;
+    uint64_t ka = 0, kl = 0;
+    uint32_t gg = 0, from = 0;  // slots of the group before `from` hold the lower half with another upper one
+    auto take = [&]() {
+        const uint32_t u = (uint32_t)__builtin_ctz(pend);
+        uint32_t hh = 0;
+#pragma unroll
+        for (int j = 0; j < N; j++)
+            if (u == (uint32_t)j) { ka = half0(key[j]); kl = half1(key[j]); hh = h[j]; }
+        gg = place(hh, kGroups128);
+        from = 0;
+    };
+    take();
+#pragma unroll 1
+    for (int tries = 0, waits = 0;;) {
+        const ulonglong2* const gs = (const ulonglong2*)&ta[4u * gg];
+        const ulonglong2 x = gs[0], y = gs[1];
+        uint32_t e;
+        (void)find(x, y, ka, e);
+        uint32_t i = 4u;
+        if (y.y == ka && from <= 3u) i = 3u;
+        if (y.x == ka && from <= 2u) i = 2u;
+        if (x.y == ka && from <= 1u) i = 1u;
+        if (x.x == ka && from == 0u) i = 0u;
+        if (i == 4u && e < 4u) {
+            const unsigned long long o = atomicCAS((unsigned long long*)&ta[4u * gg + e], ~0ull, (unsigned long long)ka);
+            if (o == ~0ull) store_half1(ta, 4u * gg + e, kl);
+            i = (o == ~0ull) | (o == ka) ? e : 4u;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+        const uint64_t o = load_half1(ta, 4u * gg + (i & 3u));
+        if (i < 4u && o == kl) {
+            atomicAdd(&tc[4u * gg + i], w);
+            pend &= pend - 1u;
+            if (!pend) break;
+            take();
+            tries = waits = 0;
+        } else if (i < 4u && o == ~0ull) {
+            if (++waits > (1 << 16)) {  // reported as a failure, not retried
+                *ovf = 2u;
+                break;
+            }
+        } else {
+            if (i < 4u) {
+                from = i + 1u;
+            } else if (e == 4u) {
+                gg = gg + 1u == kGroups128 ? 0u : gg + 1u;
+                from = 0;
+            }
+            if (++tries == kProbes) {
+                *ovf = 1u;
+                break;
+            }
+        }
+    }
+}
 template <int N>
 __device__ __forceinline__ void insert(u128* tk, uint32_t* tc, const u128* key, const uint32_t* h, uint32_t valid,
                                        uint32_t w, uint32_t* ovf) {
-    constexpr uint32_t H = KT<u128>::H;
-#pragma unroll
-    for (int u = 0; u < N; u++) {
-        if (!((valid >> u) & 1u)) continue;
-        const uint64_t khi = (uint64_t)(key[u] >> 64), klo = (uint64_t)key[u];
-        uint32_t s = place(h[u], H);
-        bool done = false;
-        for (int probe = 0; probe < kProbes && !done; probe++) {
-            unsigned long long* lo_p = (unsigned long long*)&tk[s];
-            unsigned long long* hi_p = lo_p + 1;
-            uint64_t chi = __hip_atomic_load(hi_p, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP);
-            bool won = false;
-            if (chi == ~0ull) {
-                const unsigned long long old = atomicCAS(hi_p, ~0ull, ~0ull - 1);
-                won = (old == ~0ull);
-                chi = won ? khi : old;
-            }
-            if (won) {
-                __hip_atomic_store(lo_p, klo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                __hip_atomic_store(hi_p, khi, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
-            }
-            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-            int spin = 0;
-            while (chi == ~0ull - 1) {
-                if (++spin > (1 << 16)) { *ovf = 2u; return; }  // reported as a failure, not retried
-                chi = __hip_atomic_load(hi_p, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP);
-            }
-            if (chi == khi &&
-                (won || __hip_atomic_load(lo_p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) == klo)) {
-                atomicAdd(&tc[s], w);
-                done = true;
-            }
-            s = s + 1u == H ? 0u : s + 1u;
-        }
-        if (!done) *ovf = 1u;
-    }
+    insert_rest<N>(tk, tc, key, h, insert_first<N>(tk, tc, key, h, valid, w), w, ovf);
+}
+
+// Slot s of the table: its key (empty() if none), then empty again.
+__device__ __forceinline__ uint64_t take_slot(uint64_t* tk, uint32_t s) {
+    const uint64_t x = tk[s];
+    tk[s] = ~0ull;
+    return x;
+}
+__device__ __forceinline__ u128 take_slot(u128* tk, uint32_t s) {
+    uint64_t* const ta = (uint64_t*)tk;
+    const uint64_t x = ta[s], y = ta[KT<u128>::H + s];
+    ta[s] = ta[KT<u128>::H + s] = ~0ull;
+    return x == ~0ull ? KT<u128>::empty() : ((u128)y << 63) | x;
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -485,9 +573,8 @@ template <typename K> struct Slots {
 #pragma unroll
         for (int j = 0; j < SPT; j++) {
             const uint32_t s = threadIdx.x + (uint32_t)j * kItemThreads;
-            key[j] = tkeys[s];
+            key[j] = take_slot(tkeys, s);
             cnt[j] = tcnt[s];
-            tkeys[s] = KT<K>::empty();
             tcnt[s] = 0;
         }
 #pragma unroll
@@ -560,7 +647,7 @@ __device__ __forceinline__ uint64_t first_row(const CountArgs& a, uint32_t part,
 // Bound by LDS in the insert (random 32-byte reads, CAS and count atomics: a third of the time at three
 // quarters of its rate) and by VALU issue around it. 1.2 G k-mers at 30x (360 M distinct): 9.1 ms, where
 // expanding every k-mer took 6.5 and counting the keys 6.0; 188 M (k=25) 1.35 ms, before 1.2 + 0.85; 392 M
-// 128-bit keys 7.5 ms, before 5.3 + 7.0.
+// 128-bit keys 5.8 ms, before 5.3 + 7.0.
 template <typename K>
 __global__ __launch_bounds__(kItemThreads, 4) void k_count_units(CountArgs a) {
     constexpr int TC = kItemThreads, NW = TC / 64, WPT = (int)kStageW / TC;
@@ -735,12 +822,9 @@ __global__ __launch_bounds__(kItemThreads, 4) void k_count_units(CountArgs a) {
                         h[t] = KT<K>::hash(key[t]);
                         if (filt) valid &= ~((uint32_t)(slice_of(h[t], ns) != slice) << t);
                     }
-                    if constexpr (sizeof(K) == 8)
-                        pend |= insert_first<kBatch>(tkeys, tcnt, key + t0, h + t0, valid >> t0, mul) << t0;
-                    else
-                        insert<kBatch>(tkeys, tcnt, key + t0, h + t0, valid >> t0, mul, &sh_ovf);
+                    pend |= insert_first<kBatch>(tkeys, tcnt, key + t0, h + t0, valid >> t0, mul) << t0;
                 }
-                if constexpr (sizeof(K) == 8) insert_rest<(int)kPiece>(tkeys, tcnt, key, h, pend, mul, &sh_ovf);
+                insert_rest<(int)kPiece>(tkeys, tcnt, key, h, pend, mul, &sh_ovf);
             }
             if (sh_long)
                 for (uint32_t q = 0; q < n; q++) {

@@ -1,8 +1,8 @@
 """The count stage's units of work against the oracle, where its kernels change path: records longer
 than a chunk's piece map, its staged words or the grouping's word map (tandem repeats are one superkmer);
 partitions of more units than the small grouping kernel takes; equal records; runs of one k-mer; a
-read of exactly one k-mer. Both with the largest units expanded into keys and without. Whole numbers:
-equal."""
+read of exactly one k-mer; 128-bit keys that differ in one half. Both with the largest units expanded into
+keys and without. Whole numbers: equal."""
 import numpy as np
 import pytest
 
@@ -44,7 +44,24 @@ def _many_units():
     return synth.short_reads(g, 9, 9_000, 150, 0.01)
 
 
+def _same_halves(k):
+    """k-mers that end in the same 32 bases, 16 of each: many meet in one group of the 128-bit table."""
+    def make():
+        rng = np.random.default_rng(k)
+        reads = []
+        for _ in range(900):
+            tail = bytes(rng.choice(list(b"ACGT"), 32))
+            for v in range(16):
+                head = bytes(rng.choice(list(b"ACGT"), k - 34)) if k > 34 else b""
+                reads += [(head + bytes([b"ACGT"[v % 4], b"ACGT"[v // 4]]))[-(k - 32):] + tail] * (1 + v % 3)
+        return _csr([reads[i] for i in rng.permutation(len(reads))])
+    return make
+
+
 @pytest.mark.parametrize("make,k,p,parts,cap", [
+    (_same_halves(33), 33, 5, 1, 30_000),
+    (_same_halves(34), 34, 5, 1, 30_000),
+    (_same_halves(63), 63, 5, 2, 0),
     (_long_records, 31, 11, 3, 0),
     (_long_records, 55, 13, 3, 0),
     (_long_records, 21, 7, 1, 700),
@@ -53,7 +70,7 @@ def _many_units():
     (_many_units, 31, 11, 1, 256),   # about 2000 units in one partition, 128-bit keys below
     (_many_units, 55, 11, 1, 256),
     (lambda: _csr([b"ACGTTGCATTGACCATGGACTAGGACTCATG"]), 31, 11, 64, 0),
-], ids=["long31", "long55", "long21", "equal31", "equal63", "many31", "many55", "one"])
+], ids=["halves33", "halves34", "halves63", "long31", "long55", "long21", "equal31", "equal63", "many31", "many55", "one"])
 def test_units(make, k, p, parts, cap):
     from rapidgkc_amd import native
     chars, offs = make()
