@@ -32,16 +32,10 @@ constexpr uint32_t kMaxSlices = 1u << 20;
 constexpr int kProbes = 64;        // table probes a key may take
 constexpr uint32_t kPiece = 4;     // consecutive k-mers of a record that one thread takes
 constexpr int kBatch = 2;          // of them inserted together
-constexpr uint32_t kStageW = 4096; // 2-bit words of a chunk
-constexpr uint32_t kPieces = 4096; // pieces of a chunk
-constexpr uint32_t kSame = 2048;   // slots of the chunk's record set
-constexpr uint32_t kLongPieces = 64;  // a record of more pieces is not cut into the chunk's piece map
-static_assert(kStageW <= 4096 && kItemThreads <= 1024 && kLongPieces <= 64, "packed record and piece fields");
-static_assert(kStageW % kItemThreads == 0, "whole words per thread");
-
-// LDS table: 10240 x (8 + 4) or 6144 x (16 + 4) bytes, 120 KiB either way: with the staging areas one
-// workgroup of 16 waves takes a CU. (Two workgroups of 8 waves with half the table each were 4% slower on 1.2 G
-// k-mers: twice the sweeps, more units in several slices, fewer equal records found.)
+// LDS table: 8192 x (8 + 4) or 6144 x (16 + 4) bytes: with the staging areas one workgroup of 16 waves takes a
+// CU. 64-bit keys stage two records per thread, so that a unit is nearly always one chunk; with one record per thread
+// and 10240 slots most units were two, the second one half empty (count stage of 1.2 G k-mers: 12.2 ms, now 10.9). Two
+// workgroups of 8 waves with half the table each were 4% slower: twice the sweeps, fewer equal records found.
 //
 // Hash: a 32-bit multiply per key word, its high half rotated down before the next word joins, and the
 // high half folded into the low one at the end (two multiplies for 64-bit keys; a 64-bit multiply takes
@@ -59,7 +53,8 @@ __device__ __forceinline__ uint32_t place(uint32_t h, uint32_t n) { return __umu
 
 template <typename K> struct KT;
 template <> struct KT<uint64_t> {
-    static constexpr uint32_t H = 10240;
+    static constexpr uint32_t H = 8192;
+    static constexpr int R = 2;  // records of a chunk per thread
     static __device__ __forceinline__ uint64_t empty() { return ~0ull; }
     static __device__ __forceinline__ uint32_t hash(uint64_t x) {
         return mix((mix_in((uint32_t)x) ^ (uint32_t)(x >> 32)));
@@ -67,6 +62,7 @@ template <> struct KT<uint64_t> {
 };
 template <> struct KT<u128> {
     static constexpr uint32_t H = 6144;
+    static constexpr int R = 1;
     static __device__ __forceinline__ u128 empty() { return ~(u128)0; }
     static __device__ __forceinline__ uint32_t hash(u128 v) {
         const uint64_t lo = (uint64_t)v, hi = (uint64_t)(v >> 64);
@@ -77,6 +73,18 @@ template <> struct KT<u128> {
 };
 // distinct keys a sweep is planned for: 80% of the slots (a run of 64 full groups flags the sweep)
 template <typename K> constexpr float kFill = 0.80f * (float)KT<K>::H;
+
+// A chunk of records: at most kItemThreads * R of them, W words, P pieces; S slots of its record set. A record of
+// more than `Long` pieces is not cut into the piece map (record | piece << RecBits, 16 bits).
+template <typename K> struct Chunk {
+    static constexpr int R = KT<K>::R;
+    static constexpr uint32_t W = R == 2 ? 6144 : 4096, P = 4096 * R, S = 2048 * R;
+    static constexpr uint32_t RecBits = R == 2 ? 11 : 10, Long = 1u << (16 - RecBits);
+    static constexpr uint32_t WBits = 13, WMask = (1u << WBits) - 1u;  // of a record's info: first word | k-mers << WBits
+    static constexpr uint32_t MaxLong = W / (Long * kPiece / 16u);     // a long record has more words than this divides by
+    static_assert(W <= WMask && kItemThreads * R <= (1 << RecBits) && W % kItemThreads == 0, "packed fields, whole words per thread");
+    static_assert(0x3FFFFu < (1u << (32 - WBits)), "the k-mers of a record that its side descriptor holds");
+};
 
 // Hash slice of a key among n. Slice s of n is the union of the slices s * f ... s * f + f - 1 of n * f.
 __device__ __forceinline__ uint32_t slice_of(uint32_t h, uint32_t n) {
@@ -645,19 +653,22 @@ __device__ __forceinline__ uint64_t first_row(const CountArgs& a, uint32_t part,
 // the next chunk's counting. (With the loads of a sweep's first chunk and its row stores in line, staging
 // and row output took a third of the kernel.)
 // Bound by LDS in the insert (random 32-byte reads, CAS and count atomics: a third of the time at three
-// quarters of its rate) and by VALU issue around it. 1.2 G k-mers at 30x (360 M distinct): 9.1 ms, where
-// expanding every k-mer took 6.5 and counting the keys 6.0; 188 M (k=25) 1.35 ms, before 1.2 + 0.85; 392 M
-// 128-bit keys 5.8 ms, before 5.3 + 7.0.
+// quarters of its rate) and by VALU issue around it, half of the issue slots. 1.2 G k-mers at 30x (360 M
+// distinct): 8.2 ms, where expanding every k-mer took 6.5 and counting the keys 6.0; 188 M (k=25) 1.24 ms, before
+// 1.2 + 0.85; 392 M 128-bit keys 5.8 ms, before 5.3 + 7.0. The loads take a uniform base and a thread's offset: with an
+// address per load 27 registers went to scratch, 0.6 ms of the first.
 template <typename K>
 __global__ __launch_bounds__(kItemThreads, 4) void k_count_units(CountArgs a) {
-    constexpr int TC = kItemThreads, NW = TC / 64, WPT = (int)kStageW / TC;
+    using C = Chunk<K>;
+    constexpr int TC = kItemThreads, NW = TC / 64, R = C::R, WPT = (int)C::W / TC;
     __shared__ __align__(16) K tkeys[KT<K>::H];
     __shared__ uint32_t tcnt[KT<K>::H];
-    __shared__ uint32_t stw[kStageW + 8];
-    // a chunk's records: first word | k-mers << 12, how many equal ones; the hash set of the records, then
-    // the pieces (record | piece of it << 10)
-    __shared__ uint32_t rinfo[TC], rmul[TC];
-    __shared__ union { uint32_t same[kSame]; uint16_t pmap[kPieces]; } mp;
+    __shared__ uint32_t stw[C::W + 8];
+    // a chunk's records: first word | k-mers << WBits, how many equal ones; the hash set of the records, then
+    // the pieces; the long records
+    __shared__ uint32_t rinfo[TC * R], rmul[TC * R];
+    __shared__ union { uint32_t same[C::S]; uint16_t pmap[C::P]; } mp;
+    __shared__ uint16_t longs[C::MaxLong];
     __shared__ Cut stack[kStack];
     __shared__ uint32_t tmp2[2 * NW], wtot[NW];
     __shared__ unsigned long long sh_in;  // chunk: records << 20 | words
@@ -713,35 +724,56 @@ __global__ __launch_bounds__(kItemThreads, 4) void k_count_units(CountArgs a) {
         sh_ovf = 0;
     }
 
-    uint32_t dn, wn[WPT];  // the next chunk's descriptor and words of this thread
+    uint32_t dn[R], wn[WPT];  // the next chunk's descriptors and words of this thread
     auto load = [&](const UnitDesc& d, uint32_t c, uint32_t w) {
-        dn = c + threadIdx.x < d.n_rec ? a.desc[d.desc + c + threadIdx.x] : 0u;
+        const uint32_t* const pd = a.desc + d.desc + c;
+        const uint32_t* const pw = a.words + d.word + w;
+        const uint32_t ld = d.n_rec - c, lw = d.n_word - w;
+#pragma unroll
+        for (int j = 0; j < R; j++) {
+            const uint32_t i = threadIdx.x * R + (uint32_t)j;
+            dn[j] = i < ld ? pd[i] : 0u;
+        }
 #pragma unroll
         for (int u = 0; u < WPT; u++) {
-            const uint32_t i = w + threadIdx.x + (uint32_t)u * TC;
-            wn[u] = i < d.n_word ? a.words[d.word + i] : 0u;
+            const uint32_t i = threadIdx.x + (uint32_t)u * TC;
+            wn[u] = i < lw ? pw[i] : 0u;
         }
     };
-    uint32_t km, nw, np, exW;
-    bool in;
+    uint32_t n_in;  // this thread's records in the chunk
+    auto pieces = [](uint32_t km) __attribute__((always_inline)) { return (km + kPiece - 1u) / kPiece; };
     // stages the loaded chunk (records c ... of the unit); `publish` runs in thread 0 before its last barrier
     auto stage = [&](uint32_t c, auto&& publish) {
-        const bool has = c + threadIdx.x < ud.n_rec;
-        km = dn;
-        nw = has ? rec_words(km, k) : 0u;
-        np = (km + kPiece - 1u) / kPiece;
+        uint32_t nw[R], np[R], sw = 0, sp = 0;
+#pragma unroll
+        for (int j = 0; j < R; j++) {
+            nw[j] = c + threadIdx.x * R + (uint32_t)j < ud.n_rec ? rec_words(dn[j], k) : 0u;
+            np[j] = pieces(dn[j]);
+            sw += nw[j];
+            sp += np[j];
+        }
         if (threadIdx.x == 0) { sh_in = 0; sh_np = 0; sh_long = 0; }
-        uint32_t exP, totW, totP;
-        wg_exscan2_u32(nw, np, tmp2, exW, exP, totW, totP);
-        in = has && (exW + nw <= kStageW) && (exP + np <= kPieces);
-        const uint64_t bal = __ballot(in);
-        if (in && (bal >> lane) == 1ull)
-            atomicMax(&sh_in, ((unsigned long long)(threadIdx.x + 1u) << 20) | (exW + nw));
-        rinfo[threadIdx.x] = exW | (km << 12);
-        rmul[threadIdx.x] = 1u;
+        uint32_t exW, exP, totW, totP;
+        wg_exscan2_u32(sw, sp, tmp2, exW, exP, totW, totP);
+        n_in = 0;
+        uint32_t end = 0;
+#pragma unroll
+        for (int j = 0; j < R; j++) {
+            const uint32_t r = threadIdx.x * R + (uint32_t)j;
+            rinfo[r] = (exW & C::WMask) | (dn[j] << C::WBits);
+            rmul[r] = 1u;
+            exW += nw[j];
+            exP += np[j];
+            if (c + r < ud.n_rec && exW <= C::W && exP <= C::P) {
+                n_in = (uint32_t)j + 1u;
+                end = exW;
+            }
+        }
+        const uint64_t bal = __ballot(n_in != 0);
+        if (n_in && (bal >> lane) == 1ull) atomicMax(&sh_in, ((unsigned long long)(threadIdx.x * R + n_in) << 20) | end);
 #pragma unroll
         for (int u = 0; u < WPT; u++) stw[threadIdx.x + (uint32_t)u * TC] = wn[u];
-        for (uint32_t i = threadIdx.x; i < kSame; i += TC) same[i] = 0;
+        for (uint32_t i = threadIdx.x; i < C::S; i += TC) same[i] = 0;
         if (threadIdx.x == 0) publish();
         __syncthreads();
     };
@@ -752,66 +784,103 @@ __global__ __launch_bounds__(kItemThreads, 4) void k_count_units(CountArgs a) {
         const uint32_t n = (uint32_t)(sh_in >> 20), slice = cur.slice, ns = cur.n;
         const bool filt = ns > 1;
         // n == 0: the first record alone exceeds the staging area
-        const uint32_t c1 = c0 + max(n, 1u), w1 = w0 + (n ? (uint32_t)sh_in & 0xFFFFFu : rec_words(rinfo[0] >> 12, k));
+        const uint32_t c1 = c0 + max(n, 1u), w1 = w0 + (n ? (uint32_t)sh_in & 0xFFFFFu : rec_words(rinfo[0] >> C::WBits, k));
         const bool last = c1 >= ud.n_rec;
         // the next chunk's loads: this sweep's, the unit's next sweep's, or the next unit's
         const bool again = sh_nstack > 0 || sh_first < sh_q0;
         if (!last) load(ud, c1, w1);
         else if (again) load(ud, 0, 0);
         else load(unit(ahead), 0, 0);
-        auto single = [&](const uint32_t* bw, uint32_t g) {
+        auto single = [&](const uint32_t* bw, uint32_t g, uint32_t mul) {
             Window<K> w;
             w.load(bw, g);
             const K key = w.key(0, k, m);
             const uint32_t h = KT<K>::hash(key);
-            insert<1>(tkeys, tcnt, &key, &h, !filt || slice_of(h, ns) == slice ? 1u : 0u, 1u, &sh_ovf);
+            insert<1>(tkeys, tcnt, &key, &h, !filt || slice_of(h, ns) == slice ? 1u : 0u, mul, &sh_ovf);
         };
         if (n == 0) {
-            const uint32_t km1 = rinfo[0] >> 12;  // its k-mers straight from HBM
-            for (uint32_t x = threadIdx.x; x < km1 && !sh_ovf; x += TC) single(a.words + ud.word + w0, x);
+            const uint32_t km1 = rinfo[0] >> C::WBits;  // its k-mers straight from HBM
+            for (uint32_t x = threadIdx.x; x < km1 && !sh_ovf; x += TC) single(a.words + ud.word + w0, x, 1u);
         } else {
             // Equal records (reads of one place without errors give equal records but for their ends: two in
             // five at 30x and 1% errors) are counted once, with their number: a hash set of the chunk's
             // records, compared word by word.
-            bool uniq = in;
-            if (in && nw <= 16u) {
-                uint32_t h = km;
-                for (uint32_t i = 0; i < nw; i++) h = mix_in(h) ^ stw[exW + i];
-                h = mix(h);
-                const uint32_t entry = (threadIdx.x + 1u) | (h << 16);
+            // Words in blocks of four (staged words follow a record's last, or slack), the first one kept.
+            uint32_t uniq = (1u << n_in) - 1u;
+            uint32_t x[R][4], hash[R];
+#pragma unroll
+            for (int j = 0; j < R; j++) {
+                const uint32_t info = rinfo[threadIdx.x * R + j], w0r = info & C::WMask;
+                const uint32_t nw = (uint32_t)j < n_in ? rec_words(info >> C::WBits, k) : 0u;
+                uint32_t h = info >> C::WBits;
+                auto block = [&](uint32_t i, uint32_t* v) {
+#pragma unroll
+                    for (uint32_t t = 0; t < 4; t++) v[t] = i + t < nw ? stw[w0r + i + t] : 0u;
+#pragma unroll
+                    for (int t = 0; t < 4; t++) h = mix_in(h) ^ v[t];
+                };
+                block(0, x[j]);
+                if (nw <= 16u) {
+                    uint32_t y[4];
+#pragma unroll 1
+                    for (uint32_t i = 4; i < nw; i += 4) block(i, y);
+                }
+                hash[j] = mix(h);
+            }
+#pragma unroll
+            for (int j = 0; j < R; j++) {
+                const uint32_t rec = threadIdx.x * R + (uint32_t)j, info = rinfo[rec], w0r = info & C::WMask;
+                const uint32_t nw = rec_words(info >> C::WBits, k), h = hash[j];
+                if ((uint32_t)j >= n_in || nw > 16u) continue;
+                const uint32_t entry = (rec + 1u) | (h << 16);
+#pragma unroll 1
                 for (uint32_t s = h >> 16, tries = 0; tries < 8u; s++, tries++) {
-                    const uint32_t o = atomicCAS(&same[s % kSame], 0u, entry);
+                    const uint32_t o = atomicCAS(&same[s % C::S], 0u, entry);
                     if (o == 0) break;
                     if ((o ^ entry) >> 16) continue;
                     const uint32_t other = (o & 0xFFFFu) - 1u, oi = rinfo[other];
-                    if (oi >> 12 != km) continue;
+                    if ((oi ^ info) >> C::WBits) continue;
+                    const uint32_t* const q = stw + (oi & C::WMask);
                     uint32_t diff = 0;
-                    for (uint32_t i = 0; i < nw; i++) diff |= stw[(oi & 0xFFFu) + i] ^ stw[exW + i];
+#pragma unroll
+                    for (uint32_t t = 0; t < 4; t++) diff |= t < nw ? q[t] ^ x[j][t] : 0u;
+#pragma unroll 1
+                    for (uint32_t i = 4; i < nw; i += 4)
+#pragma unroll
+                        for (uint32_t t = 0; t < 4; t++) diff |= i + t < nw ? q[i + t] ^ stw[w0r + i + t] : 0u;
                     if (diff) continue;
                     atomicAdd(&rmul[other], 1u);
-                    uniq = false;
+                    uniq &= ~(1u << j);
                     break;
                 }
             }
             __syncthreads();
-            // pieces of the records that remain; a record of more than kLongPieces apart
+            // pieces of the records that remain; a record of more than `Long` apart
             {
-                const bool big = np > kLongPieces;
-                const uint32_t mine = uniq && !big ? np : 0u;
-                const uint32_t incl = wave_incl_scan_u32(mine);
+                uint32_t mine[R], sum = 0;
+#pragma unroll
+                for (int j = 0; j < R; j++) {
+                    const uint32_t np = pieces(rinfo[threadIdx.x * R + j] >> C::WBits);
+                    const bool counts = (uniq >> j) & 1u;
+                    mine[j] = counts && np <= C::Long ? np : 0u;
+                    if (counts && np > C::Long) longs[atomicAdd(&sh_long, 1u)] = (uint16_t)(threadIdx.x * R + j);
+                    sum += mine[j];
+                }
+                const uint32_t incl = wave_incl_scan_u32(sum);
                 uint32_t wb = 0;
                 if (lane == 63u) wb = atomicAdd(&sh_np, incl);
-                uint32_t e = (uint32_t)__builtin_amdgcn_readlane((int)wb, 63) + incl - mine;
-                for (uint32_t i = 0; i < mine; i++) pmap[e++] = (uint16_t)(threadIdx.x | (i << 10));
-                if (uniq && big) sh_long = 1;
+                uint32_t e = (uint32_t)__builtin_amdgcn_readlane((int)wb, 63) + incl - sum;
+#pragma unroll
+                for (int j = 0; j < R; j++)
+                    for (uint32_t i = 0; i < mine[j]; i++) pmap[e++] = (uint16_t)((threadIdx.x * R + j) | (i << C::RecBits));
             }
             __syncthreads();
             const uint32_t npc = sh_np;
             for (uint32_t x = threadIdx.x; x < npc; x += TC) {
-                const uint32_t e = pmap[x], rec = e & 1023u, j = e >> 10, info = rinfo[rec], mul = rmul[rec];
-                const uint32_t c = min(kPiece, (info >> 12) - kPiece * j);
+                const uint32_t e = pmap[x], rec = e & ((1u << C::RecBits) - 1u), j = e >> C::RecBits, info = rinfo[rec];
+                const uint32_t mul = rmul[rec], c = min(kPiece, (info >> C::WBits) - kPiece * j);
                 Window<K> w;
-                w.load(stw, (info & 0xFFFu) * 16u + kPiece * j);
+                w.load(stw, (info & C::WMask) * 16u + kPiece * j);
                 K key[kPiece];
                 uint32_t h[kPiece], valid = (1u << c) - 1u, pend = 0;
 #pragma unroll
@@ -826,12 +895,10 @@ __global__ __launch_bounds__(kItemThreads, 4) void k_count_units(CountArgs a) {
                 }
                 insert_rest<(int)kPiece>(tkeys, tcnt, key, h, pend, mul, &sh_ovf);
             }
-            if (sh_long)
-                for (uint32_t q = 0; q < n; q++) {
-                    const uint32_t info = rinfo[q], kq = info >> 12;
-                    if ((kq + kPiece - 1u) / kPiece > kLongPieces)
-                        for (uint32_t x = threadIdx.x; x < kq; x += TC) single(stw, (info & 0xFFFu) * 16u + x);
-                }
+            for (uint32_t q = 0; q < sh_long; q++) {
+                const uint32_t info = rinfo[longs[q]], kq = info >> C::WBits, mul = rmul[longs[q]];
+                for (uint32_t x = threadIdx.x; x < kq; x += TC) single(stw, (info & C::WMask) * 16u + x, mul);
+            }
         }
         __syncthreads();
         const uint32_t ovf = sh_ovf;

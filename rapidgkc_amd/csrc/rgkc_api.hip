@@ -385,10 +385,10 @@ int do_phase1(rgkc_ctx* c, int k, int p, int parts, uint32_t* mm_hist = nullptr)
     return 0;
 }
 
-// K-mer instances planned per count sweep: for 64-bit keys what fills the table (8192 of 10240 slots) at
-// one distinct key in two instances, for 128-bit ones (4915 of 6144) at four in five. Read sets are mostly below:
-// their larger units then take fewer sweeps than planned. The count stage over 13000, 15000, 16384, 18432: 12.2,
-// 12.0, 12.1, 12.0 ms (1.2 G k-mers at 30x), 2.10, 2.05, 1.96, 2.00 (188 M, k=25); over 4608, 5400, 6144, 7200:
+// K-mer instances planned per count sweep: for 64-bit keys what fills the table (6553 of 8192 slots) at two
+// distinct keys in five instances, for 128-bit ones (4915 of 6144) at four in five. Read sets are mostly below:
+// their larger units then take fewer sweeps than planned. The count stage over 13000, 15000, 16384, 18432: 11.1,
+// 11.0, 10.9, 11.0 ms (1.2 G k-mers at 30x), 1.75, 1.74, 1.63, 1.64 (188 M, k=25); over 4608, 5400, 6144, 7200:
 // 7.58, 7.32, 7.22, 7.47 ms (392 M, k=55 at 10x), 0.54, 0.55, 0.55, 0.55 (12 M, k=55).
 uint32_t unit_cap(const rgkc_ctx* c) {
     const uint32_t cap = c->inst_cap ? c->inst_cap : (c->k <= 32 ? 16384u : 6144u);

@@ -58,7 +58,17 @@ def _same_halves(k):
     return make
 
 
+def _one_kmer_records(n, k):
+    """n records of one k-mer: a chunk of the unit to its last record, one less and one more."""
+    def make():
+        rng = np.random.default_rng(n)
+        return _csr([bytes(rng.choice(list(b"ACGT"), k)) for _ in range(n - 3)] + [b"ACGTTGCA" * 8 + b"A" * k] * 3)
+    return make
+
+
 @pytest.mark.parametrize("make,k,p,parts,cap", [
+    *[(_one_kmer_records(n, 31), 31, 9, 1, 0) for n in (2047, 2048, 2049, 4097)],
+    *[(_one_kmer_records(n, 63), 63, 9, 1, 0) for n in (1023, 1024, 1025)],
     (_same_halves(33), 33, 5, 1, 30_000),
     (_same_halves(34), 34, 5, 1, 30_000),
     (_same_halves(63), 63, 5, 2, 0),
@@ -70,7 +80,7 @@ def _same_halves(k):
     (_many_units, 31, 11, 1, 256),   # about 2000 units in one partition, 128-bit keys below
     (_many_units, 55, 11, 1, 256),
     (lambda: _csr([b"ACGTTGCATTGACCATGGACTAGGACTCATG"]), 31, 11, 64, 0),
-], ids=["halves33", "halves34", "halves63", "long31", "long55", "long21", "equal31", "equal63", "many31", "many55", "one"])
+], ids=[*[f"chunk31_{n}" for n in (2047, 2048, 2049, 4097)], *[f"chunk63_{n}" for n in (1023, 1024, 1025)], "halves33", "halves34", "halves63", "long31", "long55", "long21", "equal31", "equal63", "many31", "many55", "one"])
 def test_units(make, k, p, parts, cap):
     from rapidgkc_amd import native
     chars, offs = make()
