@@ -198,7 +198,7 @@ __device__ __forceinline__ uint32_t insert_first(uint64_t* tk, uint32_t* tc, con
         uint32_t i = find(q0[u], q1[u], key[u], e);
         if (((i >> 2) & v) && e < 4u) {
             const unsigned long long o = atomicCAS((unsigned long long*)&tk[4u * g[u] + e], ~0ull, (unsigned long long)key[u]);
-            i = (o == ~0ull) | (o == key[u]) ? e : 4u;
+            i = ((o == ~0ull) | (o == key[u])) ? e : 4u;
         }
         pend |= ((i >> 2) & v) << u;
         if (v & ~(i >> 2)) atomicAdd(&tc[4u * g[u] + i], w);
@@ -229,7 +229,7 @@ __device__ __forceinline__ void insert_rest(uint64_t* tk, uint32_t* tc, const ui
         uint32_t i = find(gs[0], gs[1], kk, e);
         if ((i >> 2) && e < 4u) {
             const unsigned long long o = atomicCAS((unsigned long long*)&tk[4u * gg + e], ~0ull, (unsigned long long)kk);
-            i = (o == ~0ull) | (o == kk) ? e : 4u;
+            i = ((o == ~0ull) | (o == kk)) ? e : 4u;
         }
         if (i < 4u) {
             atomicAdd(&tc[4u * gg + i], w);
@@ -290,7 +290,7 @@ __device__ __forceinline__ uint32_t insert_first(u128* tk, uint32_t* tc, const u
         if (((i >> 2) & v) && e < 4u) {
             const unsigned long long o = atomicCAS((unsigned long long*)&ta[g[u] + e], ~0ull, (unsigned long long)ka);
             if (o == ~0ull) store_half1(ta, g[u] + e, half1(key[u]));
-            i = (o == ~0ull) | (o == ka) ? e : 4u;
+            i = ((o == ~0ull) | (o == ka)) ? e : 4u;
         }
         at[u] = v ? i : 8u;
     }
@@ -337,7 +337,7 @@ __device__ __forceinline__ void insert_rest(u128* tk, uint32_t* tc, const u128* 
         if (i == 4u && e < 4u) {
             const unsigned long long o = atomicCAS((unsigned long long*)&ta[4u * gg + e], ~0ull, (unsigned long long)ka);
             if (o == ~0ull) store_half1(ta, 4u * gg + e, kl);
-            i = (o == ~0ull) | (o == ka) ? e : 4u;
+            i = ((o == ~0ull) | (o == ka)) ? e : 4u;
         }
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
         const uint64_t o = load_half1(ta, 4u * gg + (i & 3u));

@@ -409,7 +409,7 @@ __global__ __launch_bounds__(T, 3) void k_p1_count(P1Args a) {
         const uint32_t r = __builtin_amdgcn_alignbit(nc, np, 2u * jj) | (uint32_t)__builtin_amdgcn_sbfe((int)bad_r, 2u * jj + 1u, 1u);
         return (f < r ? f : r) & top;
     };
-    const FastDivU32 pdiv = FastDivU32::make((uint32_t)a.parts);
+    const FastDivU32 pdiv = a.pdiv;
     uint64_t* const lst = a.skm_list ? a.skm_list + (size_t)wg * a.skm_cap : nullptr;
     bool done = !has, open = false;
     uint32_t qn = 0;
@@ -651,7 +651,7 @@ __device__ void emit_tile(const P1Args& a, uint32_t wg, uint64_t n_seg, EmitLds<
     const uint64_t s = seg_lo + threadIdx.x;
     const int k = a.k;
     const uint32_t parts = (uint32_t)a.parts;
-    const FastDivU32 pdiv = FastDivU32::make(parts);
+    const FastDivU32 pdiv = a.pdiv;
     BaseSrc src;
     if (STREAM) {
         for (int i = threadIdx.x; i < a.parts; i += T) { L.hb[i] = 0; L.hr[i] = 0; L.hk[i] = 0; }
@@ -844,7 +844,7 @@ __global__ __launch_bounds__(TE) void k_p1_emit_list(P1Args a) {
     }
     const int k = a.k;
     const uint32_t parts = (uint32_t)a.parts;
-    const FastDivU32 pdiv = FastDivU32::make(parts);
+    const FastDivU32 pdiv = a.pdiv;
     const size_t stride = (size_t)a.n_wg + 1;
     for (uint32_t i = threadIdx.x; i < parts; i += TE) {
         uint64_t bo, ro;

@@ -314,7 +314,7 @@ int do_phase1(rgkc_ctx* c, int k, int p, int parts, uint32_t* mm_hist = nullptr)
     a.seg_first = c->seg_first.as<uint32_t>();
     a.n_seg = nseg_total;
     a.n_bases = c->n_bases;
-    a.k = k; a.p = p; a.parts = parts;
+    a.k = k; a.p = p; a.parts = parts; a.pdiv = FastDivU32::make((uint32_t)parts);
     a.h_bytes = c->hist.as<uint32_t>();
     a.h_recs = a.h_bytes + hwords;
     a.h_kmers = a.h_recs + hwords;
@@ -1623,7 +1623,7 @@ int rgkc_superkmers_sized(rgkc_ctx* c, int k, int p, int parts, const uint64_t* 
     a.seg_read = c->seg_read.as<uint32_t>();
     a.seg_first = c->seg_first.as<uint32_t>();
     a.n_bases = c->n_bases;
-    a.k = k; a.p = p; a.parts = parts;
+    a.k = k; a.p = p; a.parts = parts; a.pdiv = FastDivU32::make((uint32_t)parts);
     region_args(c, a);
     a.n_seg_dev = c->seg_off.as<uint64_t>() + n;
     if (c->list_cap != 0xFFFFFFFFu) {
@@ -1717,7 +1717,7 @@ int rgkc_stream_begin(rgkc_ctx* c, int k, int p, int parts, uint64_t max_reads, 
     a.seg_read = c->seg_read.as<uint32_t>();
     a.seg_first = c->seg_first.as<uint32_t>();
     a.n_bases = max_bases;
-    a.k = k; a.p = p; a.parts = parts;
+    a.k = k; a.p = p; a.parts = parts; a.pdiv = FastDivU32::make((uint32_t)parts);
     region_args(c, a);
     a.n_seg_dev = c->hdr.as<uint64_t>() + 2;
     if (c->list_cap != 0xFFFFFFFFu) {

@@ -114,9 +114,15 @@ __device__ __forceinline__ uint32_t load_u16(const uint8_t* p) {
 // The 16 bases from base t0 on of a record (cpu_funcs.cpp:219-250 layout: base t at digit (bm3 + t) % 3
 // of byte (bm3 + t) / 3, digit 0 in bits 5:4) as one LSB-first 2-bit word. Six bytes hold them; zeros
 // follow the record's last base, L - 1.
-__device__ __forceinline__ uint32_t record_word(const uint8_t* rec, uint32_t bm3, uint32_t t0, uint32_t L) {
-    const uint32_t b = bm3 + t0, j = b / 3u, r = b - 3u * j;
-    const uint32_t lo = load_u32(rec + j), hi = load_u16(rec + j + 4);
+struct RecordBytes {
+    uint32_t lo, hi;
+};
+__device__ __forceinline__ RecordBytes record_bytes(const uint8_t* rec, uint32_t bm3, uint32_t t0) {
+    const uint8_t* const p = rec + (bm3 + t0) / 3u;
+    return {load_u32(p), load_u16(p + 4)};
+}
+__device__ __forceinline__ uint32_t record_word(RecordBytes rb, uint32_t bm3, uint32_t t0, uint32_t L) {
+    const uint32_t lo = rb.lo, hi = rb.hi, r = (bm3 + t0) % 3u;
     // the three digits of every byte reversed in place, then the bytes' six bits packed
     auto rev = [](uint32_t x) { return ((x & 0x03030303u) << 4) | (x & 0x0C0C0C0Cu) | ((x >> 4) & 0x03030303u); };
     auto pack = [](uint32_t x) {
@@ -128,20 +134,34 @@ __device__ __forceinline__ uint32_t record_word(const uint8_t* rec, uint32_t bm3
     return left < 16u ? w & ((1u << (2u * left)) - 1u) : w;
 }
 
+__device__ __forceinline__ uint32_t record_word(const uint8_t* rec, uint32_t bm3, uint32_t t0, uint32_t L) {
+    return record_word(record_bytes(rec, bm3, t0), bm3, t0, L);
+}
+
+// What the waves before this one sum to and what all do, from each wave's sum in lane w of a row of 16:
+// uniform values.
+__device__ __forceinline__ uint32_t wave_sums(uint32_t x, uint32_t wave, uint32_t& total) {
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xF, 0xF, false);
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xF, 0xF, false);
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xF, 0xF, false);
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xF, 0xF, false);
+    total = (uint32_t)__builtin_amdgcn_readlane((int)x, 15);
+    return wave ? (uint32_t)__builtin_amdgcn_readlane((int)x, (int)wave - 1) : 0u;
+}
+
 // Workgroup-wide exclusive scan of one uint32 per thread (blockDim.x <= 1024, multiple of 64).
 // `tmp` needs blockDim.x/64 + 1 words of LDS. Returns the exclusive prefix; *total gets the sum.
 // Ends with a barrier, so `tmp` may be reused at once.
+// The waves' sums are read by 16 lanes at once and scanned there: read one after another they were
+// up to 16 LDS latencies, a quarter of the grouping kernel's chunk.
 __device__ __forceinline__ uint32_t wg_exscan_u32(uint32_t v, uint32_t* tmp, uint32_t* total) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    const uint32_t lane = threadIdx.x & 63u, nw = blockDim.x >> 6;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const uint32_t x = wave_incl_scan_u32(v);
-    if (lane == 63) tmp[wave] = x;
+    if (lane == 63u) tmp[wave] = x;
     __syncthreads();
-    uint32_t pre = 0, tot = 0;
-    for (int w = 0; w < nw; w++) {
-        const uint32_t t = tmp[w];
-        pre += (w < wave) ? t : 0u;
-        tot += t;
-    }
+    uint32_t tot;
+    const uint32_t pre = wave_sums(lane < nw ? tmp[lane] : 0u, wave, tot);
     *total = tot;
     __syncthreads();
     return pre + x - v;
@@ -151,20 +171,13 @@ __device__ __forceinline__ uint32_t wg_exscan_u32(uint32_t v, uint32_t* tmp, uin
 // 2 * blockDim.x/64 words of LDS. Ends with a barrier.
 __device__ __forceinline__ void wg_exscan2_u32(uint32_t v0, uint32_t v1, uint32_t* tmp, uint32_t& e0, uint32_t& e1,
                                                uint32_t& t0, uint32_t& t1) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    const uint32_t lane = threadIdx.x & 63u, nw = blockDim.x >> 6;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const uint32_t x0 = wave_incl_scan_u32(v0), x1 = wave_incl_scan_u32(v1);
-    if (lane == 63) { tmp[2 * wave] = x0; tmp[2 * wave + 1] = x1; }
+    if (lane == 63u) { tmp[2 * wave] = x0; tmp[2 * wave + 1] = x1; }
     __syncthreads();
-    uint32_t p0 = 0, p1 = 0, s0 = 0, s1 = 0;
-    for (int w = 0; w < nw; w++) {
-        const uint32_t a = tmp[2 * w], b = tmp[2 * w + 1];
-        if (w < wave) { p0 += a; p1 += b; }
-        s0 += a;
-        s1 += b;
-    }
-    e0 = p0 + x0 - v0;
-    e1 = p1 + x1 - v1;
-    t0 = s0;
-    t1 = s1;
+    const uint32_t a = lane < nw ? tmp[2 * lane] : 0u, b = lane < nw ? tmp[2 * lane + 1] : 0u;
+    e0 = wave_sums(a, wave, t0) + x0 - v0;
+    e1 = wave_sums(b, wave, t1) + x1 - v1;
     __syncthreads();
 }

@@ -3,6 +3,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "rgkc_device.h"
+
 namespace rgkc {
 
 constexpr int kScanTile = 4096;      // elements per workgroup tile in the device scans
@@ -62,6 +64,7 @@ struct P1Args {
     uint64_t n_seg;
     uint64_t n_bases;  // bases in the batch (bases2 holds n_bases/16 + 2 words)
     int k, p, parts;
+    FastDivU32 pdiv;  // division by parts
     // count mode: per-(partition, workgroup) histograms, partition-major [parts][n_wg]
     uint32_t* h_bytes;
     uint32_t* h_recs;
