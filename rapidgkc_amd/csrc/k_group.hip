@@ -237,36 +237,43 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan(CountArgs a) {
 // (a scan over the units) and reserved in the units' runs (one packed atomic per unit, whose latency
 // passes under the next step); a map from each of the chunk's words to its record; then lane i writes
 // the chunk's i-th descriptor and word in unit order, so neighbouring lanes write neighbouring places.
-// A word is made from six bytes of the store read where they lie (neighbouring lanes share lines).
+// The chunk's store bytes are staged in LDS, their loads in flight while the places are worked out; a word is
+// made from six of them.
 // Before: records grouped by 1024 fixed groups, a thread re-encoding a whole record byte by byte out of
-// staged LDS bytes; 3.6 ms for 114 M records (1.65 GB of store), now 2.35 ms.
+// staged LDS bytes; 3.6 ms for 114 M records (1.65 GB of store). With the bytes read where they lie, two
+// unaligned loads a word: 2.35 ms, three fifths of it for the words (the chunks of a CU exceed its L1); now
+// 1.5 ms.
+constexpr uint32_t kGroupBytes = 17280;  // staged store bytes of a chunk: three workgroups of the small size share a CU
 template <int TG, int CH, int WC, int UM>  // threads, records and words per chunk, units
 __global__ __launch_bounds__(TG) void k_group(CountArgs a) {
     static_assert(CH < 4096 && WC < (1 << 16) && UM <= 4096 && UM % TG == 0 && CH % TG == 0, "packed fields");
     constexpr int RPT = CH / TG, UPT = UM / TG;
-    __shared__ uint16_t umap[kSubIds];
+    constexpr uint32_t SB = kGroupBytes;
+    constexpr int SPT = (int)((SB / 16u + TG - 1u) / TG);
+    static_assert(SB % 16u == 0 && SB < (1u << 15) && WC * 16 < (1 << 17), "packed fields");
+    __shared__ __align__(4) uint16_t umap[kSubIds];
     __shared__ uint32_t ucnt[UM];           // words << 12 | records of the chunk per unit, then their starts
     __shared__ uint32_t gw[UM], gr[UM];     // unit's run minus its start in the chunk: words, records
     __shared__ uint16_t wrec[WC];           // record (its place in the chunk) of each word
-    __shared__ uint32_t rbyte[CH], rkm[CH]; // per place: store byte from the chunk's first, k-mers
+    __shared__ __align__(16) uint32_t stb[SB / 4 + 4]; // the chunk's store bytes, from a 16-byte boundary on
+    __shared__ uint32_t rpos[CH];           // per place: first byte in stb | k-mers << 15
     __shared__ uint32_t rinfo[CH];          // per place: first word << 16 | unit << 2 | start % 3
     __shared__ uint32_t tmp[2 * (TG / 64) + 1];
     __shared__ unsigned long long sh_cut;   // records << 40 | store bytes of the chunk
-    // segments of a bucket go to one XCD (workgroup b runs on XCD b % 8): the runs that its chunks append
-    // to then meet in one L2
+    // Segments of a bucket go to one XCD (workgroup b runs on XCD b % 8): the runs that its chunks append
+    // to then meet in one L2. Which one moves on by one every eight buckets: buckets of one residue mod 8
+    // are of one minimizer residue and differ in size as a class (the largest held 1.25 times its share of 1.2 G
+    // k-mers, which the other XCDs waited for).
     const uint32_t per_xcd = (a.n_buckets + 7) / 8 * a.n_segs;
-    const uint32_t xcd = blockIdx.x % 8u, ix = blockIdx.x / 8u;
-    const uint32_t bucket = (ix / a.n_segs) * 8u + xcd, sg = ix % a.n_segs;
+    const uint32_t ix = blockIdx.x / 8u, row = ix / a.n_segs;
+    const uint32_t bucket = row * 8u + ((blockIdx.x + row) & 7u), sg = ix % a.n_segs;
     if (ix >= per_xcd || bucket >= a.n_buckets) return;
+    // all that the first chunk needs is loaded before anything is waited for or checked
     const uint64_t byte0 = a.b_byte[bucket];
     const uint64_t nbytes = (a.b_byte_end ? a.b_byte_end[bucket] : a.b_byte[bucket + 1]) - byte0;
     const uint64_t* const sgb = a.seg_bytes + (size_t)bucket * (a.n_segs + 1);
-    if (sgb[a.n_segs] != nbytes) {  // the records' sizes do not add up to the store
-        if (threadIdx.x == 0) raise_err(a.err, RGKC_ERR_BAD_STORE);
-        return;
-    }
+    const uint64_t seg0 = sgb[sg], segs_end = sgb[a.n_segs];
     const uint32_t n_units = a.n_units[bucket];
-    if (n_units > (uint32_t)UM || (UM > kSmallUnits && n_units <= (uint32_t)kSmallUnits)) return;  // the other size
     const uint64_t rec0 = a.b_rec[bucket];
     const SegRange sr = group_seg(bucket_nrec(a, bucket), sg, a.n_segs);
     const uint32_t wcap = (uint32_t)min(a.b_word[bucket + 1] - a.b_word[bucket], (uint64_t)0xFFFFFFFFu);
@@ -274,20 +281,38 @@ __global__ __launch_bounds__(TG) void k_group(CountArgs a) {
     uint32_t* const words = a.words + a.b_word[bucket];
     uint32_t* const desc = a.desc + (rec0 - a.rec_base);
     unsigned long long* const ucur = a.unit_cur + (size_t)bucket * kSubIds;
-    const uint8_t* store = a.store + byte0 + sgb[sg];
-    if (sr.lo >= sr.hi) return;
-    {
-        const uint32_t* const src = (const uint32_t*)(a.sub_unit + (size_t)bucket * kSubIds);
-        for (int i = threadIdx.x; i < kSubIds / 2; i += TG) ((uint32_t*)umap)[i] = src[i];
-    }
-    uint32_t nsd[RPT];
+    const uint8_t* store = a.store + byte0 + seg0;
+    const uint8_t* const store_end = a.store + byte0 + nbytes;
+    uint4 sv[SPT];
+    auto load_bytes = [&](const uint8_t* from) {
+        const uint8_t* const p = from - ((uintptr_t)from & 15u);
+#pragma unroll
+        for (int j = 0; j < SPT; j++) {
+            const uint32_t o = 16u * (threadIdx.x + (uint32_t)j * TG);
+            sv[j] = o < SB && p + o < store_end ? *(const uint4*)(p + o) : make_uint4(0, 0, 0, 0);  // (the store has slack past its end)
+        }
+    };
+    uint32_t nsd[RPT], um[kSubIds / 2 / TG];
 #pragma unroll
     for (int j = 0; j < RPT; j++) {
         const uint32_t r = sr.lo + threadIdx.x * RPT + j;
         nsd[j] = r < sr.hi ? a.side[rec0 + r] : 0u;
     }
+#pragma unroll
+    for (int j = 0; j < kSubIds / 2 / TG; j++)
+        um[j] = ((const uint32_t*)(a.sub_unit + (size_t)bucket * kSubIds))[threadIdx.x + j * TG];
+    load_bytes(store);
+    if (segs_end != nbytes) {  // the records' sizes do not add up to the store
+        if (threadIdx.x == 0) raise_err(a.err, RGKC_ERR_BAD_STORE);
+        return;
+    }
+    if (n_units > (uint32_t)UM || (UM > kSmallUnits && n_units <= (uint32_t)kSmallUnits)) return;  // the other size
+    if (sr.lo >= sr.hi) return;
+#pragma unroll
+    for (int j = 0; j < kSubIds / 2 / TG; j++) ((uint32_t*)umap)[threadIdx.x + j * TG] = um[j];
     for (uint32_t c0 = sr.lo; c0 < sr.hi;) {
         uint32_t sd[RPT], nb[RPT], nw[RPT], old[RPT], accb = 0, accw = 0;
+        const uint32_t lead = (uint32_t)((uintptr_t)store & 15u);
 #pragma unroll
         for (int j = 0; j < RPT; j++) {
             const uint32_t r = c0 + threadIdx.x * RPT + j;
@@ -302,8 +327,8 @@ __global__ __launch_bounds__(TG) void k_group(CountArgs a) {
         if (threadIdx.x == 0) sh_cut = 0;
         uint32_t exb, exw, totb, totw;
         wg_exscan2_u32(accb, accw, tmp, exb, exw, totb, totw);  // ends with a barrier
-        // the chunk: the leading records whose words fit the map (at least one record: a longer one is
-        // a chunk of its own)
+        // the chunk: the leading records whose words fit the map and whose bytes are staged (at least one
+        // record: a longer one is a chunk of its own)
         uint32_t off[RPT], mine = 0;
         {
             uint32_t eb = exb, ew = exw;
@@ -313,7 +338,7 @@ __global__ __launch_bounds__(TG) void k_group(CountArgs a) {
                 eb += nb[j];
                 ew += nw[j];
                 const uint32_t r = c0 + threadIdx.x * RPT + j;
-                if (r < sr.hi && (ew <= (uint32_t)WC || r == c0)) {
+                if (r < sr.hi && ((ew <= (uint32_t)WC && lead + eb <= SB) || r == c0)) {
                     mine = j + 1;
                     old[j] = atomicAdd(&ucnt[umap[side_sub(sd[j])]], (min(nw[j], (uint32_t)WC) << 12) | 1u);
                 }
@@ -358,6 +383,15 @@ __global__ __launch_bounds__(TG) void k_group(CountArgs a) {
                 run[j] = atomicAdd(&ucur[u], ((unsigned long long)(uc[j] >> 12) << 32) | (uc[j] & 0xFFFu));
             ue += uc[j];
         }
+#pragma unroll
+        for (int j = 0; j < SPT; j++) {
+            const uint32_t o = 4u * (threadIdx.x + (uint32_t)j * TG);
+            if (o < SB / 4u) *(uint4*)&stb[o] = sv[j];
+        }
+        // the next chunk's descriptors are there by now; its bytes, before this chunk's stores
+#pragma unroll
+        for (int j = 0; j < RPT; j++) asm volatile("" : "+v"(nsd[j]));
+        load_bytes(store + cbytes);
         __syncthreads();
         if (alone) {
             // one record: all threads make its words
@@ -366,14 +400,14 @@ __global__ __launch_bounds__(TG) void k_group(CountArgs a) {
                 const unsigned long long o = atomicAdd(&ucur[u], ((unsigned long long)nw[0] << 32) | 1ull);
                 gw[0] = (uint32_t)(o >> 32);
                 gr[0] = (uint32_t)o;
-                rkm[0] = side_kmers(sd[0]);
+                rpos[0] = side_kmers(sd[0]);
                 rinfo[0] = side_bm3(sd[0]);
             }
             __syncthreads();
-            const uint32_t w0 = gw[0], n1 = rec_words(rkm[0], k);
-            if (threadIdx.x == 0) desc[gr[0]] = rkm[0];
+            const uint32_t w0 = gw[0], km1 = rpos[0], n1 = rec_words(km1, k);
+            if (threadIdx.x == 0) desc[gr[0]] = km1;
             for (uint32_t i = threadIdx.x; i < n1; i += TG)
-                if (w0 + i < wcap) words[w0 + i] = record_word(store, rinfo[0], 16u * i, rkm[0] + (uint32_t)k - 1u);
+                if (w0 + i < wcap) words[w0 + i] = record_word(store, rinfo[0], 16u * i, km1 + (uint32_t)k - 1u);
         } else {
             // per place: the record's store byte, k-mers and words
 #pragma unroll
@@ -382,8 +416,7 @@ __global__ __launch_bounds__(TG) void k_group(CountArgs a) {
                 const uint32_t u = umap[side_sub(sd[j])];
                 const uint32_t st = ucnt[u];
                 const uint32_t pl = (st & 0xFFFu) + (old[j] & 0xFFFu), w0 = (st >> 12) + (old[j] >> 12);
-                rbyte[pl] = off[j];
-                rkm[pl] = side_kmers(sd[j]);
+                rpos[pl] = (lead + off[j]) | (side_kmers(sd[j]) << 15);
                 rinfo[pl] = (w0 << 16) | (u << 2) | side_bm3(sd[j]);
                 for (uint32_t i = 0; i < nw[j]; i++) wrec[w0 + i] = (uint16_t)pl;
             }
@@ -396,11 +429,15 @@ __global__ __launch_bounds__(TG) void k_group(CountArgs a) {
                 }
             __syncthreads();
             const uint32_t nwc = utot >> 12;
-            for (uint32_t i = threadIdx.x; i < m; i += TG) desc[gr[(rinfo[i] >> 2) & 0xFFFu] + i] = rkm[i];
+            for (uint32_t i = threadIdx.x; i < m; i += TG) desc[gr[(rinfo[i] >> 2) & 0xFFFu] + i] = rpos[i] >> 15;
             for (uint32_t i = threadIdx.x; i < nwc; i += TG) {
                 const uint32_t pl = wrec[i], inf = rinfo[pl];
                 const uint32_t at = gw[(inf >> 2) & 0xFFFu] + i;
-                const uint32_t v = record_word(store + rbyte[pl], inf & 3u, 16u * (i - (inf >> 16)), rkm[pl] + (uint32_t)k - 1u);
+                const uint32_t ps = rpos[pl], bm3 = inf & 3u, t0 = 16u * (i - (inf >> 16));
+                const uint32_t o = (ps & 0x7FFFu) + (bm3 + t0) / 3u, *const q = stb + (o >> 2);
+                const uint32_t x0 = q[0], x1 = q[1], x2 = q[2];
+                const RecordBytes rb = {__builtin_amdgcn_alignbyte(x1, x0, o & 3u), __builtin_amdgcn_alignbyte(x2, x1, o & 3u) & 0xFFFFu};
+                const uint32_t v = record_word(rb, bm3, t0, (ps >> 15) + (uint32_t)k - 1u);
                 if (at < wcap) words[at] = v;
             }
         }
