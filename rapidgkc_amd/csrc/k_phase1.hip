@@ -583,8 +583,9 @@ __device__ __forceinline__ uint32_t record_bytes4(uint32_t x) {
 // Write record bytes [0, nb) of superkmer [b, e) of a read into dst (cpu_funcs.cpp:238-244).
 // Record byte x is packed-read byte m = b/3 + x: 11|b0|b1|b2 for a full group, the read's tail
 // byte (len%3)<<6 with its bases high, or 0 when len%3 == 0 (only the record's last byte can be that
-// one); then the first and last indicators are patched. Four bytes at a time, from one word pair: a byte
-// at a time took 43 instructions a byte, and the list emit was bound by them.
+// one); then the first and last indicators are patched. Four bytes are made at a time, from one word pair (a byte
+// at a time took 43 instructions a byte), and leave in stores of 16 and 8 bytes; the last 8 overlap those
+// before, so that most records take two or three.
 __device__ __forceinline__ void write_record(const BaseSrc& src, uint64_t R0, uint32_t len, uint32_t b, uint32_t e, int k,
                                              uint32_t nb, uint8_t* dst) {
     const uint32_t m0 = b / 3u;
@@ -592,25 +593,36 @@ __device__ __forceinline__ void write_record(const BaseSrc& src, uint64_t R0, ui
     const uint32_t first_ind = (3u - (b - 3u * m0)) << 6, last_ind = ((e - 1u + (uint32_t)k) % 3u) << 6;
     const int32_t rem = (int32_t)(len - 3u * (m0 + nb - 1u));  // of the read's bases from the last byte's first on
     const uint32_t last_mask = rem >= 3 ? 0x3Fu : rem == 2 ? 0x3Cu : rem == 1 ? 0x30u : 0u;
-    auto bytes = [&](auto word, uint32_t p) {  // p: the record's first base, relative to word(0)
-        uint32_t x = 0;
-        for (;; x += 4u, p += 12u) {
-            uint32_t v = record_bytes4(__builtin_amdgcn_alignbit(word((p >> 4) + 1u), word(p >> 4), 2u * (p & 15u)));
-            if (x == 0) v = (v & ~0xC0u) | first_ind;
-            if (x + 4u < nb) {
-                __builtin_memcpy(dst + x, &v, 4);
-                continue;
+    auto bytes = [&](auto word, uint32_t p0) {  // p0: the record's first base, relative to word(0)
+        auto four = [&](uint32_t x) __attribute__((always_inline)) {
+            const uint32_t p = p0 + 3u * x;
+            const uint32_t v = record_bytes4(__builtin_amdgcn_alignbit(word((p >> 4) + 1u), word(p >> 4), 2u * (p & 15u)));
+            return x == 0 ? (v & ~0xC0u) | first_ind : v;
+        };
+        auto ends = [&](uint32_t v) __attribute__((always_inline)) {  // the top byte of v is the record's last
+            return (v & 0xFFFFFFu) | ((((v >> 24) & last_mask) | last_ind) << 24);
+        };
+        if (nb >= 8u) {
+            uint32_t x = 0;
+            for (; nb - x > 16u; x += 16u) {
+                const uint32_t v[4] = {four(x), four(x + 4u), four(x + 8u), four(x + 12u)};
+                __builtin_memcpy(dst + x, v, 16);
             }
-            // the last one to four bytes, the record's last byte patched
-            const uint32_t n = nb - x, sh = 8u * (n - 1u);
-            v = (v & ((1u << sh) - 1u)) | (((((v >> sh) & last_mask) | last_ind)) << sh);
-            if (n == 4u) {
-                __builtin_memcpy(dst + x, &v, 4);
-            } else {
-                if (n & 2u) { const uint16_t h = (uint16_t)v; __builtin_memcpy(dst + x, &h, 2); v >>= 16; }
-                if (n & 1u) dst[x + (n & 2u)] = (uint8_t)v;
+            if (nb - x > 8u) {
+                const uint32_t v[2] = {four(x), four(x + 4u)};
+                __builtin_memcpy(dst + x, v, 8);
             }
-            break;
+            const uint32_t v[2] = {four(nb - 8u), ends(four(nb - 4u))};
+            __builtin_memcpy(dst + (nb - 8u), v, 8);
+        } else if (nb >= 4u) {
+            const uint32_t v = four(0);
+            if (nb > 4u) __builtin_memcpy(dst, &v, 4);
+            const uint32_t e = ends(four(nb - 4u));
+            __builtin_memcpy(dst + (nb - 4u), &e, 4);
+        } else {
+            const uint32_t sh = 8u * (nb - 1u), v = four(0);
+            for (uint32_t x = 0; x + 1u < nb; x++) dst[x] = (uint8_t)(v >> (8u * x));
+            dst[nb - 1u] = (uint8_t)(((v >> sh) & last_mask) | last_ind);
         }
     };
     // a record whose words are all staged is read from LDS (its first byte can begin up to two bases, and
@@ -810,7 +822,8 @@ __global__ __launch_bounds__(T) void k_p1_emit(P1Args a) {
 // A tile's loads (its entries, run starts, segments) all start before anything waits, and two threads
 // per segment take the entries: with one, entries loaded in each pass from HBM and the records written a
 // byte at a time, the kernel took 3.5 ms for 114 M records (1.65 GB of store, 0.46 GB of side words) on
-// 12 waves a CU; written four bytes at a time 2.9, and so 2.4.
+// 12 waves a CU; so 2.4, and with two or three stores a record instead of five or six 1.9. Bound by those
+// stores' lines in L2: 8 or 32 waves a CU instead of 16 take 2.3 ms.
 constexpr uint32_t kListStageW = 2560;  // staged 2-bit words per tile (the rest read from HBM)
 constexpr uint32_t kReorderMax = 3840;  // list entries a tile of 256 segments can put in store order (more: list order)
 
@@ -1038,14 +1051,14 @@ hipError_t launch_batch_prep(const uint8_t* reads, const uint64_t* offs, uint64_
 
 // The list emit over all tiles, with partition tables sized for a.parts: two workgroups of 512 threads share
 // a CU with tables for 512 partitions (75 KB of LDS), one of 1024 takes it with the full ones; tiles of 128
-// segments (49 KB) three of 256.
+// segments (49 KB) three of 512.
 static hipError_t launch_list(const P1Args& a, bool big, hipStream_t s) {
     const bool small = a.parts <= 512;
     if (!big) {
         if (small) hipLaunchKernelGGL((k_p1_emit_list<256, 512, 512>), dim3(a.n_wg), dim3(512), 0, s, a);
         else hipLaunchKernelGGL((k_p1_emit_list<256, 1024, kMaxParts>), dim3(a.n_wg), dim3(1024), 0, s, a);
     } else {
-        if (small) hipLaunchKernelGGL((k_p1_emit_list<128, 256, 512>), dim3(a.n_wg), dim3(256), 0, s, a);
+        if (small) hipLaunchKernelGGL((k_p1_emit_list<128, 512, 512>), dim3(a.n_wg), dim3(512), 0, s, a);
         else hipLaunchKernelGGL((k_p1_emit_list<128, 512, kMaxParts>), dim3(a.n_wg), dim3(512), 0, s, a);
     }
     return hipGetLastError();
