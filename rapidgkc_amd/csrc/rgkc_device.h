@@ -18,13 +18,18 @@ enum : uint32_t {
 
 __device__ __forceinline__ void raise_err(uint32_t* err, uint32_t bit) { atomicOr(err, bit); }
 
-// 2-bit code of an ASCII base: A/a/N/n -> 0, C/c -> 1, G/g -> 2, T/t -> 3, anything else -> 0
-// (cpu_funcs.cpp:20-53 maps N to A; other bytes are outside the reference's contract).
-__device__ __forceinline__ uint32_t base_code(uint32_t c) {
-    const uint32_t u = c & 0xDFu;  // upper-case
-    const uint32_t v = ((u >> 1) ^ (u >> 2)) & 3u;
-    const bool ok = (u == 'A') | (u == 'C') | (u == 'G') | (u == 'T');
-    return ok ? v : 0u;
+// 2-bit codes of four ASCII bases (byte i's at bits 2i): A/a/N/n -> 0, C/c -> 1, G/g -> 2, T/t -> 3, anything
+// else -> 0 (cpu_funcs.cpp:20-53 maps N to A; other bytes are outside the reference's contract). All four bytes
+// at once: the two bits that tell A, C, G and T apart, looked up as the letter they stand for, and
+// cleared in bytes that are another one.
+__device__ __forceinline__ uint32_t base_codes4(uint32_t c) {
+    const uint32_t u = c & 0xDFDFDFDFu;  // upper-case
+    const uint32_t v = ((u >> 1) ^ (u >> 2)) & 0x03030303u;
+    const uint32_t diff = u ^ __builtin_amdgcn_perm(0u, 0x54474341u, v);  // "ACGT"[v], byte by byte
+    const uint32_t bad = (((diff & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | diff) & 0x80808080u;
+    uint32_t x = v & ~((bad >> 7) | (bad >> 6));
+    x |= x >> 6;
+    return (x & 0xFu) | ((x >> 12) & 0xF0u);
 }
 
 // minimizer_filter.h:19-20
