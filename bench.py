@@ -114,7 +114,7 @@ def summarize(wl, N, ms_per_step, per):
     stage = {k: float(np.mean([s[k] for _, s in per])) for k in STAGES}
     cs_ms = count_ms + stage["plan_ms"] + stage["expand_ms"]
     return st, stage, {"bound": "hbm", "achieved": alg_bytes / (count_ms * 1e-3) / 1e9, "peak": PEAK_HBM / 1e9,
-                       "unit": "GB/s", "frac": alg_bytes / (count_ms * 1e-3) / PEAK_HBM, "kernel": "k_count_items",
+                       "unit": "GB/s", "frac": alg_bytes / (count_ms * 1e-3) / PEAK_HBM, "kernel": "k_count_units",
                        "alg_bytes_per_launch": alg_bytes, "kernel_ms": count_ms, "count_stage_ms": cs_ms,
                        "count_stage_frac": alg_bytes / (cs_ms * 1e-3) / PEAK_HBM}
 
