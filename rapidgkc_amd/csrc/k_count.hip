@@ -31,7 +31,6 @@ constexpr uint32_t kMaxCut = 8;    // slices an overflowing sweep is cut into, a
 constexpr uint32_t kMaxSlices = 1u << 20;
 constexpr int kProbes = 64;        // table probes a key may take
 constexpr uint32_t kPiece = 4;     // consecutive k-mers of a record that one thread takes
-constexpr int kBatch = 2;          // of them inserted together
 // LDS table: 8192 x (8 + 4) or 6144 x (16 + 4) bytes: with the staging areas one workgroup of 16 waves takes a
 // CU. 64-bit keys stage two records per thread, so that a unit is nearly always one chunk; with one record per thread
 // and 10240 slots most units were two, the second one half empty (count stage of 1.2 G k-mers: 12.2 ms, now 10.9). Two
@@ -256,7 +255,7 @@ __device__ __forceinline__ void insert(uint64_t* tk, uint32_t* tc, const uint64_
 // key that meets its own lower half reads the upper one: ~0 until it is written, when the key tries again. Keys
 // that differ in the lower half (the k-mer's last 31 bases), nearly all that share a group, never wait for each
 // other. A slot of both words, marked busy until both were there and tried one by one: 392 M 128-bit keys
-// 7.3 ms, now 5.8.
+// 7.3 ms, so 5.8.
 // The claimer writes in straight-line code before any lane of its wave tries again, and a full fence keeps the
 // compiler from moving the write past the tries.
 __device__ __forceinline__ uint64_t half0(u128 key) { return (uint64_t)key & (~0ull >> 1); }
@@ -654,8 +653,8 @@ __device__ __forceinline__ uint64_t first_row(const CountArgs& a, uint32_t part,
 // and row output took a third of the kernel.)
 // Bound by LDS in the insert (random 32-byte reads, CAS and count atomics: a third of the time at three
 // quarters of its rate) and by VALU issue around it, half of the issue slots. 1.2 G k-mers at 30x (360 M
-// distinct): 8.2 ms, where expanding every k-mer took 6.5 and counting the keys 6.0; 188 M (k=25) 1.24 ms, before
-// 1.2 + 0.85; 392 M 128-bit keys 5.8 ms, before 5.3 + 7.0. The loads take a uniform base and a thread's offset: with an
+// distinct): 7.85 ms, where expanding every k-mer took 6.5 and counting the keys 6.0; 188 M (k=25) 1.14 ms, before
+// 1.2 + 0.85; 392 M 128-bit keys 5.55 ms, before 5.3 + 7.0. The loads take a uniform base and a thread's offset: with an
 // address per load 27 registers went to scratch, 0.6 ms of the first.
 template <typename K>
 __global__ __launch_bounds__(kItemThreads, 4) void k_count_units(CountArgs a) {
@@ -884,14 +883,12 @@ __global__ __launch_bounds__(kItemThreads, 4) void k_count_units(CountArgs a) {
                 K key[kPiece];
                 uint32_t h[kPiece], valid = (1u << c) - 1u, pend = 0;
 #pragma unroll
-                for (int t0 = 0; t0 < (int)kPiece; t0 += kBatch) {
-#pragma unroll
-                    for (int t = t0; t < t0 + kBatch; t++) {
-                        key[t] = w.key(t, k, m);
-                        h[t] = KT<K>::hash(key[t]);
-                        if (filt) valid &= ~((uint32_t)(slice_of(h[t], ns) != slice) << t);
-                    }
-                    pend |= insert_first<kBatch>(tkeys, tcnt, key + t0, h + t0, valid >> t0, mul) << t0;
+                for (int t = 0; t < (int)kPiece; t++) {
+                    key[t] = w.key(t, k, m);
+                    h[t] = KT<K>::hash(key[t]);
+                    if (filt) valid &= ~((uint32_t)(slice_of(h[t], ns) != slice) << t);
+                    // one at a time: two or four together read no slot sooner (16 waves do) and take 1 and 4% longer
+                    pend |= insert_first<1>(tkeys, tcnt, key + t, h + t, valid >> t, mul) << t;
                 }
                 insert_rest<(int)kPiece>(tkeys, tcnt, key, h, pend, mul, &sh_ovf);
             }
