@@ -631,8 +631,8 @@ __device__ __forceinline__ bool cut_sweep(const CountArgs& a, uint32_t ovf, Cut 
     for (uint32_t j = 0; j < f; j++) stack[n_stack++] = Cut{c.slice * f + j, c.n * f};
     return true;
 }
-// Row reservation of a sweep (thread 0): the rows its partition had before, and its first row from them
-// (apart, so that the atomic's latency can pass in between).
+// Row reservation of a sweep (thread 0): the rows its partition had before, and its first row from them, or ~0 (and
+// an error) if they don't fit its region (apart, so that the atomic's latency can pass in between).
 __device__ __forceinline__ uint64_t reserve_rows(const CountArgs& a, uint32_t part, uint32_t kept, uint32_t nd) {
     uint64_t rows = 0;
     if (kept) rows = atomicAdd(&a.row_cursor[part], (unsigned long long)kept);
@@ -640,9 +640,10 @@ __device__ __forceinline__ uint64_t reserve_rows(const CountArgs& a, uint32_t pa
     return rows;
 }
 __device__ __forceinline__ uint64_t first_row(const CountArgs& a, uint32_t part, uint64_t rows, uint32_t kept) {
-    const uint64_t row = a.row_base[part] + rows;
-    if (row + kept > a.row_end[part]) raise_err(a.err, RGKC_ERR_ROW_OVERFLOW);
-    return row;
+    const uint64_t base = a.row_base[part], end = a.row_end[part];
+    if (base + rows + kept <= end) return base + rows;
+    raise_err(a.err, RGKC_ERR_ROW_OVERFLOW);
+    return ~0ull;
 }
 
 // Units, from their records: chunk after chunk of up to kItemThreads records. A chunk is staged (record
@@ -653,8 +654,8 @@ __device__ __forceinline__ uint64_t first_row(const CountArgs& a, uint32_t part,
 // and row output took a third of the kernel.)
 // Bound by LDS in the insert (random 32-byte reads, CAS and count atomics: a third of the time at three
 // quarters of its rate) and by VALU issue around it, half of the issue slots. 1.2 G k-mers at 30x (360 M
-// distinct): 7.85 ms, where expanding every k-mer took 6.5 and counting the keys 6.0; 188 M (k=25) 1.14 ms, before
-// 1.2 + 0.85; 392 M 128-bit keys 5.55 ms, before 5.3 + 7.0. The loads take a uniform base and a thread's offset: with an
+// distinct): 7.7 ms, where expanding every k-mer took 6.5 and counting the keys 6.0; 188 M (k=25) 1.14 ms, before
+// 1.2 + 0.85; 392 M 128-bit keys 5.4 ms, before 5.3 + 7.0. The loads take a uniform base and a thread's offset: with an
 // address per load 27 registers went to scratch, 0.6 ms of the first.
 template <typename K>
 __global__ __launch_bounds__(kItemThreads, 4) void k_count_units(CountArgs a) {
@@ -672,7 +673,7 @@ __global__ __launch_bounds__(kItemThreads, 4) void k_count_units(CountArgs a) {
     __shared__ uint32_t tmp2[2 * NW], wtot[NW];
     __shared__ unsigned long long sh_in;  // chunk: records << 20 | words
     __shared__ uint64_t sh_row_base;
-    __shared__ uint32_t sh_ovf, sh_np, sh_long, sh_nstack, sh_first, sh_q0, sh_next;
+    __shared__ uint32_t sh_ovf, sh_np, sh_long, sh_nstack, sh_first, sh_q0, sh_next, sh_next_q;
     __shared__ Cut cur;
     uint32_t* const same = mp.same;
     uint16_t* const pmap = mp.pmap;
@@ -686,7 +687,7 @@ __global__ __launch_bounds__(kItemThreads, 4) void k_count_units(CountArgs a) {
     // the workgroup's sweep, retry and distinct totals, added to the global counters once at the end;
     // instances and distinct keys of its sweeps are added to the shared totals every few sweeps
     unsigned long long n_sweeps = 0, n_retries = 0, n_distinct = 0, seen_i = 0, seen_d = 0;
-    unsigned long long est_i = 0, est_d = 0;  // the shared totals, read one unit ahead by thread 0
+    unsigned long long est_i = 0, est_d = 0;  // the shared totals, read one unit ahead by the last wave
     for (uint32_t i = threadIdx.x; i < KT<K>::H; i += TC) { tkeys[i] = KT<K>::empty(); tcnt[i] = 0; }
 
     // descriptors: lane i of every wave loads word i one unit ahead, and the fields are wave-uniform
@@ -705,7 +706,9 @@ __global__ __launch_bounds__(kItemThreads, 4) void k_count_units(CountArgs a) {
     };
     UnitDesc ud = unit(fetch(it));
     uint32_t ahead = fetch(it + G);
-    // initial hash slices of a unit (thread 0): what its distinct keys should take by the ratio seen so far
+    // Initial hash slices of a unit: what its distinct keys should take by the ratio seen so far. The next unit's are
+    // worked out by the last wave, which has the fewest records, while the others look for equal ones (at the sweep's
+    // end by thread 0 they took 6% of the kernel).
     auto slices = [&](uint32_t inst) {
         const float ratio = est_i > 4ull * a.unit_cap ? (float)est_d / (float)est_i : kFill<K> / (float)a.unit_cap;
         uint32_t q = (uint32_t)ceilf(1.1f * (float)inst * fminf(ratio, 1.0f) / kFill<K>);
@@ -715,6 +718,7 @@ __global__ __launch_bounds__(kItemThreads, 4) void k_count_units(CountArgs a) {
         est_d = __hip_atomic_load(&a.plan_n[kPlanSeenDistinct], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         return q;
     };
+    bool planned = false;  // the next unit's slices are in sh_next_q
     if (threadIdx.x == 0) {
         sh_nstack = 0;
         sh_q0 = slices(ud.inst);
@@ -790,6 +794,11 @@ __global__ __launch_bounds__(kItemThreads, 4) void k_count_units(CountArgs a) {
         if (!last) load(ud, c1, w1);
         else if (again) load(ud, 0, 0);
         else load(unit(ahead), 0, 0);
+        if (!planned && wave == (uint32_t)NW - 1u) {
+            const uint32_t q = slices((uint32_t)__builtin_amdgcn_readlane((int)ahead, 1));
+            if (lane == 0) sh_next_q = q;
+        }
+        planned = true;
         auto single = [&](const uint32_t* bw, uint32_t g, uint32_t mul) {
             Window<K> w;
             w.load(bw, g);
@@ -942,7 +951,7 @@ __global__ __launch_bounds__(kItemThreads, 4) void k_count_units(CountArgs a) {
             } else {
                 sh_next = 1;
                 if (it + G < it_end) {
-                    sh_q0 = slices((uint32_t)__builtin_amdgcn_readlane((int)ahead, 1));
+                    sh_q0 = sh_next_q;
                     sh_first = 1;
                     cur = Cut{0, sh_q0};
                 }
@@ -957,18 +966,19 @@ __global__ __launch_bounds__(kItemThreads, 4) void k_count_units(CountArgs a) {
             if (it >= it_end) {
                 if (threadIdx.x == 0 && !ovf) sh_row_base = first_row(a, part, row0, kept);
                 __syncthreads();
-                if (!ovf && sh_row_base + kept <= a.row_end[part]) sl.store(a, sh_row_base + before);
+                if (!ovf && sh_row_base != ~0ull) sl.store(a, sh_row_base + before);
                 break;
             }
             ud = unit(ahead);
             ahead = fetch(it + G);
+            planned = false;
         }
         if (reload) load(ud, 0, 0);
         c0 = w0 = 0;
         stage(0, [&] {
             if (!ovf) sh_row_base = first_row(a, part, row0, kept);
         });
-        if (!ovf && sh_row_base + kept <= a.row_end[part]) sl.store(a, sh_row_base + before);
+        if (!ovf && sh_row_base != ~0ull) sl.store(a, sh_row_base + before);
     }
     if (threadIdx.x == 0) {
         if (n_sweeps) atomicAdd(&a.stats[0], n_sweeps);
@@ -1048,7 +1058,7 @@ __global__ __launch_bounds__(kItemThreads, 4) void k_count_keys(CountArgs a) {
                 }
             }
             __syncthreads();
-            if (!ovf && sh_row_base + kept <= a.row_end[kd.part]) sl.store(a, sh_row_base + before);
+            if (!ovf && sh_row_base != ~0ull) sl.store(a, sh_row_base + before);
         }
     }
     if (threadIdx.x == 0) {
