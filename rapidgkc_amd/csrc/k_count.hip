@@ -33,7 +33,7 @@ constexpr int kProbes = 64;        // table probes a key may take
 constexpr uint32_t kPiece = 4;     // consecutive k-mers of a record that one thread takes
 // LDS table: 8192 x (8 + 4) or 6144 x (16 + 4) bytes: with the staging areas one workgroup of 16 waves takes a
 // CU. 64-bit keys stage two records per thread, so that a unit is nearly always one chunk; with one record per thread
-// and 10240 slots most units were two, the second one half empty (count stage of 1.2 G k-mers: 12.2 ms, now 10.9). Two
+// and 10240 slots most units were two, the second one half empty (count kernel of 1.2 G k-mers: 9.2 ms, so 8.15). Two
 // workgroups of 8 waves with half the table each were 4% slower: twice the sweeps, fewer equal records found.
 //
 // Hash: a 32-bit multiply per key word, its high half rotated down before the next word joins, and the

@@ -387,9 +387,9 @@ int do_phase1(rgkc_ctx* c, int k, int p, int parts, uint32_t* mm_hist = nullptr)
 
 // K-mer instances planned per count sweep: for 64-bit keys what fills the table (6553 of 8192 slots) at two
 // distinct keys in five instances, for 128-bit ones (4915 of 6144) at four in five. Read sets are mostly below:
-// their larger units then take fewer sweeps than planned. The count stage over 13000, 15000, 16384, 18432: 11.1,
-// 11.0, 10.9, 11.0 ms (1.2 G k-mers at 30x), 1.75, 1.74, 1.63, 1.64 (188 M, k=25); over 4608, 5400, 6144, 7200:
-// 7.58, 7.32, 7.22, 7.47 ms (392 M, k=55 at 10x), 0.54, 0.55, 0.55, 0.55 (12 M, k=55).
+// their larger units then take fewer sweeps than planned. The count stage over 13000, 15000, 16384, 18432: 9.90,
+// 9.74, 9.67, 9.93 ms (1.2 G k-mers at 30x), 1.61, 1.61, 1.51, 1.55 (188 M, k=25); over 4608, 5400, 6144, 7200:
+// 6.89, 6.65, 6.59, 6.83 ms (392 M, k=55 at 10x), 0.50, 0.52, 0.51, 0.52 (12 M, k=55).
 uint32_t unit_cap(const rgkc_ctx* c) {
     const uint32_t cap = c->inst_cap ? c->inst_cap : (c->k <= 32 ? 16384u : 6144u);
     return std::min<uint32_t>(std::max<uint32_t>(cap, 256u), 1u << 19);
