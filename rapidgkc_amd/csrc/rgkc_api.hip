@@ -53,6 +53,8 @@ static __device__ __align__(256) uint8_t scratch[kNoAllocBytes];
 // allocation on a context's first copy (a 4 MiB pair made a first k=55 table of 20 MB slower than
 // 128 separate copies); 1 MiB keeps the copy at the host's copying rate.
 constexpr size_t kTableChunk = 1u << 20;
+// Rows a partition, from which the runtime's copies into mapped memory are no slower than the gather.
+constexpr uint64_t kLongRun = 1u << 23;
 
 constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
@@ -1328,9 +1330,55 @@ int rgkc_count_host_store(rgkc_ctx* c, const uint8_t* store, const uint64_t* par
     return 0;
 }
 
-// The partitions' rows leave the device as one dense table: chunks of it are gathered straight into
-// two pinned buffers by turns, and the host copies one chunk to the caller while the device fills the
-// other. A copy per partition and array (1024 of them for 512 partitions) cost 11-12 us each.
+// Where a copy's destination lies.
+enum class Dst { kHost, kMapped, kOther };
+// kMapped: memory that this device's kernels write at *view (pinned host memory, or the device's own), first
+// to last byte, aligned for their stores; kHost: memory only the host writes; kOther: what the runtime's copies reach.
+static Dst destination(const rgkc_ctx* c, void* p, uint64_t bytes, size_t align, uint8_t** view) {
+    hipPointerAttribute_t a{}, z{};
+    if (hipPointerGetAttributes(&a, p) != hipSuccess || hipPointerGetAttributes(&z, (uint8_t*)p + bytes - 1) != hipSuccess) {
+        (void)hipGetLastError();
+        return Dst::kHost;
+    }
+    if (a.type == hipMemoryTypeUnregistered && z.type == hipMemoryTypeUnregistered) return Dst::kHost;
+    const bool own = a.type == hipMemoryTypeDevice && a.device == c->device && z.device == a.device && a.devicePointer == p;
+    const bool mapped = a.type == z.type && (own || a.type == hipMemoryTypeHost) && a.devicePointer &&
+                        z.devicePointer == (void*)((uint8_t*)a.devicePointer + bytes - 1) &&
+                        (uintptr_t)a.devicePointer % align == 0;
+    *view = mapped ? (uint8_t*)a.devicePointer : nullptr;
+    return mapped ? Dst::kMapped : Dst::kOther;
+}
+
+// The two pinned buffers of the table copy; false if the host has no room for them.
+static bool table_pin_need(rgkc_ctx* c, uint64_t bytes) {
+    for (hipEvent_t& e : c->table_ev)
+        if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
+            (void)hipGetLastError();
+            e = nullptr;
+            return false;
+        }
+    if (bytes <= c->table_pin_cap) return true;
+    c->table_pin_cap = 0;
+    for (int i = 0; i < 2; i++) {
+        if (c->table_pin[i]) (void)hipHostFree(c->table_pin[i]);
+        c->table_pin[i] = nullptr;
+        if (hipHostMalloc((void**)&c->table_pin[i], bytes, hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
+            c->table_pin[i] = nullptr;
+            return false;
+        }
+    }
+    c->table_pin_cap = bytes;
+    return true;
+}
+
+// The partitions' rows leave the device as one dense table. Pinned and device destinations are written by the
+// gather itself, at the link's rate: 1.18 GB into pinned memory 22.0 ms from 512 partitions (a copy each and
+// array 30.4) and from 64 (21.9), 21.2 from one (20.7: few long runs go by the runtime's copies). For ordinary memory,
+// chunks of the table are gathered into two pinned buffers by turns, and the host copies one to the caller
+// while the device fills the other: 46-48 ms, the rate of one thread's copy (the runtime's copies to
+// pageable memory 68-75). A copy per partition and array costs 11-12 us; they remain for destinations of other
+// kinds and when no buffer can be pinned.
 int rgkc_copy_table(rgkc_ctx* c, void* keys, uint32_t* counts) {
     if (!c) return RGKC_E_ARG;
     if (!c->table_ok) return fail(c, RGKC_E_STATE, "no table");
@@ -1348,53 +1396,70 @@ int rgkc_copy_table(rgkc_ctx* c, void* keys, uint32_t* counts) {
     }
     const uint64_t total = first[n];
     if (!total) return 0;
+    uint8_t *dk = nullptr, *dc = nullptr;  // the device's view of mapped destinations
+    const Dst tk = keys ? destination(c, keys, total * W, W, &dk) : Dst::kMapped;
+    const Dst tc = counts ? destination(c, counts, total * 4, 4, &dc) : Dst::kMapped;
+    if (total / (uint64_t)n >= kLongRun) dk = dc = nullptr;
     const uint64_t chunk = std::min<uint64_t>(total, kTableChunk / (W + 4));
-    if (c->table_pin_cap < chunk * (W + 4)) {
-        for (int i = 0; i < 2; i++) {
-            if (c->table_pin[i]) (void)hipHostFree(c->table_pin[i]);
-            c->table_pin[i] = nullptr;
-        }
-        c->table_pin_cap = 0;
-        for (int i = 0; i < 2; i++)
-            if (hipHostMalloc((void**)&c->table_pin[i], chunk * (W + 4), hipHostMallocDefault) != hipSuccess) {
-                (void)hipGetLastError();
-                return fail(c, RGKC_E_NOMEM, "pinned allocation of %zu bytes failed", (size_t)(chunk * (W + 4)));
-            }
-        for (hipEvent_t& e : c->table_ev)
-            if (!e) HIPC(c, hipEventCreateWithFlags(&e, hipEventDisableTiming));
-        c->table_pin_cap = chunk * (W + 4);
-    }
+    const bool host = tk == Dst::kHost || tc == Dst::kHost;
+    const bool staged = host && table_pin_need(c, chunk * (W + 4));
+    void* const hk = tk == Dst::kHost && staged ? keys : nullptr;  // through the pinned buffers
+    uint32_t* const hc = tc == Dst::kHost && staged ? counts : nullptr;
     NEED(c, c->gather_plan, plan.size() * 8);
     HIPC(c, hipMemcpyAsync(c->gather_plan.p, plan.data(), plan.size() * 8, hipMemcpyHostToDevice, s));
-    struct Chunk { uint64_t r0 = 0, r1 = 0; } inflight[2];
-    uint64_t next = 0;
-    int p0 = 0;  // first partition with rows at or after `next`
-    auto launch = [&](int b) -> hipError_t {
-        inflight[b] = Chunk{next, next};
-        if (next >= total) return hipSuccess;
-        while (first[p0 + 1] <= next) p0++;
+    // rows [r0, r1) by one launch, r1 cut to the partitions one takes; p0: the partition of r0 or one before it
+    auto gather = [&](uint64_t r0, uint64_t& r1, int& p0, void* to_k, uint32_t* to_c) -> hipError_t {
+        while (first[p0 + 1] <= r0) p0++;
         const int np = std::min(n - p0, kGatherParts);
-        const uint64_t r1 = std::min(std::min(next + chunk, total), first[p0 + np]);
+        r1 = std::min(r1, first[p0 + np]);
         GatherArgs a{};
         a.first = c->gather_plan.as<uint64_t>() + p0;
         a.src = c->gather_plan.as<uint64_t>() + n + 1 + p0;
         a.n_parts = np;
         a.keys = c->keys.p; a.keys2 = c->keys2.p;
         a.counts = c->counts.as<uint32_t>(); a.counts2 = c->counts2.as<uint32_t>();
-        a.r0 = next; a.r1 = r1;
-        a.dst_keys = keys ? (void*)c->table_pin[b] : nullptr;
-        a.dst_counts = counts ? (uint32_t*)(c->table_pin[b] + (r1 - next) * W) : nullptr;
-        inflight[b].r1 = next = r1;
-        if (hipError_t e = launch_gather_rows(a, (int)W, s)) return e;
-        return hipEventRecord(c->table_ev[b], s);
+        a.r0 = r0; a.r1 = r1;
+        a.dst_keys = to_k;
+        a.dst_counts = to_c;
+        return launch_gather_rows(a, (int)W, s);
     };
-    for (int b = 0; b < 2; b++) HIPC(c, launch(b));
-    for (int b = 0; inflight[b].r1 > inflight[b].r0; b ^= 1) {
-        HIPC(c, hipEventSynchronize(c->table_ev[b]));
-        const uint64_t r0 = inflight[b].r0, nr = inflight[b].r1 - r0;
-        if (keys) memcpy((uint8_t*)keys + r0 * W, c->table_pin[b], nr * W);
-        if (counts) memcpy(counts + r0, c->table_pin[b] + nr * W, nr * 4);
-        HIPC(c, launch(b));
+    if (dk || dc) {
+        int p0 = 0;
+        for (uint64_t r0 = 0, r1 = total; r0 < total; r0 = r1, r1 = total)
+            HIPC(c, gather(r0, r1, p0, dk ? dk + r0 * W : nullptr, dc ? (uint32_t*)dc + r0 : nullptr));
+    }
+    const bool rk = keys && !dk && !hk, rc = counts && !dc && !hc;  // the runtime's copies
+    for (int i = 0; i < n && (rk || rc); i++) {
+        const uint64_t r = first[i], nr = c->h_rows[i], at = c->h_row_start[i];
+        if (!nr) continue;
+        const uint8_t* const sk = (const uint8_t*)(c->h_row_buf[i] ? c->keys2 : c->keys).p;
+        const uint32_t* const sc = (c->h_row_buf[i] ? c->counts2 : c->counts).as<uint32_t>();
+        if (rk) HIPC(c, hipMemcpyAsync((uint8_t*)keys + r * W, sk + at * W, nr * W, hipMemcpyDefault, s));
+        if (rc) HIPC(c, hipMemcpyAsync(counts + r, sc + at, nr * 4, hipMemcpyDefault, s));
+    }
+    if (hk || hc) {
+        struct Chunk { uint64_t r0 = 0, r1 = 0; } inflight[2];
+        uint64_t next = 0;
+        int p0 = 0;
+        auto launch = [&](int b) -> hipError_t {
+            inflight[b] = Chunk{next, next};
+            if (next >= total) return hipSuccess;
+            uint64_t r1 = std::min(next + chunk, total);
+            // the counts' place in the buffer does not wait for r1: a whole chunk's keys come before it
+            const hipError_t e = gather(next, r1, p0, hk ? (void*)c->table_pin[b] : nullptr,
+                                        hc ? (uint32_t*)(c->table_pin[b] + chunk * W) : nullptr);
+            if (e) return e;
+            inflight[b].r1 = next = r1;
+            return hipEventRecord(c->table_ev[b], s);
+        };
+        for (int b = 0; b < 2; b++) HIPC(c, launch(b));
+        for (int b = 0; inflight[b].r1 > inflight[b].r0; b ^= 1) {
+            HIPC(c, hipEventSynchronize(c->table_ev[b]));
+            const uint64_t r0 = inflight[b].r0, nr = inflight[b].r1 - r0;
+            if (hk) memcpy((uint8_t*)hk + r0 * W, c->table_pin[b], nr * W);
+            if (hc) memcpy(hc + r0, c->table_pin[b] + chunk * W, nr * 4);
+            HIPC(c, launch(b));
+        }
     }
     HIPC(c, hipStreamSynchronize(s));  // also on the way out: nothing reads `plan` any more
     return 0;
