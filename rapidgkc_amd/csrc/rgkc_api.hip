@@ -1195,8 +1195,14 @@ static uint32_t host_kmer_mm(const uint8_t* r, uint32_t bm3, uint32_t t0, int k,
     return mm;
 }
 
+// Offsets that decrease would put a partition's end past the store's last byte, which is the last offset.
+static bool offsets_ascend(const uint64_t* part_offs, int n_parts) {
+    return std::is_sorted(part_offs, part_offs + n_parts + 1);
+}
+
 int rgkc_store_minimizer_length(const uint8_t* store, const uint64_t* part_offs, int n_parts, int k, int* p_out) {
     if (!part_offs || !p_out || n_parts < 1 || k < 8 || k > 63 || (!store && part_offs[n_parts] > 0)) return RGKC_E_ARG;
+    if (!offsets_ascend(part_offs, n_parts)) return RGKC_E_ARG;
     // records of two or more k-mers: every k-mer of a superkmer has the superkmer's minimizer, so
     // the minimizer length is the one under which all of them agree
     struct Rec { const uint8_t* r; uint32_t bm3, L; };
@@ -1234,6 +1240,7 @@ int rgkc_count_host_store(rgkc_ctx* c, const uint8_t* store, const uint64_t* par
                           uint64_t* row_counts, uint64_t* distinct) {
     (void)part_ids;
     if (!c || !part_offs || n_parts < 1 || (!store && part_offs[n_parts] > 0)) return RGKC_E_ARG;
+    if (!offsets_ascend(part_offs, n_parts)) return fail(c, RGKC_E_ARG, "partition offsets must not decrease");
     if (p == 0) {
         const int rc = rgkc_store_minimizer_length(store, part_offs, n_parts, k, &p);
         if (rc) return fail(c, rc, "the minimizer length could not be recovered from the records");
