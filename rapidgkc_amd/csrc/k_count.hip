@@ -2,7 +2,7 @@
 // laid out.
 //
 //  1. k_count_units, persistent: a workgroup takes units b, b + G, b + 2G, ... and counts each in
-//     one or more sweeps over its records: chunks of records have their 2-bit words copied into LDS, the
+//     one or more sweeps over its records (of a large unit a share of its hash slices): chunks of records have their 2-bit words copied into LDS, the
 //     k-mers are taken from there four at a time and counted in an open-addressing LDS table. A unit with
 //     more distinct keys than the table holds is counted in hash slices, one sweep each, that read the
 //     records again; their number follows the ratio of distinct keys to instances seen so far, and a sweep
@@ -17,6 +17,8 @@
 //
 // The canonical key is the smaller of the digit-reversed 2k-bit window and the complemented one
 // (cpu_funcs.cpp:427-436, gpu_kmercounting.cu:63-74).
+#include <stddef.h>
+
 #include <algorithm>
 
 #include "rgkc_device.h"
@@ -673,7 +675,8 @@ __global__ __launch_bounds__(kItemThreads, 4) void k_count_units(CountArgs a) {
     __shared__ uint32_t tmp2[2 * NW], wtot[NW];
     __shared__ unsigned long long sh_in;  // chunk: records << 20 | words
     __shared__ uint64_t sh_row_base;
-    __shared__ uint32_t sh_ovf, sh_np, sh_long, sh_nstack, sh_first, sh_q0, sh_next, sh_next_q;
+    __shared__ uint32_t sh_ovf, sh_np, sh_long, sh_nstack, sh_next, sh_next_q;
+    __shared__ uint32_t sh_first, sh_q0, sh_s0, sh_ns;  // next slice of the item, of q0 from slice s0 of ns on
     __shared__ Cut cur;
     uint32_t* const same = mp.same;
     uint16_t* const pmap = mp.pmap;
@@ -701,31 +704,43 @@ __global__ __launch_bounds__(kItemThreads, 4) void k_count_units(CountArgs a) {
         d.part = word(0); d.inst = word(1); d.n_rec = word(2); d.n_word = word(3);
         d.desc = (uint64_t)word(4) | ((uint64_t)word(5) << 32);
         d.word = (uint64_t)word(6) | ((uint64_t)word(7) << 32);
-        d.q = d.pad = 0;
+        d.q = d.share = 0;
         return d;
     };
-    UnitDesc ud = unit(fetch(it));
-    uint32_t ahead = fetch(it + G);
-    // Initial hash slices of a unit: what its distinct keys should take by the ratio seen so far. The next unit's are
+    constexpr int kQ = offsetof(UnitDesc, q) / 4, kShare = offsetof(UnitDesc, share) / 4;
+    uint32_t ahead = fetch(it);
+    UnitDesc ud = unit(ahead);
+    // Initial hash slices of a unit's share (one of q): what its distinct keys should take by the ratio seen so far. The next unit's are
     // worked out by the last wave, which has the fewest records, while the others look for equal ones (at the sweep's
     // end by thread 0 they took 6% of the kernel).
-    auto slices = [&](uint32_t inst) {
+    auto slices = [&](uint32_t v) {
+        const uint32_t inst = (uint32_t)__builtin_amdgcn_readlane((int)v, 1), shares = max((uint32_t)__builtin_amdgcn_readlane((int)v, kQ), 1u);
         const float ratio = est_i > 4ull * a.unit_cap ? (float)est_d / (float)est_i : kFill<K> / (float)a.unit_cap;
         uint32_t q = (uint32_t)ceilf(1.1f * (float)inst * fminf(ratio, 1.0f) / kFill<K>);
         q = max(1u, min(q, kMaxSlices));
         if ((float)inst <= kFill<K>) q = 1u;
         est_i = __hip_atomic_load(&a.plan_n[kPlanSeenInst], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         est_d = __hip_atomic_load(&a.plan_n[kPlanSeenDistinct], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        return q;
+        return (q + shares - 1u) / shares;
+    };
+    // thread 0: the item `v` begins, its share cut into q slices
+    auto begin = [&](uint32_t v, uint32_t q) {
+        sh_q0 = q;
+        sh_s0 = (uint32_t)__builtin_amdgcn_readlane((int)v, kShare) * q;
+        sh_ns = (uint32_t)__builtin_amdgcn_readlane((int)v, kQ) * q;
+        sh_first = 1;
+        cur = Cut{sh_s0, sh_ns};
     };
     bool planned = false;  // the next unit's slices are in sh_next_q
-    if (threadIdx.x == 0) {
-        sh_nstack = 0;
-        sh_q0 = slices(ud.inst);
-        sh_first = 1;
-        cur = Cut{0, sh_q0};
-        sh_ovf = 0;
+    {
+        const uint32_t q = slices(ahead);
+        if (threadIdx.x == 0) {
+            sh_nstack = 0;
+            begin(ahead, q);
+            sh_ovf = 0;
+        }
     }
+    ahead = fetch(it + G);
 
     uint32_t dn[R], wn[WPT];  // the next chunk's descriptors and words of this thread
     auto load = [&](const UnitDesc& d, uint32_t c, uint32_t w) {
@@ -795,7 +810,7 @@ __global__ __launch_bounds__(kItemThreads, 4) void k_count_units(CountArgs a) {
         else if (again) load(ud, 0, 0);
         else load(unit(ahead), 0, 0);
         if (!planned && wave == (uint32_t)NW - 1u) {
-            const uint32_t q = slices((uint32_t)__builtin_amdgcn_readlane((int)ahead, 1));
+            const uint32_t q = slices(ahead);
             if (lane == 0) sh_next_q = q;
         }
         planned = true;
@@ -946,15 +961,11 @@ __global__ __launch_bounds__(kItemThreads, 4) void k_count_units(CountArgs a) {
                 cur = stack[--sh_nstack];
                 sh_next = 0;
             } else if (sh_first < sh_q0) {
-                cur = Cut{sh_first++, sh_q0};
+                cur = Cut{sh_s0 + sh_first++, sh_ns};
                 sh_next = 0;
             } else {
                 sh_next = 1;
-                if (it + G < it_end) {
-                    sh_q0 = sh_next_q;
-                    sh_first = 1;
-                    cur = Cut{0, sh_q0};
-                }
+                if (it + G < it_end) begin(ahead, sh_next_q);
             }
         }
         __syncthreads();

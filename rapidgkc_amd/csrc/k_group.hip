@@ -77,7 +77,8 @@ __global__ __launch_bounds__(1024) void k_hist(CountArgs a) {
 // the first. A serial walk over the 4096 counts by one thread, run twice (to count and to fill), took
 // 1.5 ms for 512 partitions; the links are a few hundred LDS reads.
 // A unit of more than kDirectSlices * unit_cap instances gets a key region per hash slice (heavy_on)
-// and is expanded by k_expand; every other unit is counted from its records (k_count.hip).
+// and is expanded by k_expand; every other unit is counted from its records (k_count.hip), a large one by
+// several work items (unit_shares).
 __global__ __launch_bounds__(kPlanThreads) void k_plan(CountArgs a) {
     __shared__ uint32_t pre[kSubIds + 1];             // instances of the light sub-buckets before each one
     __shared__ uint16_t nxt[kSubIds];                 // end of the unit that begins here, then the unit
@@ -175,7 +176,7 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan(CountArgs a) {
         sr += ur[j];
         sw += uw[j];
         const bool keyed = a.heavy_on && (uint64_t)ui[j] > (uint64_t)cap * kDirectSlices;
-        nd += (ui[j] && !keyed) ? 1u : 0u;
+        nd += keyed ? 0u : unit_shares(ui[j], cap);
     }
     uint32_t er, ew, tr, tw, td;
     wg_exscan2_u32(sr, sw, tmp, er, ew, tr, tw);
@@ -205,7 +206,7 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan(CountArgs a) {
         d.inst = ui[j];
         d.n_rec = ur[j];
         d.n_word = uw[j];
-        d.q = 0;
+        d.share = 0;
         d.desc = desc0 + er;
         d.word = word0 + ew;
         if (a.heavy_on && (uint64_t)ui[j] > (uint64_t)cap * kDirectSlices) {
@@ -222,8 +223,8 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan(CountArgs a) {
             a.key_units[ix] = ku;
             for (uint32_t s = 0; s < q; s++) a.key_items[ku.item0 + s] = (ix << 8) | s;
         } else {
-            a.unit_items[base_d + ed] = d;
-            ed++;
+            d.q = unit_shares(ui[j], cap);
+            for (d.share = 0; d.share < d.q; d.share++) a.unit_items[base_d + ed++] = d;
         }
         er += ur[j];
         ew += uw[j];

@@ -442,8 +442,8 @@ int count_buckets(rgkc_ctx* c, uint32_t b0, uint32_t b1, uint32_t cmin, uint32_t
     const uint64_t most_segs = std::max<uint64_t>(16, std::min<uint64_t>(kGroupSegments, 4096 / nb));
     const uint32_t n_segs = (uint32_t)std::min<uint64_t>(std::max<uint64_t>((most_rec + 1023) / 1024, 1), most_segs);
     // item bounds: two neighbouring units of a bucket hold more than `cap` instances together, an expanded
-    // unit more than kDirectSlices * cap
-    const uint64_t most_items = std::min<uint64_t>(2 * N / cap + 2 * nb, (uint64_t)nb * kSubIds);
+    // unit more than kDirectSlices * cap; a unit of more than kShareCaps * cap is an item for each of them
+    const uint64_t most_items = std::min<uint64_t>(2 * N / cap + 2 * nb, (uint64_t)nb * kSubIds + N / (cap * kShareCaps));
     const uint64_t most_kunits = N / (cap * kDirectSlices) + 1, most_kitems = (N + N / kDirectSlices) / cap + 2;
     const size_t area = (size_t)nb * kSubIds * 12 + kPlanWords * 8;
     NEEDC(c, c->plan_area, area);
@@ -516,7 +516,9 @@ int count_buckets(rgkc_ctx* c, uint32_t b0, uint32_t b1, uint32_t cmin, uint32_t
         a.heavy_on = 0;
         HIPC(c, hipMemsetAsync(a.plan_n, 0, kPlanWords * 8, s));
         HIPC(c, launch_plan(a, s));
-        n_items += n_kunits;
+        HIPC(c, hipMemcpyAsync(c->h_plan, a.plan_n, kPlanWords * 8, hipMemcpyDeviceToHost, s));
+        HIPC(c, hipStreamSynchronize(s));
+        n_items = c->h_plan[kPlanItems];
         n_kunits = n_kitems = 0;
     }
     REC(c, EV_PLAN, s);

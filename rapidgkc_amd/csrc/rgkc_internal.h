@@ -126,13 +126,22 @@ hipError_t launch_p1_batch(const P1Args& a, hipStream_t s);
 // 12.1 with 2 (1.2 G k-mers at 30x), 2.43 and 1.96 (188 M, k=25): a unit is read once per sweep.
 constexpr uint32_t kDirectSlices = 2;
 constexpr uint32_t kMaxKeySlices = 127; // hash slices (key regions) of an expanded unit
+// A unit counted from its records goes in shares of at most this many unit_caps (hash slices, a work item
+// each): one workgroup took all sweeps of a large one. 13 M k-mers of 7 minimizers (k=21, p=3) without
+// expansion 2270 ms, so 25; 12 M (k=55, p=5) 513, 17; 11 M of low complexity 301, 8.0.
+// A share's sweeps are a whole number, so that smaller ones read the records more often.
+constexpr uint32_t kShareCaps = 4;
+__host__ __device__ inline uint32_t unit_shares(uint32_t inst, uint32_t cap) {
+    const uint64_t most = (uint64_t)cap * kShareCaps, n = (inst + most - 1) / most;
+    return (uint32_t)(n < (1u << 16) ? n : 1u << 16);
+}
 constexpr int kSmallUnits = 1024;       // units of a bucket that the small grouping kernel takes
 enum { kPlanItems, kPlanKeySlots, kPlanKeyUnits, kPlanKeyItems, kPlanSeenInst, kPlanSeenDistinct, kPlanWords };
 // A unit of work: sub-buckets of one partition whose records lie together.
 struct UnitDesc {
     uint32_t part, inst, n_rec, n_word;  // partition, k-mer instances, records, their 2-bit words
     uint64_t desc, word;                 // first record descriptor and first word
-    uint32_t q, pad;                     // slices (expanded units)
+    uint32_t q, share;                   // its hash slices: key regions, or work items and which of them
 };
 // An expanded unit: key regions of 1 + cs slots per slice (the fill count, then keys) from slot key0 on.
 struct KeyUnit {
