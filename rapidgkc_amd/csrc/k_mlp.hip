@@ -1,12 +1,14 @@
 // Load predictor network on gfx950: a 3-layer MLP (ReLU) with BF16 weights and FP32
 // accumulation, trained with masked MSE and Adam. Training batches go row by row in three launches;
-// larger ones through plain LDS-tiled GEMMs (64x64 tiles, 4x4 per thread).
+// larger ones and wide layers through plain LDS-tiled GEMMs (64x64 tiles, 4x4 per thread).
 //
 // Parameters (flat FP32 master copy, the BF16 copy is what the GEMMs read):
 //   W1[n_in x h1] b1[h1] W2[h1 x h2] b2[h2] W3[h2 x n_out] b3[n_out]   (row-major, x @ W)
 #include <hip/hip_bf16.h>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+
+#include <algorithm>
 
 #include "rgkc_internal.h"
 
@@ -127,12 +129,12 @@ __global__ void k_to_bf16(size_t n, const float* __restrict__ w, __hip_bfloat16*
     if (i < n) wb[i] = __float2bfloat16(w[i]);
 }
 
-// ---- batches of at most kRowBatch rows: three launches ------------------------------------------------
+// ---- batches that go row by row (mlp_by_rows): three launches -----------------------------------------
 // A training batch is 16 to 64 rows, so the layers are vector-matrix products whose cost is latency: as
 // GEMMs of 64 x 64 tiles over the whole K, two workgroups walked layer 1's 2563 inputs in 160 steps
 // (0.57 ms of 16 launches for the gradient of 16 rows, n_in 2563, 128 x 128 hidden, 1024 out). Instead:
-//   k_rows_in    layer 1's products, split over K: a workgroup takes kKC inputs x 64 outputs of up to 64
-//                rows and leaves partial sums (summed in a fixed order by the next kernel);
+//   k_rows_in    layer 1's products, split over K: a workgroup takes kper inputs (kKC at a time) x 64
+//                outputs of up to 64 rows and leaves partial sums (summed in a fixed order by the next kernel);
 //   k_rows_net   one workgroup per row: the rest of the forward pass, the loss and the activations'
 //                gradients, row vectors in LDS, weights read once per row (they stay in L2);
 //   k_rows_grad  a thread per parameter sums its gradient over the rows.
@@ -140,26 +142,30 @@ __global__ void k_to_bf16(size_t n, const float* __restrict__ w, __hip_bfloat16*
 constexpr int kKC = 32;
 constexpr int kRowThreads = 1024;
 
-__global__ __launch_bounds__(256) void k_rows_in(int B, int n_in, int h1, const float* __restrict__ X,
+__global__ __launch_bounds__(256) void k_rows_in(int B, int n_in, int h1, int kper, const float* __restrict__ X,
                                                  const __hip_bfloat16* __restrict__ W, float* __restrict__ part) {
     __shared__ float xs[kKC][65];
     __shared__ float ws[kKC][64];
-    const int n0 = blockIdx.x * 64, k0 = blockIdx.y * kKC, b0 = blockIdx.z * 64;
-    const int kn = min(kKC, n_in - k0), bn = min(64, B - b0);
-    for (int i = threadIdx.x; i < 64 * kKC; i += 256) {
-        const int b = i / kKC, kk = i % kKC;
-        xs[kk][b] = (b < bn && kk < kn) ? X[(size_t)(b0 + b) * n_in + k0 + kk] : 0.f;
-        const int n = i % 64, kw = i / 64;
-        ws[kw][n] = (n0 + n < h1 && kw < kn) ? __bfloat162float(W[(size_t)(k0 + kw) * h1 + n0 + n]) : 0.f;
-    }
-    __syncthreads();
+    const int n0 = blockIdx.x * 64, b0 = blockIdx.z * 64, bn = min(64, B - b0);
+    const int kb = blockIdx.y * kper, ke = min(kb + kper, n_in);
     const int n = threadIdx.x & 63, r0 = threadIdx.x >> 6;
     float acc[16] = {};
-    for (int kk = 0; kk < kKC; kk++) {
-        const float w = ws[kk][n];
+    for (int k0 = kb; k0 < ke; k0 += kKC) {
+        const int kn = min(kKC, ke - k0);
+        if (k0 > kb) __syncthreads();
+        for (int i = threadIdx.x; i < 64 * kKC; i += 256) {
+            const int b = i / kKC, kk = i % kKC;
+            xs[kk][b] = (b < bn && kk < kn) ? X[(size_t)(b0 + b) * n_in + k0 + kk] : 0.f;
+            const int nn = i % 64, kw = i / 64;
+            ws[kw][nn] = (n0 + nn < h1 && kw < kn) ? __bfloat162float(W[(size_t)(k0 + kw) * h1 + n0 + nn]) : 0.f;
+        }
+        __syncthreads();
+        for (int kk = 0; kk < kKC; kk++) {
+            const float w = ws[kk][n];
 #pragma unroll
-        for (int i = 0; i < 16; i++)
-            if (4 * i < bn) acc[i] = fmaf(xs[kk][r0 + 4 * i], w, acc[i]);
+            for (int i = 0; i < 16; i++)
+                if (4 * i < bn) acc[i] = fmaf(xs[kk][r0 + 4 * i], w, acc[i]);
+        }
     }
     if (n0 + n >= h1) return;
 #pragma unroll
@@ -306,19 +312,43 @@ hipError_t mlp_to_bf16(const float* w, void* wb, size_t n, hipStream_t s) {
     return hipGetLastError();
 }
 
-// Batches that go row by row: up to kRowBatch rows whose vectors fit a workgroup's LDS.
+// Batches that go row by row: up to kRowBatch rows whose vectors fit a workgroup's LDS, and
+//  - layers 2 and 3 of at most kRowWeights weights, and kRowReads of them over all rows: k_rows_net reads
+//    them once per row, the tiles once per 64 rows. Forward, tiles / rows: 2048 x 2048 x 2048 (8.4 M) 0.50 / 0.58 ms at
+//    1 row; 1024 x 1024 x 1024 (2.1 M) 1.26 / 0.82 at 512 rows, 1.55 / 1.62 at 1024.
+//  - training: as many products of parameters and rows as k_rows_grad sums (kRowProducts), or as many as the tiles'
+//    walk over n_in makes up for. A step, tiles / rows: 100 x 1400 x 1400 x 10 1.23 / 0.64 ms at 256 rows, 2.20 / 2.49 at 1024;
+//    1000 x 10000 x 100 x 100 1.93 / 0.60 at 16, 4.6 / 9.3 at 1024; 50000 x 512 x 64 x 64 22.4 / 18.1 at 1024.
+//  - forward alone: a walk that is worth it. 16 x 16 x 16 x 16 0.055 / 0.071 ms at 1024 rows, 300 x 64 x 64 x 64 0.19 / 0.14;
+//    64 x 128 x 128 x 8000 0.068 / 0.104 at 1 row (a row's outputs are made 1024 at a time).
 constexpr int kRowBatch = 1024;
+constexpr uint64_t kRowWeights = 1u << 22, kRowReads = 1u << 30, kRowProducts = 1u << 31;
 static size_t row_lds(const MlpDims& d) { return ((size_t)kRowThreads + d.h1 + d.h2 + d.n_out) * 4; }
-bool mlp_by_rows(const MlpDims& d, int B) { return B <= kRowBatch && row_lds(d) <= 60 * 1024; }
-size_t mlp_part_floats(const MlpDims& d, int B) { return (size_t)((d.n_in + kKC - 1) / kKC) * B * d.h1; }
+bool mlp_by_rows(const MlpDims& d, int B, bool train) {
+    const uint64_t w = (uint64_t)d.h1 * d.h2 + (uint64_t)d.h2 * d.n_out, walk = (uint64_t)d.n_in + d.h1 + d.h2;
+    if (B > kRowBatch || row_lds(d) > 60 * 1024 || w > kRowWeights || w * B > kRowReads) return false;
+    if (train) return d.total() * B <= kRowProducts || d.total() * B <= (uint64_t)d.n_in << 20;
+    return walk >= 256 && (uint64_t)d.n_out <= 4 * walk;
+}
+// Inputs per workgroup of layer 1: kKC, or as many of them as keep the partial sums within kPartFloats (64 MB; a
+// row path has at most 14336 * 1024 outputs of layer 1) and the grid within the device's limit.
+constexpr uint64_t kPartFloats = 1u << 24, kPartSplits = 1u << 15;
+static int row_kper(const MlpDims& d, int B) {
+    const uint64_t most = std::max<uint64_t>(1, std::min(kPartSplits, kPartFloats / ((uint64_t)B * d.h1)));
+    const uint64_t chunks = ((uint64_t)d.n_in + kKC - 1) / kKC;
+    return (int)((chunks + most - 1) / most) * kKC;
+}
+static int row_splits(const MlpDims& d, int B) { return (int)(((uint64_t)d.n_in + row_kper(d, B) - 1) / row_kper(d, B)); }
+size_t mlp_part_floats(const MlpDims& d, int B) { return (size_t)row_splits(d, B) * B * d.h1; }
 
 hipError_t mlp_rows_forward(const MlpDims& d, const void* wb, const float* w32, const float* X, int B, float* part,
                             const float* T, const float* mask, float mask_sum, float* H1, float* H2, float* Y, float* dY,
                             float* dH1, float* dH2, float* row_loss, hipStream_t s) {
     const __hip_bfloat16* W = (const __hip_bfloat16*)wb;
-    const int S = (d.n_in + kKC - 1) / kKC;
-    hipLaunchKernelGGL(k_rows_in, dim3((d.h1 + 63) / 64, S, (B + 63) / 64), dim3(256), 0, s, B, d.n_in, d.h1, X, W + d.off_W1(),
-                       part);
+    const int S = row_splits(d, B);
+    hipLaunchKernelGGL(k_rows_in, dim3((d.h1 + 63) / 64, S, (B + 63) / 64), dim3(256), 0, s, B, d.n_in, d.h1, row_kper(d, B), X,
+                       W + d.off_W1(), part);
+    if (hipError_t e = hipGetLastError()) return e;
     hipLaunchKernelGGL(k_rows_net, dim3(B), dim3(kRowThreads), row_lds(d), s, d, B, S, W, w32, (const float*)part, T, mask,
                        1.f / (mask_sum > 1.f ? mask_sum : 1.f), H1, H2, Y, dY, dH1, dH2, row_loss);
     return hipGetLastError();

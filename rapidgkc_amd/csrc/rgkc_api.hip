@@ -2012,12 +2012,15 @@ static int mlp_stage(rgkc_mlp* m, const float* x, const float* t, const float* m
     const MlpDims& d = m->d;
     hipStream_t s = c->stream;
     const size_t nY = (size_t)B * d.n_out;
-    const bool rows = mlp_by_rows(d, B);
+    bool rows = mlp_by_rows(d, B, t != nullptr);
     NEED(c, m->X, (size_t)B * d.n_in * 4);
     NEED(c, m->H1, (size_t)B * d.h1 * 4);
     NEED(c, m->H2, (size_t)B * d.h2 * 4);
     NEED(c, m->Y, nY * 4);
-    if (rows) NEED(c, m->part, (mlp_part_floats(d, B) + B) * 4);
+    if (rows && m->part.need((mlp_part_floats(d, B) + B) * 4) != hipSuccess) {  // the tiles take no partial sums
+        (void)hipGetLastError();
+        rows = false;
+    }
     HIPC(c, hipMemcpyAsync(m->X.p, x, (size_t)B * d.n_in * 4, hipMemcpyHostToDevice, s));
     float msum = (float)nY;
     if (t) {

@@ -284,7 +284,7 @@ hipError_t mlp_backward(const MlpDims& d, const void* wb, const float* X, int B,
 // The same for batches that go row by row (mlp_by_rows): `part` holds mlp_part_floats, row_loss B floats.
 // T null: forward only; else the activations' gradients and each row's loss too, from which mlp_rows_grad
 // makes the parameters' gradients and the loss.
-bool mlp_by_rows(const MlpDims& d, int B);
+bool mlp_by_rows(const MlpDims& d, int B, bool train);
 size_t mlp_part_floats(const MlpDims& d, int B);
 hipError_t mlp_rows_forward(const MlpDims& d, const void* wb, const float* w32, const float* X, int B, float* part,
                             const float* T, const float* mask, float mask_sum, float* H1, float* H2, float* Y, float* dY,
