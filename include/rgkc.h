@@ -185,6 +185,7 @@ int rgkc_sample_features(rgkc_ctx* ctx, int k, int p, int parts, uint32_t* hist,
  * x: B x n_in, targets/mask/y: B x n_out (host arrays). Gradients are w.r.t. the BF16 weights. */
 typedef struct rgkc_mlp rgkc_mlp;
 int rgkc_mlp_create(rgkc_ctx* ctx, int n_in, int h1, int h2, int n_out, rgkc_mlp** out);
+/* In any order with the context: a network whose context is gone can only be destroyed (RGKC_E_STATE). */
 int rgkc_mlp_destroy(rgkc_mlp* m);
 int rgkc_mlp_num_params(const rgkc_mlp* m, uint64_t* n);
 int rgkc_mlp_set_params(rgkc_mlp* m, const float* params);

@@ -85,6 +85,7 @@ enum Ev { EV_START, EV_PACK, EV_SEG, EV_P1C, EV_P1E, EV_CB, EV_IDX, EV_PLAN, EV_
 
 struct rgkc_ctx {
     int device = 0;
+    std::vector<rgkc_mlp*> nets;  // the context's networks: told when it goes first
     hipStream_t stream = nullptr;
     std::string err;
     hipEvent_t ev[EV_N] = {};
@@ -1037,6 +1038,13 @@ int do_sort_rows(rgkc_ctx* c) {
 
 }  // namespace
 
+struct rgkc_mlp {
+    rgkc_ctx* c = nullptr;  // null once the context is destroyed
+    MlpDims d;
+    DevBuf w32, wb, g, m1, m2, X, T, M, H1, H2, Y, dY, dH1, dH2, loss, part;
+    int step = 0;
+};
+
 extern "C" {
 
 size_t rgkc_device_reset(int device) {
@@ -1076,6 +1084,7 @@ int rgkc_destroy(rgkc_ctx* c) {
     if (!c) return 0;
     (void)hipSetDevice(c->device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
+    for (rgkc_mlp* m : c->nets) m->c = nullptr;
     stream_free(c);
     stage_free(c);
     for (int i = 0; i < EV_N; i++) if (c->ev[i]) (void)hipEventDestroy(c->ev[i]);
@@ -1948,13 +1957,6 @@ int rgkc_sample_features(rgkc_ctx* c, int k, int p, int parts, uint32_t* hist, u
 }
 
 // ---- load predictor network -------------------------------------------------------------------
-struct rgkc_mlp {
-    rgkc_ctx* c = nullptr;
-    MlpDims d;
-    DevBuf w32, wb, g, m1, m2, X, T, M, H1, H2, Y, dY, dH1, dH2, loss, part;
-    int step = 0;
-};
-
 int rgkc_mlp_create(rgkc_ctx* c, int n_in, int h1, int h2, int n_out, rgkc_mlp** out) {
     if (!c || !out || n_in < 1 || h1 < 1 || h2 < 1 || n_out < 1) return RGKC_E_ARG;
     (void)hipGetLastError();
@@ -1970,12 +1972,18 @@ int rgkc_mlp_create(rgkc_ctx* c, int n_in, int h1, int h2, int n_out, rgkc_mlp**
     HIPC(c, hipMemsetAsync(m->m1.p, 0, P * 4, c->stream));
     HIPC(c, hipMemsetAsync(m->m2.p, 0, P * 4, c->stream));
     HIPC(c, hipStreamSynchronize(c->stream));
+    c->nets.push_back(m);
     *out = m;
     return 0;
 }
 
 int rgkc_mlp_destroy(rgkc_mlp* m) {
-    if (m) { (void)hipStreamSynchronize(m->c->stream); delete m; }
+    if (!m) return 0;
+    if (rgkc_ctx* c = m->c) {
+        (void)hipStreamSynchronize(c->stream);
+        c->nets.erase(std::find(c->nets.begin(), c->nets.end(), m));
+    }
+    delete m;
     return 0;
 }
 
@@ -1988,6 +1996,7 @@ int rgkc_mlp_num_params(const rgkc_mlp* m, uint64_t* n) {
 int rgkc_mlp_set_params(rgkc_mlp* m, const float* p) {
     if (!m || !p) return RGKC_E_ARG;
     rgkc_ctx* c = m->c;
+    if (!c) return RGKC_E_STATE;  // its context is gone
     const size_t P = m->d.total();
     HIPC(c, hipMemcpyAsync(m->w32.p, p, P * 4, hipMemcpyHostToDevice, c->stream));
     HIPC(c, mlp_to_bf16(m->w32.as<float>(), m->wb.p, P, c->stream));
@@ -2001,6 +2010,7 @@ int rgkc_mlp_set_params(rgkc_mlp* m, const float* p) {
 int rgkc_mlp_get_params(rgkc_mlp* m, float* p) {
     if (!m || !p) return RGKC_E_ARG;
     rgkc_ctx* c = m->c;
+    if (!c) return RGKC_E_STATE;  // its context is gone
     HIPC(c, hipMemcpyAsync(p, m->w32.p, m->d.total() * 4, hipMemcpyDeviceToHost, c->stream));
     HIPC(c, hipStreamSynchronize(c->stream));
     return 0;
@@ -2059,6 +2069,7 @@ static int mlp_stage(rgkc_mlp* m, const float* x, const float* t, const float* m
 int rgkc_mlp_forward(rgkc_mlp* m, const float* x, int B, float* y) {
     if (!m || !x || !y || B < 1) return RGKC_E_ARG;
     rgkc_ctx* c = m->c;
+    if (!c) return RGKC_E_STATE;  // its context is gone
     (void)hipGetLastError();
     HIPC(c, hipSetDevice(c->device));
     if (int r = mlp_stage(m, x, nullptr, nullptr, B, nullptr)) return r;
@@ -2070,6 +2081,7 @@ int rgkc_mlp_forward(rgkc_mlp* m, const float* x, int B, float* y) {
 int rgkc_mlp_grad(rgkc_mlp* m, const float* x, const float* t, const float* mask, int B, float* grad, float* loss) {
     if (!m || !x || !t || B < 1) return RGKC_E_ARG;
     rgkc_ctx* c = m->c;
+    if (!c) return RGKC_E_STATE;  // its context is gone
     (void)hipGetLastError();
     HIPC(c, hipSetDevice(c->device));
     if (int r = mlp_stage(m, x, t, mask, B, loss)) return r;
@@ -2082,6 +2094,7 @@ int rgkc_mlp_train_step(rgkc_mlp* m, const float* x, const float* t, const float
                         float* loss) {
     if (!m || !x || !t || B < 1) return RGKC_E_ARG;
     rgkc_ctx* c = m->c;
+    if (!c) return RGKC_E_STATE;  // its context is gone
     (void)hipGetLastError();
     HIPC(c, hipSetDevice(c->device));
     if (int r = mlp_stage(m, x, t, mask, B, loss)) return r;
