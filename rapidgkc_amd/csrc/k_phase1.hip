@@ -94,7 +94,10 @@ __global__ void k_seg_fill_dev(const uint64_t* __restrict__ offs, const uint64_t
     const uint64_t gid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (gid == 0) {
         hdr[2] = seg_off[n];
-        if (n_rescan) *n_rescan = 0;  // of this batch's count pass (a captured graph records no memset)
+        if (n_rescan) {  // this batch's count pass starts from none (a captured graph records no memset)
+            n_rescan[2] += n_rescan[0];
+            n_rescan[0] = 0;
+        }
     }
     for (uint64_t r = gid; r < n && r < cap_reads; r += (uint64_t)gridDim.x * blockDim.x) {
         const uint64_t len = offs[r + 1] - offs[r];

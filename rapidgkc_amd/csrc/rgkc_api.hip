@@ -224,8 +224,9 @@ static int setup_lists(rgkc_ctx* c, P1Args& a, int T1, uint32_t n_wg) {
         }
     }
     NEED(c, c->skm_list, lbytes);
-    NEED(c, c->skm_n, ((size_t)2 * n_wg + 2) * 4);  // counts, rescan tiles, rescan count, list-order tiles
-    HIPC(c, hipMemsetAsync(c->skm_n.as<uint32_t>() + 2 * (size_t)n_wg, 0, 8, s));
+    // counts, rescan tiles, rescan count, list-order tiles, rescans of the stream's batches before the last
+    NEED(c, c->skm_n, ((size_t)2 * n_wg + 3) * 4);
+    HIPC(c, hipMemsetAsync(c->skm_n.as<uint32_t>() + 2 * (size_t)n_wg, 0, 12, s));
     a.skm_list = c->skm_list.as<uint64_t>();
     a.skm_n = c->skm_n.as<uint32_t>();
     a.skm_cap = (uint32_t)lcap;
@@ -266,6 +267,11 @@ int check_err_word(rgkc_ctx* c) {
     return 0;
 }
 
+void new_stats(rgkc_ctx* c) {
+    c->st = rgkc_stats{};
+    c->h_listorder = 0;
+}
+
 // Phase 1 on the resident batch (mm_hist: optional device histogram for sample features).
 int do_phase1(rgkc_ctx* c, int k, int p, int parts, uint32_t* mm_hist = nullptr) {
     if (!c->reads_ok) return fail(c, RGKC_E_STATE, "no read batch uploaded");
@@ -275,7 +281,7 @@ int do_phase1(rgkc_ctx* c, int k, int p, int parts, uint32_t* mm_hist = nullptr)
     hipStream_t s = c->stream;
     c->k = k; c->p = p; c->parts = parts;
     c->store_ok = false; c->table_ok = false; c->stream_ended = false;
-    c->st = rgkc_stats{};
+    new_stats(c);
     c->st.n_reads = c->n_reads; c->st.n_bases = c->n_bases;
     NEED(c, c->err_word, 64);
     HIPC(c, hipMemsetAsync(c->err_word.p, 0, 64, s));
@@ -372,7 +378,6 @@ int do_phase1(rgkc_ctx* c, int k, int p, int parts, uint32_t* mm_hist = nullptr)
     a.wg_map = a.skm_list ? a.wg_rescan : nullptr;
     HIPC(c, launch_p1_emit(a, n_rescan, s));
     REC(c, EV_P1E, s);
-    c->h_listorder = 0;
     if (a.skm_list) HIPC(c, hipMemcpyAsync(&c->h_listorder, a.n_listorder, 4, hipMemcpyDeviceToHost, s));
     // buckets: one per partition
     std::vector<uint32_t> bp(parts);
@@ -1261,7 +1266,7 @@ int rgkc_count_host_store(rgkc_ctx* c, const uint8_t* store, const uint64_t* par
     HIPC(c, hipSetDevice(c->device));
     hipStream_t s = c->stream;
     c->store_ok = false; c->table_ok = false; c->stream_ended = false;
-    c->st = rgkc_stats{};
+    new_stats(c);
     const uint64_t S = part_offs[n_parts];
     NEED(c, c->err_word, 64);
     HIPC(c, hipMemsetAsync(c->err_word.p, 0, 64, s));
@@ -1678,7 +1683,7 @@ int rgkc_superkmers_sized(rgkc_ctx* c, int k, int p, int parts, const uint64_t* 
     hipStream_t s = c->stream;
     c->k = k; c->p = p; c->parts = parts;
     c->store_ok = c->table_ok = false; c->stream_ended = false;
-    c->st = rgkc_stats{};
+    new_stats(c);
     c->st.n_reads = c->n_reads; c->st.n_bases = c->n_bases;
     NEED(c, c->err_word, 64);
     HIPC(c, hipMemsetAsync(c->err_word.p, 0, 64, s));
@@ -1774,7 +1779,7 @@ int rgkc_stream_begin(rgkc_ctx* c, int k, int p, int parts, uint64_t max_reads, 
     c->k = k; c->p = p; c->parts = parts;
     c->cap_reads = max_reads; c->cap_bases = max_bases;
     c->store_ok = c->table_ok = c->reads_ok = false;
-    c->st = rgkc_stats{};
+    new_stats(c);
     const uint64_t n_words = (max_bases >> 4) + 2;
     const uint64_t max_seg = max_reads + max_bases / kSegKmers + 2;
     NEED(c, c->reads, n_words * 16);
@@ -1878,9 +1883,13 @@ int rgkc_stream_end(rgkc_ctx* c, uint64_t* part_bytes, uint64_t* skm_cnt, uint64
     hipStream_t s = c->stream;
     const int parts = c->parts;
     std::vector<uint64_t> cur(3 * (size_t)parts);
+    uint32_t lists[3] = {0, 0, 0};  // tiles rescanned in the last batch, written in list order, rescanned before it
     HIPC(c, hipMemcpyAsync(cur.data(), c->cursors3.p, cur.size() * 8, hipMemcpyDeviceToHost, s));
+    if (c->sargs.skm_list) HIPC(c, hipMemcpyAsync(lists, c->sargs.n_rescan, 12, hipMemcpyDeviceToHost, s));
     HIPC(c, hipStreamSynchronize(s));
     unpack_cursors(cur, parts);
+    c->st.p1_rescans = lists[0] + lists[2];
+    c->h_listorder = lists[1];
     const uint64_t nbat = c->n_batches, nr = c->st.n_reads, nbs = c->st.n_bases;
     stream_free(c);
     if (int r = check_err_word(c)) return r;  // RGKC_E_OVERFLOW when a capacity was too small

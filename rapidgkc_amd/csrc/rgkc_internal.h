@@ -114,7 +114,7 @@ hipError_t launch_p1_emit_stream(const P1Args& a, unsigned grid, hipStream_t s);
 // the persistent scanning emit over the n_rescan tiles whose list overflowed (a.wg_map).
 hipError_t launch_p1_emit_sized(const P1Args& a, uint32_t n_rescan, hipStream_t s);
 // Batched input: pack + segment table from a device header ([0] reads, [1] bases; [2] set to the
-// segment count; *n_rescan cleared), all launched over the batch capacity.
+// segment count; n_rescan[0], the last batch's, added to n_rescan[2] and cleared), all launched over the batch capacity.
 hipError_t launch_batch_prep(const uint8_t* reads, const uint64_t* offs, uint64_t* hdr, uint64_t cap_reads,
                              uint64_t cap_bases, int k, uint32_t* bases2, uint64_t* nseg, uint64_t* seg_off,
                              uint64_t* scan_tmp, uint32_t* seg_read, uint32_t* seg_first, uint32_t* n_rescan,
