@@ -206,8 +206,9 @@ hipError_t need_count(rgkc_ctx* c, DevBuf& b, size_t bytes);
 int p1_threads(int k, int p) { return (k - p + 1) <= 32 ? 256 : 128; }
 
 // Phase-1 superkmer lists (unless switched off): room for 3x the superkmers a random sequence
-// gives (2 / (w + 1) per k-mer) per workgroup; a workgroup with more is rescanned by the emit pass.
-static int setup_lists(rgkc_ctx* c, P1Args& a, int T1, uint32_t n_wg) {
+// gives (2 / (w + 1) per k-mer) per workgroup; a workgroup with more is rescanned by the emit pass. Without
+// memory for them, and for `beside` bytes that are only needed with them, the emit pass scans (a.skm_list stays null).
+static int setup_lists(rgkc_ctx* c, P1Args& a, int T1, uint32_t n_wg, DevBuf* hist = nullptr, size_t beside = 0) {
     if (c->list_cap == 0xFFFFFFFFu) return 0;
     hipStream_t s = c->stream;
     const uint64_t w = (uint64_t)(a.k - a.p + 1);
@@ -215,17 +216,21 @@ static int setup_lists(rgkc_ctx* c, P1Args& a, int T1, uint32_t n_wg) {
     lcap = std::min<uint64_t>(std::max<uint64_t>((lcap + 63) / 64 * 64, 256), (uint64_t)T1 * kSegKmers);
     if (c->list_cap) lcap = std::min<uint64_t>(c->list_cap, (uint64_t)T1 * kSegKmers);
     const size_t lbytes = (size_t)n_wg * lcap * 8;
-    if (lbytes > c->skm_list.cap) {
+    const size_t more = (lbytes > c->skm_list.cap ? lbytes : 0) + (hist && beside > hist->cap ? beside : 0);
+    if (more) {
         // lists only when they fit in half the free device memory; otherwise the emit pass scans
         size_t fr = 0, tt = 0;
-        if (hipMemGetInfo(&fr, &tt) != hipSuccess || lbytes > fr / 2) {
+        if (hipMemGetInfo(&fr, &tt) != hipSuccess || more > fr / 2) {
             (void)hipGetLastError();
             return 0;
         }
     }
-    NEED(c, c->skm_list, lbytes);
-    // counts, rescan tiles, rescan count, list-order tiles, rescans of the stream's batches before the last
-    NEED(c, c->skm_n, ((size_t)2 * n_wg + 3) * 4);
+    // skm_n: counts, rescan tiles, rescan count, list-order tiles, rescans of the stream's batches before the last
+    if (c->skm_list.need(lbytes) != hipSuccess || c->skm_n.need(((size_t)2 * n_wg + 3) * 4) != hipSuccess ||
+        (hist && hist->need(beside) != hipSuccess)) {
+        (void)hipGetLastError();
+        return 0;
+    }
     HIPC(c, hipMemsetAsync(c->skm_n.as<uint32_t>() + 2 * (size_t)n_wg, 0, 12, s));
     a.skm_list = c->skm_list.as<uint64_t>();
     a.skm_n = c->skm_n.as<uint32_t>();
@@ -233,6 +238,24 @@ static int setup_lists(rgkc_ctx* c, P1Args& a, int T1, uint32_t n_wg) {
     a.wg_rescan = a.skm_n + n_wg;
     a.n_rescan = a.skm_n + 2 * (size_t)n_wg;
     a.n_listorder = a.n_rescan + 1;
+    return 0;
+}
+
+// The same for capacity-sized regions of n_seg segments at most: the list emit reserves each tile's runs from its
+// histogram columns, which nothing else reads.
+static int setup_region_lists(rgkc_ctx* c, P1Args& a, uint64_t n_seg) {
+    const int T1 = p1_threads(a.k, a.p);
+    const uint32_t n_wg = (uint32_t)((n_seg + T1 - 1) / T1);
+    const size_t hwords = (size_t)a.parts * ((size_t)n_wg + 1);
+    if (int r = setup_lists(c, a, T1, n_wg, &c->hist, 3 * hwords * 4)) return r;
+    if (!a.skm_list) return 0;
+    a.n_seg = n_seg;
+    a.n_wg = n_wg;
+    a.h_bytes = c->hist.as<uint32_t>();
+    a.h_recs = a.h_bytes + hwords;
+    a.h_kmers = a.h_recs + hwords;
+    a.list_reserve = 1;
+    a.wg_map = a.wg_rescan;
     return 0;
 }
 
@@ -1721,17 +1744,8 @@ int rgkc_superkmers_sized(rgkc_ctx* c, int k, int p, int parts, const uint64_t* 
         HIPC(c, hipMemcpyAsync(&nseg_total, c->seg_off.as<uint64_t>() + n, 8, hipMemcpyDeviceToHost, s));
         HIPC(c, hipStreamSynchronize(s));
         if (nseg_total > 0xFFFFFFFFull) return fail(c, RGKC_E_ARG, "too many read segments in one batch");
-        const int T1 = p1_threads(k, p);
-        const uint32_t n_wg = (uint32_t)((nseg_total + T1 - 1) / T1);
-        const size_t hwords = (size_t)parts * ((size_t)n_wg + 1);
-        NEED(c, c->hist, 3 * hwords * 4);
-        HIPC(c, hipMemsetAsync(c->hist.p, 0, 3 * hwords * 4, s));
-        a.n_seg = nseg_total;
-        a.h_bytes = c->hist.as<uint32_t>();
-        a.h_recs = a.h_bytes + hwords;
-        a.h_kmers = a.h_recs + hwords;
-        a.n_wg = n_wg;
-        if (int r = setup_lists(c, a, T1, n_wg)) return r;
+        if (int r = setup_region_lists(c, a, nseg_total)) return r;
+        if (a.skm_list) HIPC(c, hipMemsetAsync(c->hist.p, 0, 3 * (size_t)parts * ((size_t)a.n_wg + 1) * 4, s));
     }
     if (a.skm_list) {
         HIPC(c, launch_p1_count(a, s));
@@ -1740,8 +1754,6 @@ int rgkc_superkmers_sized(rgkc_ctx* c, int k, int p, int parts, const uint64_t* 
         HIPC(c, hipMemcpyAsync(&n_rescan, a.n_rescan, 4, hipMemcpyDeviceToHost, s));
         HIPC(c, hipStreamSynchronize(s));
         c->st.p1_rescans = n_rescan;
-        a.list_reserve = 1;
-        a.wg_map = a.wg_rescan;
         HIPC(c, launch_p1_emit_sized(a, n_rescan, s));
         HIPC(c, hipMemcpyAsync(&c->h_listorder, a.n_listorder, 4, hipMemcpyDeviceToHost, s));
     } else {
@@ -1808,22 +1820,9 @@ int rgkc_stream_begin(rgkc_ctx* c, int k, int p, int parts, uint64_t max_reads, 
     a.k = k; a.p = p; a.parts = parts; a.pdiv = FastDivU32::make((uint32_t)parts);
     region_args(c, a);
     a.n_seg_dev = c->hdr.as<uint64_t>() + 2;
-    if (c->list_cap != 0xFFFFFFFFu) {
-        // superkmer lists and tile histograms of one batch
-        const int T1 = p1_threads(k, p);
-        const uint32_t n_wg = (uint32_t)((max_seg + T1 - 1) / T1);
-        const size_t hwords = (size_t)parts * ((size_t)n_wg + 1);
-        NEED(c, c->hist, 3 * hwords * 4);
-        a.n_seg = max_seg;
-        a.h_bytes = c->hist.as<uint32_t>();
-        a.h_recs = a.h_bytes + hwords;
-        a.h_kmers = a.h_recs + hwords;
-        a.n_wg = n_wg;
-        if (int r = setup_lists(c, a, T1, n_wg)) return r;
-        a.list_reserve = 1;
-        a.wg_map = a.wg_rescan;
-        a.n_map_dev = a.n_rescan;
-    }
+    // superkmer lists and tile histograms of one batch
+    if (int r = setup_region_lists(c, a, max_seg)) return r;
+    a.n_map_dev = a.n_rescan;
     HIPC(c, hipStreamSynchronize(s));
     c->stream_graph = use_graph != 0;
     if (c->stream_graph) {
