@@ -56,6 +56,10 @@ constexpr size_t kTableChunk = 1u << 20;
 // Rows a partition, from which the runtime's copies into mapped memory are no slower than the gather.
 constexpr uint64_t kLongRun = 1u << 23;
 
+// Pinned staging memory that a context keeps from one stream to the next; more is given back when the
+// stream ends.
+constexpr uint64_t kStageKeep = 512u << 20;
+
 constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
 uint8_t* g_scratch_ptr[kMaxDevices] = {};
@@ -1650,6 +1654,7 @@ static int stream_free(rgkc_ctx* c) {
     if (c->gexec) { (void)hipGraphExecDestroy(c->gexec); c->gexec = nullptr; }
     if (c->graph) { (void)hipGraphDestroy(c->graph); c->graph = nullptr; }
     for (int i = 0; i < 2; i++) c->stage_ev_rec[i] = false;
+    if (2 * (c->stage_bytes + 8 * c->stage_reads) > kStageKeep) stage_free(c);
     (void)hipGetLastError();
     c->stream_on = false;
     return 0;
@@ -1666,8 +1671,8 @@ static void stage_free(rgkc_ctx* c) {
     c->stage_bytes = c->stage_reads = 0;
 }
 
-// The two pinned staging sets, kept by the context from stream to stream (grow-only like its device
-// buffers): allocated and freed with each stream, they cost up to 9 ms of a 20 ms pass over 32 batches.
+// The two pinned staging sets, kept by the context from stream to stream up to kStageKeep: allocated and
+// freed with each stream, they cost up to 9 ms of a 20 ms pass over 32 batches.
 static int stage_need(rgkc_ctx* c, uint64_t bytes, uint64_t reads) {
     if (bytes <= c->stage_bytes && reads <= c->stage_reads) return 0;
     bytes = std::max(bytes, c->stage_bytes);

@@ -31,3 +31,30 @@ def test_lists_that_do_not_fit_cost_nothing():
         assert np.array_equal(pb, np.diff(po)) and np.array_equal(sc, ps) and np.array_equal(kc, pk)
         c.close()
     assert abs(used[1] - used[0]) <= 32 << 20, used
+
+
+def _mapped():
+    """Address space of the process: pinned host memory, and the device's buffers too."""
+    with open("/proc/self/status") as f:
+        return next(int(line.split()[1]) << 10 for line in f if line.startswith("VmSize:"))
+
+
+@pytest.mark.parametrize("max_bases,kept", [(300_000_000, False), (100_000_000, True)])
+def test_staging_memory_is_given_back(max_bases, kept):
+    """The staging sets of a large batch capacity go with their stream, those of a small one stay."""
+    chars, offs = synth.short_reads(synth.genome(63, 50_000, gc=0.45), 64, 1_000, 150, 0.01)
+    c = native.Counter(0)
+    c.set_reads(chars, offs)
+    po, ps, _ = c.superkmers(31, 11, 32)
+    c.stream_begin(31, 11, 32, 1_000, len(chars), np.diff(po), ps)  # all that is allocated once
+    c.stream_add(chars, offs)
+    c.stream_end()
+    print(f"[gpu] case staging memory {max_bases}", flush=True)
+    c.stream_begin(31, 11, 32, 1_000, max_bases, np.diff(po), ps)
+    during = _mapped()
+    c.stream_add(chars, offs)
+    pb, _, _ = c.stream_end()
+    after = _mapped()
+    assert np.array_equal(pb, np.diff(po))
+    assert (during - after >= 2 * max_bases) == (not kept), (during, after)
+    c.close()
