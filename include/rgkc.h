@@ -150,8 +150,8 @@ int rgkc_stream_end(rgkc_ctx* ctx, uint64_t* part_bytes, uint64_t* skm_cnt, uint
 /* Device memory the count stage may plan with (0 = all it finds free; no counterpart in the
  * reference, whose VRAM grouping is gkc_main.cpp:324-352). Partitions are counted in groups whose
  * working set fits; when the table regions by k-mer instances do not fit beside them, each group is
- * counted into a temporary table and its rows are compacted into the final one. Results are the same
- * at every limit. */
+ * counted into a temporary table and its rows are compacted into the final one. Key regions larger than
+ * the limit are not made (rgkc_set_heavy_expand). Results are the same at every limit. */
 int rgkc_set_memory_limit(rgkc_ctx* ctx, uint64_t bytes);
 
 /* Accepted and without effect: one workgroup of the count kernel takes a CU's LDS (per_cu 0..4). */

@@ -430,9 +430,10 @@ uint32_t unit_cap(const rgkc_ctx* c) {
     return std::min<uint32_t>(std::max<uint32_t>(cap, 256u), 1u << 19);
 }
 
-// Count-stage working set of buckets [b0, b1) in bytes (2-bit words, record descriptors, key
-// regions, per-bucket plan arrays; plus a temporary table of one row per k-mer instance in compact
-// mode). An estimate used to cut the buckets into groups that fit the device memory.
+// Count-stage working set of buckets [b0, b1) in bytes (2-bit words, record descriptors, key regions, per-bucket
+// plan arrays; plus a temporary table of one row per k-mer instance in compact mode). An upper bound, used
+// to cut the buckets into groups that fit the device memory: which units are expanded is known only once a group
+// is planned, so key regions are charged for all k-mers.
 uint64_t group_bytes(const rgkc_ctx* c, uint32_t b0, uint32_t b1, size_t W, bool temp_table) {
     const uint64_t kmi = c->h_kmers[b1] - c->h_kmers[b0], ri = c->h_rec_off[b1] - c->h_rec_off[b0];
     const uint64_t nb = b1 - b0;
@@ -542,9 +543,10 @@ int count_buckets(rgkc_ctx* c, uint32_t b0, uint32_t b1, uint32_t cmin, uint32_t
     HIPC(c, launch_group(a, 2 * most_kmers / cap + 2 > (uint64_t)kSmallUnits, s));
     HIPC(c, hipEventSynchronize(c->plan_ev));
     uint64_t n_kunits = c->h_plan[kPlanKeyUnits], n_kitems = c->h_plan[kPlanKeyItems], n_items = c->h_plan[kPlanItems];
-    if (n_kunits && need_count(c, c->heavy_keys, (size_t)c->h_plan[kPlanKeySlots] * W + 64) != hipSuccess) {
-        // the key regions (the groups were sized to hold them) do not fit after all: planned again
-        // without them, every unit is counted from its records
+    const uint64_t key_bytes = c->h_plan[kPlanKeySlots] * W + 64;
+    if (n_kunits && ((c->mem_limit && key_bytes > c->mem_limit) || need_count(c, c->heavy_keys, key_bytes) != hipSuccess)) {
+        // the key regions do not fit (a single bucket's may exceed what its group was sized for): planned
+        // again without them, every unit is counted from its records
         (void)hipGetLastError();
         a.heavy_on = 0;
         HIPC(c, hipMemsetAsync(a.plan_n, 0, kPlanWords * 8, s));
