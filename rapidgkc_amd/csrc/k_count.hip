@@ -721,7 +721,7 @@ __global__ __launch_bounds__(kItemThreads, 4) void k_count_units(CountArgs a) {
         if ((float)inst <= kFill<K>) q = 1u;
         est_i = __hip_atomic_load(&a.plan_n[kPlanSeenInst], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         est_d = __hip_atomic_load(&a.plan_n[kPlanSeenDistinct], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        return (q + shares - 1u) / shares;
+        return shares == 1u ? q : (q + shares - 1u) / shares;
     };
     // thread 0: the item `v` begins, its share cut into q slices
     auto begin = [&](uint32_t v, uint32_t q) {
