@@ -60,6 +60,9 @@ constexpr uint64_t kLongRun = 1u << 23;
 // stream ends.
 constexpr uint64_t kStageKeep = 512u << 20;
 
+// Change of the free device memory that leaves the count stage's plan as it was.
+constexpr uint64_t kPlanSlack = 512u << 20;
+
 constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
 uint8_t* g_scratch_ptr[kMaxDevices] = {};
@@ -139,6 +142,7 @@ struct rgkc_ctx {
     bool table_ok = false;
     uint32_t inst_cap = 0;
     uint64_t mem_limit = 0;  // count stage: device memory to plan with (0: what is free)
+    uint64_t plan_avail = 0; // and what it planned with last
     bool compact_active = false;  // a count in compact mode holds its temporary table in tkeys/tcounts
     bool recount_active = false;  // the predicted path's recount writes keys2/counts2
     uint32_t list_cap = 0;  // phase-1 superkmer list entries per workgroup (0 default, ~0 off)
@@ -728,6 +732,12 @@ int do_count_once(rgkc_ctx* c, uint32_t cmin, uint32_t cmax, bool predicted) {
         held += d->cap;
     const uint64_t reserve = 4ull << 30;  // other users of the device and the runtime
     uint64_t avail = (uint64_t)fr + held > reserve ? ((uint64_t)fr + held - reserve) / 100 * 92 : 0;
+    // What is free moves from count to count by what the runtime allocates and rounds up (30 MB to 0.4 GB seen). The
+    // same figure then cuts the same batch into the same groups (kPlanSlack is far within the reserve): groups that
+    // end elsewhere want larger buffers, and the second count of 16 G k-mers reallocated 75 GB (2.14 s, so 0.22).
+    const uint64_t moved = std::max(avail, c->plan_avail) - std::min(avail, c->plan_avail);
+    if (c->plan_avail && avail && moved <= std::max(c->plan_avail / 64, kPlanSlack)) avail = c->plan_avail;
+    else c->plan_avail = avail;
     if (c->mem_limit) avail = std::min<uint64_t>(avail, c->mem_limit);
     if (predicted) {
         // predicted regions that would take more than 45% of the memory: a smaller margin (the
