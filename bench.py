@@ -8,8 +8,11 @@ minimizer scan + superkmer partitioning (exact two-pass sizing), and the count s
 produces every partition's (k-mer, count) table in HBM.
 
 Prints one JSON line (rank 0). `value` = k-mers counted per second (N / step time), N = sum over
-reads of (len - k + 1). `roofline` covers the count kernel: algorithmic bytes N*W + D_out*(W+4)
-(read every key once, write the table once) over its HIP-event time. `cpu_baseline` times the
+reads of (len - k + 1). `roofline` covers the count kernels (k_count_units, and k_count_keys for the
+largest units): algorithmic bytes N*W + D_out*(W+4) (a count that reads every key once and writes the
+table once) over their HIP-event time, a fixed measure and no bandwidth: k_count_units reads records
+and not keys. `traffic` and `traffic_frac` are the bytes that it moves, and their share of the peak over
+its own time, as measured in profiles/. `cpu_baseline` times the
 reference's own CPU path (cpu_funcs.cpp built from source into oracle/_ref) on a bounded sample of
 the same workload on this host.
 
@@ -418,11 +421,15 @@ def main():
     W = 8 if wl.k <= 32 else 16
     rows = int(st["rows"])
     tpath = os.path.join(ROOT, "profiles", f"count_traffic_{wl.name}.json")
-    traffic = None
+    traffic = traffic_frac = None
     if os.path.exists(tpath) and args.scale == 1.0:
         with open(tpath) as f:
-            traffic = json.load(f).get("bytes_per_launch")
+            prof = json.load(f)
+        traffic = prof.get("bytes_per_launch")
+        ns = prof.get("kernels", {}).get(prof.get("kernel"), {}).get("kernel_ns")
+        traffic_frac = traffic / (ns * 1e-9) / PEAK_HBM if traffic and ns else None
     roof = {**{k: roof[k] for k in ("bound", "achieved", "peak", "unit", "frac")}, "traffic": traffic,
+            "traffic_frac": traffic_frac,
             **{k: roof[k] for k in ("kernel", "alg_bytes_per_launch", "kernel_ms", "count_stage_ms", "count_stage_frac")}}
     # the reference's table order: each partition's rows ascending. The first call after a count
     # also allocates the sort's second row buffer (kept for later calls); the second call is the

@@ -93,10 +93,10 @@ int rgkc_count_host_store(rgkc_ctx* ctx, const uint8_t* store, const uint64_t* p
  * RGKC_E_ARG if the records do not decide it. rgkc_count_host_store calls it for p == 0. */
 int rgkc_store_minimizer_length(const uint8_t* store, const uint64_t* part_offs, int n_parts, int k, int* p);
 
-/* Copy the table of the last count to host memory: partition i's rows go to
- * keys[row_offs[i] .. row_offs[i+1]) where row_offs is the prefix of row_counts. keys holds
- * W bytes per row. Within a partition, rows are grouped by minimizer sub-bucket and ascending by
- * key inside each group (rgkc_sort_rows orders them fully). */
+/* Copy the table of the last count: partition i's rows go to keys[row_offs[i] .. row_offs[i+1])
+ * where row_offs is the prefix of row_counts. keys holds W bytes per row. Within a partition, rows come
+ * in no order (rgkc_sort_rows puts them in ascending key order). The destinations are host memory, best
+ * pinned (written at the link's rate; ordinary memory at one thread's copying rate), or device memory. */
 int rgkc_copy_table(rgkc_ctx* ctx, void* keys, uint32_t* counts);
 
 /* Order each partition's rows by ascending key on the device (the reference's table order,

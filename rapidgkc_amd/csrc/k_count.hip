@@ -31,7 +31,7 @@ constexpr int kItemThreads = 1024; // count workgroup size (one per CU)
 constexpr int kStack = 128;        // pending sweeps of one unit
 constexpr uint32_t kMaxCut = 8;    // slices an overflowing sweep is cut into, at most
 constexpr uint32_t kMaxSlices = 1u << 20;
-constexpr int kProbes = 64;        // table probes a key may take
+constexpr int kProbes = 64;        // tries a key may take to find its slot
 constexpr uint32_t kPiece = 4;     // consecutive k-mers of a record that one thread takes
 // LDS table: 8192 x (8 + 4) or 6144 x (16 + 4) bytes: with the staging areas one workgroup of 16 waves takes a
 // CU. 64-bit keys stage two records per thread, so that a unit is nearly always one chunk; with one record per thread
@@ -72,7 +72,8 @@ template <> struct KT<u128> {
         return mix(mix_in(h) ^ (uint32_t)(hi >> 32));
     }
 };
-// distinct keys a sweep is planned for: 80% of the slots (a run of 64 full groups flags the sweep)
+// distinct keys a sweep is planned for: 80% of the slots (a key that spends kProbes tries, on full groups, lost claims
+// and halves of other keys, flags the sweep)
 template <typename K> constexpr float kFill = 0.80f * (float)KT<K>::H;
 
 // A chunk of records: at most kItemThreads * R of them, W words, P pieces; S slots of its record set. A record of
@@ -648,14 +649,15 @@ __device__ __forceinline__ uint64_t first_row(const CountArgs& a, uint32_t part,
     return ~0ull;
 }
 
-// Units, from their records: chunk after chunk of up to kItemThreads records. A chunk is staged (record
+// Units, from their records: chunk after chunk of up to kItemThreads * R records. A chunk is staged (record
 // sizes scanned, words and record info to LDS) from registers whose loads were issued while the chunk
 // before it was counted, across the ends of sweeps and units as well; a sweep's rows leave only after the
 // next chunk is staged, so the row reservation's latency passes under the staging and the stores' under
 // the next chunk's counting. (With the loads of a sweep's first chunk and its row stores in line, staging
 // and row output took a third of the kernel.)
-// Bound by LDS in the insert (random 32-byte reads, CAS and count atomics: a third of the time at three
-// quarters of its rate) and by VALU issue around it, half of the issue slots. 1.2 G k-mers at 30x (360 M
+// Bound by LDS in the insert (random 32-byte reads, CAS and count atomics: a third of the time) and by the phases
+// around it, one after another: equal records 15%, the wait for the slowest wave 14%, staging 11% (clocks of the
+// first thread over 10 M reads at 30x). 1.2 G k-mers at 30x (360 M
 // distinct): 7.7 ms, where expanding every k-mer took 6.5 and counting the keys 6.0; 188 M (k=25) 1.14 ms, before
 // 1.2 + 0.85; 392 M 128-bit keys 5.4 ms, before 5.3 + 7.0. The loads take a uniform base and a thread's offset: with an
 // address per load 27 registers went to scratch, 0.6 ms of the first.
@@ -710,7 +712,7 @@ __global__ __launch_bounds__(kItemThreads, 4) void k_count_units(CountArgs a) {
     constexpr int kQ = offsetof(UnitDesc, q) / 4, kShare = offsetof(UnitDesc, share) / 4;
     uint32_t ahead = fetch(it);
     UnitDesc ud = unit(ahead);
-    // Initial hash slices of a unit's share (one of q): what its distinct keys should take by the ratio seen so far. The next unit's are
+    // Initial hash slices of a unit's share: what its distinct keys should take by the ratio seen so far. The next unit's are
     // worked out by the last wave, which has the fewest records, while the others look for equal ones (at the sweep's
     // end by thread 0 they took 6% of the kernel).
     auto slices = [&](uint32_t v) {

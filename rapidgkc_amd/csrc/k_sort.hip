@@ -2,8 +2,8 @@
 // order, the order of the reference's table (cpu_funcs.cpp:614-640: its rows come from a run-length
 // pass over the sorted keys).
 //
-// Rows of one partition arrive as runs (one per count sweep), each ascending; the keys of different
-// runs interleave. Keys of a table are distinct, so the sort needs no stability. MSD radix over
+// Rows of one partition arrive in no order (a run per count sweep, in the order of its table's slots). Keys of a
+// table are distinct, so the sort needs no stability. MSD radix over
 // segments planned on the host, each split by a digit of 4 to 12 bits sized to the segment (the
 // histogram rows are as wide as the round's widest digit):
 //   - a segment of at most kLeaf rows is loaded into LDS by one workgroup, bitonic-sorted there
