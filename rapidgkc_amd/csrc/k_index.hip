@@ -27,19 +27,26 @@ __device__ __forceinline__ uint32_t full_bits(uint32_t x) {
     return (t & 1u) | ((t >> 7) & 2u) | ((t >> 14) & 4u) | ((t >> 21) & 8u);
 }
 
+// Bytes after which a record cannot end with k-mers that a side word holds (18 bits): it is not followed further, so
+// that bytes without an end (60 MB of them kept one thread busy for 2.2 s) cost no more than a long record.
+constexpr uint64_t kMostBytes = (0x3FFFFu + 64u) / 3u + 4u;
+
 // Record starting at byte i of a partition of n bytes: sets bm3 and bases.
 __device__ __forceinline__ void record_shape(const uint8_t* s, uint64_t i, uint64_t n, uint32_t& bm3, uint32_t& L, bool& ok) {
     const uint32_t ind0 = (uint32_t)s[i] >> 6;
+    const uint64_t end = min(n, i + kMostBytes);
     uint64_t j = i + 1;
-    while (j < n) {  // the store's buffer holds 64 bytes after its last
+    bool ends = false;
+    while (j < end) {  // the store's buffer holds 64 bytes after its last
         const uint32_t f = full_bits(load_u32(s + j));
         if (f != 15u) {
             j += (uint32_t)__builtin_ctz(~f);
+            ends = j < n;
             break;
         }
         j += 4;
     }
-    ok = ind0 != 0 && j < n;
+    ok = ind0 != 0 && ends;
     bm3 = ok ? 3u - ind0 : 0u;
     L = ok ? ind0 + 3u * (uint32_t)(j - i - 1) + ((uint32_t)s[j] >> 6) : 0u;
 }
