@@ -141,7 +141,8 @@ int rgkc_superkmers_sized(rgkc_ctx* ctx, int k, int p, int parts, const uint64_t
  * cap_recs (e.g. from the learned predictor). Each batch is one H2D copy plus one replay of a
  * captured hipGraph (use_graph) of persistent kernels that read the batch size from device
  * memory. rgkc_stream_end returns RGKC_E_OVERFLOW if a region was too small (recount with exact
- * sizing), else the store is ready for rgkc_count. */
+ * sizing), else the store is ready for rgkc_count. A phase 1, a host store or reads larger than the
+ * stream's in between end it: adding to it is then RGKC_E_STATE. */
 int rgkc_stream_begin(rgkc_ctx* ctx, int k, int p, int parts, uint64_t max_reads, uint64_t max_bases,
                       const uint64_t* cap_bytes, const uint64_t* cap_recs, int use_graph);
 int rgkc_stream_add(rgkc_ctx* ctx, const char* reads, const uint64_t* offs, int64_t n_reads);

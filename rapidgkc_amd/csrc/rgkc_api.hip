@@ -172,6 +172,10 @@ struct rgkc_ctx {
     uint32_t h_listorder = 0;  // list-order tile count of the last phase-1 emit (read after a stream sync)
 };
 
+extern "C" {
+static int stream_free(rgkc_ctx* c);
+}
+
 namespace {
 
 int fail(rgkc_ctx* c, int code, const char* fmt, ...) {
@@ -298,6 +302,12 @@ int check_err_word(rgkc_ctx* c) {
     return 0;
 }
 
+// Before anything replaces what the stream's kernels (its captured graph) point at: regions, store, lists, reads.
+// The stream ends here, and adding to it is a state error.
+void stream_abandon(rgkc_ctx* c) {
+    if (c->stream_on) stream_free(c);
+}
+
 void new_stats(rgkc_ctx* c) {
     c->st = rgkc_stats{};
     c->h_listorder = 0;
@@ -310,6 +320,7 @@ int do_phase1(rgkc_ctx* c, int k, int p, int parts, uint32_t* mm_hist = nullptr)
     if (parts < 1 || parts > kMaxParts) return fail(c, RGKC_E_ARG, "parts must be in [1, %d]", kMaxParts);
     if (k - p + 1 > 64) return fail(c, RGKC_E_ARG, "window k-p+1 must be <= 64");
     hipStream_t s = c->stream;
+    stream_abandon(c);
     c->k = k; c->p = p; c->parts = parts;
     c->store_ok = false; c->table_ok = false; c->stream_ended = false;
     new_stats(c);
@@ -1121,7 +1132,6 @@ int rgkc_create(int device, rgkc_ctx** out) {
     return 0;
 }
 
-static int stream_free(rgkc_ctx* c);
 static void stage_free(rgkc_ctx* c);
 
 int rgkc_destroy(rgkc_ctx* c) {
@@ -1153,6 +1163,8 @@ int rgkc_set_reads(rgkc_ctx* c, const char* reads, const uint64_t* offs, int64_t
     const uint64_t nb = offs[n_reads];
     if (offs[0] != 0) return fail(c, RGKC_E_ARG, "offs[0] must be 0");
     const uint64_t n_words = (nb >> 4) + 2;  // packed words written by the pack kernel
+    if (n_words * 16 > c->reads.cap || ((uint64_t)n_reads + 1) * 8 > c->offs.cap || (n_words + 2) * 4 > c->bases2.cap)
+        stream_abandon(c);
     NEED(c, c->reads, n_words * 16);
     NEED(c, c->offs, (n_reads + 1) * 8);
     NEED(c, c->bases2, (n_words + 2) * 4);
@@ -1304,6 +1316,7 @@ int rgkc_count_host_store(rgkc_ctx* c, const uint8_t* store, const uint64_t* par
     (void)hipGetLastError();
     HIPC(c, hipSetDevice(c->device));
     hipStream_t s = c->stream;
+    stream_abandon(c);
     c->store_ok = false; c->table_ok = false; c->stream_ended = false;
     new_stats(c);
     const uint64_t S = part_offs[n_parts];
@@ -1721,6 +1734,7 @@ int rgkc_superkmers_sized(rgkc_ctx* c, int k, int p, int parts, const uint64_t* 
     if (k < 8 || k > 63 || p < 3 || p > 16 || p > k || k - p + 1 > 64) return fail(c, RGKC_E_ARG, "bad k/p");
     if (parts < 1 || parts > kMaxParts) return fail(c, RGKC_E_ARG, "parts must be in [1, %d]", kMaxParts);
     hipStream_t s = c->stream;
+    stream_abandon(c);
     c->k = k; c->p = p; c->parts = parts;
     c->store_ok = c->table_ok = false; c->stream_ended = false;
     new_stats(c);
